@@ -1,0 +1,54 @@
+"""Kernels at the sizes where their tiling can go wrong (remainders, one
+short of and one past a tile, unaligned outputs), against the FP64 oracle.
+
+Tolerances are the FP32 error model's: a sphere centre or frame entry lies
+within 2e-6 of FP64 (parity_common), a box distance within 1e-5 of
+max(|ref|, 0.05 m).
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+import pyoracle as PO
+from prismplan_amd import _ppl
+from prismplan_amd import substrate as S
+from prismplan_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module")
+def robots():
+    return {n: S.Robot(n) for n in ("panda", "fetch", "baxter")}
+
+
+@pytest.mark.parametrize("name,n,shift", [("panda", 1, 0), ("panda", 3, 1), ("fetch", 5, 0), ("fetch", 130, 1),
+                                          ("baxter", 4, 3), ("baxter", 67, 0), ("fetch", 40001, 0)])
+def test_fk_remainders_and_alignment(robots, name, n, shift):
+    """Four configurations a wave; outputs `shift` floats off 16-byte alignment
+    take the float-by-float stores. Nothing past the outputs is written."""
+    rob = robots[name]
+    info, D = rob.info(), rob.n_dof
+    J, Sn = info["n_joints"], info["n_spheres"]
+    q = W.uniform_configs(np.random.default_rng(n), rob.arrays, n)
+    d_q = torch.from_numpy(q).to(DEV)
+    f = torch.full((shift + n * J * 16 + 64,), -7.0, device=DEV)
+    s = torch.full((shift + n * Sn * 4 + 64,), -7.0, device=DEV)
+    plan = S.Plan.configs(rob, n)
+    p = lambda t: C.c_void_p(t.data_ptr() + 4 * shift)
+    _ppl.call("ppl_fk_batched", plan.handle, C.c_void_p(d_q.data_ptr()), p(f), p(s),
+              C.c_void_p(torch.cuda.current_stream().cuda_stream))
+    f, s = f.cpu().numpy(), s.cpu().numpy()
+    for x, m in ((f, n * J * 16), (s, n * Sn * 4)):
+        assert np.all(x[:shift] == -7.0) and np.all(x[shift + m:] == -7.0)
+    o = PO.Oracle(rob.arrays)
+    k = np.unique(np.linspace(0, n - 1, min(n, 2000)).astype(int))
+    got_f = f[shift:shift + n * J * 16].reshape(n, J, 4, 4).transpose(0, 1, 3, 2)[k]
+    got_s = s[shift:shift + n * Sn * 4].reshape(n, Sn, 4)[k]
+    assert np.abs(got_f[:, :, :3] - o.fk_frames(q[k])).max() < 2e-6
+    assert np.all(got_f[:, :, 3] == [0, 0, 0, 1])
+    assert np.abs(got_s[..., :3] - o.fk_spheres(q[k])).max() < 2e-6
+    np.testing.assert_array_equal(got_s[..., 3], np.broadcast_to(rob.arrays.spheres[:, 3], (len(k), Sn)))
