@@ -52,3 +52,20 @@ def test_fk_remainders_and_alignment(robots, name, n, shift):
     assert np.all(got_f[:, :, 3] == [0, 0, 0, 1])
     assert np.abs(got_s[..., :3] - o.fk_spheres(q[k])).max() < 2e-6
     np.testing.assert_array_equal(got_s[..., 3], np.broadcast_to(rob.arrays.spheres[:, 3], (len(k), Sn)))
+
+
+@pytest.mark.parametrize("dims,boxes", [((1, 1, 1), 1), ((4, 4, 16), 5), ((5, 3, 17), 64), ((33, 18, 47), 65),
+                                        ((21, 40, 15), 130), ((30, 31, 32), 60)])
+def test_esdf_brick_remainders(dims, boxes):
+    """Grids of one node, exact bricks and remainders; boxes below, at and past
+    a tile of 64; a rotated grid."""
+    rng = np.random.default_rng(boxes)
+    obbs = W.random_obbs(rng, boxes, half_lo=0.02, half_hi=0.15)
+    prm = np.array([0.03 * (d - 1) for d in dims] + [0.03], np.float32)
+    q = rng.normal(size=4)
+    q /= np.linalg.norm(q)
+    pose = np.array([-0.5, 0.1, -0.4, *q, 0.0], np.float32)
+    got = S.esdf_from_obbs(S.DeviceScene.from_host(obbs), prm, pose).cpu().numpy()
+    ref = PO.esdf_from_obbs(obbs.obb_dims, obbs.obb_pose, prm, pose)
+    assert got.shape == (dims[0] * dims[1] * dims[2],)
+    assert np.max(np.abs(got - ref.reshape(-1)) / np.maximum(np.abs(ref.reshape(-1)), 0.05)) < 1e-5
