@@ -1260,15 +1260,7 @@ ppl_status ppl_edge_eval_evaluate(ppl_edge_eval ev, const float* h_from, const f
     if (want_clr && total > 0) {
         HIP_TRY(ev->d_clr_state.ensure((size_t)total * 4));
         HIP_TRY(ev->d_clr_edge.ensure((size_t)n * 4));
-        CostArgs c{};
-        c.R = r->R;
-        c.S = ev->S;
-        c.X = X;
-        c.P.weight = 1.0f;
-        c.clearance_only = 1;
-        c.margin = p->collision_margin;
-        c.cost_out = ev->d_clr_state.as<float>();
-        HIP_TRY(launch_cost_flat(c, total, ev->stream));
+        HIP_TRY(launch_clear(ClearArgs{r->R, ev->S, X, p->collision_margin, ev->d_clr_state.as<float>()}, ev->stream));
         hipLaunchKernelGGL(k_segment_min, dim3(n), dim3(64), 0, ev->stream, ev->d_clr_state.as<float>(), d_off, n,
                            ev->d_clr_edge.as<float>());
         HIP_TRY(hipGetLastError());
@@ -2402,21 +2394,7 @@ ppl_status ppl_min_clearance_batched(ppl_plan P, const ppl_scene_view* view, con
     ppl_status st = plan_scene(P, view, S);
     if (st != PPL_OK) return st;
     if (P->n_states == 0) return PPL_OK;
-    CostArgs a{};
-    a.R = P->robot->R;
-    a.S = S;
-    a.X = plan_states(P, d_cfg);
-    int grid = 0;
-    const int max_obbs = plan_obb_cap(P, S);
-    const bool tiled = max_obbs > kMaxObbLds;   // the grouped kernel streams the OBBs in tiles
-    HIP_TRY(ensure_table(P, tiled ? kGrp : 1));
-    a.C = plan_chunks(P, tiled ? kKCostGrp : kKCost, max_obbs, tiled ? kGrp : 1, &grid);
-    a.group = tiled ? kGrp : 1;
-    a.P.weight = 1.0f;
-    a.clearance_only = 1;
-    a.margin = margin;
-    a.cost_out = d_out;
-    HIP_TRY(tiled ? launch_cost_grp(a, grid, (hipStream_t)stream) : launch_cost(a, grid, (hipStream_t)stream));
+    HIP_TRY(launch_clear(ClearArgs{P->robot->R, S, plan_states(P, d_cfg), margin, d_out}, (hipStream_t)stream));
     return PPL_OK;
 } catch (const std::bad_alloc&) {
     return ppl::fail_msg(PPL_ERR_ALLOC, "out of host memory");
@@ -2426,22 +2404,16 @@ ppl_status ppl_min_clearance_batched(ppl_plan P, const ppl_scene_view* view, con
 
 namespace {
 // Min ESDF clearance (+ margin) of n configurations d_cfg [n][D] into d_out,
-// scene_min_clearance_runtime semantics (the clearance mode of the cost kernel).
+// scene_min_clearance_runtime semantics.
 ppl_status configs_clearance(const ppl_robot_s* r, const DScene& S, const float* d_cfg, int n, float margin,
                              float* d_out, hipStream_t s) {
     if (n <= 0) return PPL_OK;
-    CostArgs c{};
-    c.R = r->R;
-    c.S = S;
-    c.X.source = kSrcConfig;
-    c.X.n_states = n;
-    c.X.cfg = d_cfg;
-    c.X.cfg_stride = r->R.n_dof;
-    c.P.weight = 1.0f;
-    c.clearance_only = 1;
-    c.margin = margin;
-    c.cost_out = d_out;
-    HIP_TRY(launch_cost_flat(c, n, s));
+    DStates X{};
+    X.source = kSrcConfig;
+    X.n_states = n;
+    X.cfg = d_cfg;
+    X.cfg_stride = r->R.n_dof;
+    HIP_TRY(launch_clear(ClearArgs{r->R, S, X, margin, d_out}, s));
     return PPL_OK;
 }
 

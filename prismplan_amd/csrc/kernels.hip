@@ -37,6 +37,21 @@ __device__ __forceinline__ float uniform(float v) {
     return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
 }
 
+// Wave-uniform reads of tables that no launch writes (robot tables, layer
+// parameters), through the constant address space: they become scalar loads
+// into SGPRs. A plain read after a barrier or an LDS write is a vector load
+// per lane instead, since the compiler cannot tell that the table stays.
+typedef float f4u __attribute__((ext_vector_type(4)));
+typedef int i4u __attribute__((ext_vector_type(4)));
+template <typename T>
+__device__ __forceinline__ T uload(const void* p, int i) {
+    return reinterpret_cast<const __attribute__((address_space(4))) T*>(reinterpret_cast<uintptr_t>(p))[i];
+}
+__device__ __forceinline__ float4 uload4(const void* p, int i) {
+    const f4u v = uload<f4u>(p, i);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
 // ---------------------------------------------------------------------------
 // 3x4 affine helpers (row-major, implicit last row 0 0 0 1)
 // ---------------------------------------------------------------------------
@@ -65,6 +80,35 @@ __device__ __forceinline__ void joint_step(const float* __restrict__ ft, int typ
     } else if (type >= kXPrism) {
 #pragma unroll
         for (int r = 0; r < 3; ++r) S[r * 4 + 3] = fmaf(ft[r * 4 + type], q, ft[r * 4 + 3]);
+    }
+}
+
+// The same step for a joint that is the same in every lane (rows of the fixed
+// transform by scalar loads; the same operations, so the same bits).
+template <int A, int B>
+__device__ __forceinline__ void rot_cols(float s, float c, float* S) {
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        const float fa = S[r * 4 + A], fb = S[r * 4 + B];
+        S[r * 4 + A] = fmaf(fa, c, fb * s);
+        S[r * 4 + B] = fmaf(fb, c, -fa * s);
+    }
+}
+__device__ __forceinline__ void joint_step_u(const float* tab, int jj, int type, float q, float s, float c, float* S) {
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        const f4u f = uload<f4u>(tab, 3 * jj + r);
+        S[r * 4] = f.x; S[r * 4 + 1] = f.y; S[r * 4 + 2] = f.z; S[r * 4 + 3] = f.w;
+    }
+    if (type == kXRot) rot_cols<1, 2>(s, c, S);
+    else if (type == kYRot) rot_cols<2, 0>(s, c, S);
+    else if (type == kZRot) rot_cols<0, 1>(s, c, S);
+    else if (type >= kXPrism) {
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            const float f = type == kXPrism ? S[r * 4] : type == kYPrism ? S[r * 4 + 1] : S[r * 4 + 2];
+            S[r * 4 + 3] = fmaf(f, q, S[r * 4 + 3]);
+        }
     }
 }
 
@@ -117,14 +161,18 @@ struct Slots {
 // joint types.
 template <bool APPROX = false>
 __device__ __forceinline__ void fk_joint(const DRobot& R, int jj, const float* s_q, Slots& sl, float* T, int4& meta) {
-    meta = R.jmeta[jj];
+    const i4u m = uload<i4u>(R.jmeta, jj);
+    meta = make_int4(m.x, m.y, m.z, m.w);
     if (jj == 0) {
         aff_identity(T);
     } else {
         float P[12], S[12];
         sl.load(meta.w, P);
         const float q = meta.y >= 0 ? s_q[meta.y * kWave] : 0.0f;
-        joint_step(APPROX ? R.aft + 12 * jj : R.ft + 12 * jj, APPROX ? R.atype[jj] : meta.x, q, S);
+        const int type = APPROX ? uload<int>(R.atype, jj) : meta.x;
+        float s = 0.0f, c = 0.0f;
+        if (type >= kXRot) sincosf(q, &s, &c);
+        joint_step_u(APPROX ? R.aft : R.ft, jj, type, q, s, c, S);
         aff_compose(P, S, T);
     }
     sl.store(meta.z, T);
@@ -244,14 +292,16 @@ __device__ __forceinline__ int robust_floor(float x) {
     return (int)nearest;
 }
 
-__device__ __forceinline__ void quat_local(const float* pose, float sx, float sy, float sz, float& lx, float& ly, float& lz) {
-    const float qw = pose[3], qx = pose[4], qy = pose[5], qz = pose[6];
+// Stored inverse pose (t, qw | qx, qy, qz, pad) applied to a world point.
+__device__ __forceinline__ void quat_local(const float4& p0, const float4& p1, float sx, float sy, float sz, float& lx,
+                                           float& ly, float& lz) {
+    const float qw = p0.w, qx = p1.x, qy = p1.y, qz = p1.z;
     const float tx = 2.0f * (qy * sz - qz * sy);
     const float ty = 2.0f * (qz * sx - qx * sz);
     const float tz = 2.0f * (qx * sy - qy * sx);
-    lx = sx + qw * tx + (qy * tz - qz * ty) + pose[0];
-    ly = sy + qw * ty + (qz * tx - qx * tz) + pose[1];
-    lz = sz + qw * tz + (qx * ty - qy * tx) + pose[2];
+    lx = sx + qw * tx + (qy * tz - qz * ty) + p0.x;
+    ly = sy + qw * ty + (qz * tx - qx * tz) + p0.y;
+    lz = sz + qw * tz + (qx * ty - qy * tx) + p0.z;
 }
 
 // Minimum ESDF clearance (-dist - r) over enabled layers, 1000 when none
@@ -273,7 +323,8 @@ __device__ float esdf_clearance(const DScene& S, float px, float py, float pz, f
         const int ny = robust_floor(prm[1] * inv_vs) + 1;
         const int nz = robust_floor(prm[2] * inv_vs) + 1;
         float lx, ly, lz;
-        quat_local(pose, px, py, pz, lx, ly, lz);
+        quat_local(make_float4(pose[0], pose[1], pose[2], pose[3]), make_float4(pose[4], pose[5], pose[6], pose[7]), px, py, pz,
+                   lx, ly, lz);
         const float ux = (lx + prm[0] * 0.5f) * inv_vs, uy = (ly + prm[1] * 0.5f) * inv_vs, uz = (lz + prm[2] * 0.5f) * inv_vs;
         const float* feat = S.voxel_features + (size_t)layer * S.max_voxels_per_layer;
         if (S.esdf_interp == 0) {
@@ -328,6 +379,83 @@ __device__ __forceinline__ bool esdf_hit(const DScene& S, float px, float py, fl
     // min clearance < 0  <=>  some layer has dist > -r
     return esdf_clearance(S, px, py, pz, r, sph_orig, false, gx, gy, gz) < 0.0f;
 }
+
+// A single trilinear layer without masks, the usual world: its parameters once
+// per wave instead of once per lookup, and the lookup split in two so that two
+// spheres' grid loads can be in flight together. Values and gradients equal
+// esdf_clearance's.
+__host__ __device__ inline bool esdf_single(const DScene& S) {
+    return S.n_voxel_layers == 1 && S.esdf_interp != 0 && !S.sphere_acm;
+}
+struct EsdfLayer {
+    float4 prm, p0, p1;
+    float inv_vs;
+    int nx, ny, nz, max_lin;
+    bool on;   // enabled, with a voxel size: else it has no inside
+    const float* feat;
+    EsdfLayer() = default;
+    __device__ __forceinline__ explicit EsdfLayer(const DScene& S)
+        : prm(uload4(S.voxel_params, 0)), p0(uload4(S.voxel_pose, 0)), p1(uload4(S.voxel_pose, 1)) {
+        on = S.voxel_enable[0] != 0 && prm.w > 0.0f;
+        inv_vs = uniform(1.0f / prm.w);
+        nx = uniform(robust_floor(prm.x * inv_vs) + 1);
+        ny = uniform(robust_floor(prm.y * inv_vs) + 1);
+        nz = uniform(robust_floor(prm.z * inv_vs) + 1);
+        feat = S.voxel_features;
+        max_lin = S.max_voxels_per_layer;
+    }
+};
+struct EsdfTap {
+    float fx, fy, fz;
+    bool ok;
+    float c000, c001, c010, c011, c100, c101, c110, c111;
+    __device__ __forceinline__ void load(const EsdfLayer& L, float px, float py, float pz, bool on) {
+        float lx, ly, lz;
+        quat_local(L.p0, L.p1, px, py, pz, lx, ly, lz);
+        const float ux = (lx + L.prm.x * 0.5f) * L.inv_vs, uy = (ly + L.prm.y * 0.5f) * L.inv_vs,
+                    uz = (lz + L.prm.z * 0.5f) * L.inv_vs;
+        const float fx0 = floorf(ux), fy0 = floorf(uy), fz0 = floorf(uz);
+        const int ix = (int)fx0, iy = (int)fy0, iz = (int)fz0;
+        fx = ux - fx0; fy = uy - fy0; fz = uz - fz0;
+        ok = on && L.on && !(ix >= L.nx - 2 || iy >= L.ny - 2 || iz >= L.nz - 2 || ix <= 2 || iy <= 2 || iz <= 2);
+        const long sx = (long)L.ny * L.nz, sy = L.nz;
+        const long base = ok ? (long)ix * sx + (long)iy * sy + iz : 0;
+        ok = ok && base + sx + sy + 1 < L.max_lin;
+        if (ok) {
+            const float* f = L.feat + base;
+            c000 = f[0]; c001 = f[1]; c010 = f[sy]; c011 = f[sy + 1];
+            c100 = f[sx]; c101 = f[sx + 1]; c110 = f[sx + sy]; c111 = f[sx + sy + 1];
+        }
+    }
+    __device__ __forceinline__ float value(float r) const {
+        if (!ok) return 1000.0f;
+        const float mn = fminf(fminf(fminf(c000, c001), fminf(c010, c011)), fminf(fminf(c100, c101), fminf(c110, c111)));
+        if (mn <= -999.0f) return 1000.0f;
+        const float c00 = fmaf(c100 - c000, fx, c000), c01 = fmaf(c101 - c001, fx, c001);
+        const float c10 = fmaf(c110 - c010, fx, c010), c11 = fmaf(c111 - c011, fx, c011);
+        const float c0 = fmaf(c10 - c00, fy, c00), c1 = fmaf(c11 - c01, fy, c01);
+        const float d = fmaf(c1 - c0, fz, c0);
+        const float c = -d - r;
+        return c < 1000.0f ? c : 1000.0f;
+    }
+    // d dist / d p (world) where value() came from the grid
+    __device__ __forceinline__ void grad(const EsdfLayer& L, float& gx, float& gy, float& gz) const {
+        const float c00 = fmaf(c100 - c000, fx, c000), c01 = fmaf(c101 - c001, fx, c001);
+        const float c10 = fmaf(c110 - c010, fx, c010), c11 = fmaf(c111 - c011, fx, c011);
+        const float c0 = fmaf(c10 - c00, fy, c00), c1 = fmaf(c11 - c01, fy, c01);
+        const float ofy = 1.0f - fy, ofz = 1.0f - fz;
+        const float dx = ((c100 - c000) * ofy * ofz + (c101 - c001) * ofy * fz + (c110 - c010) * fy * ofz +
+                          (c111 - c011) * fy * fz) * L.inv_vs;
+        const float dy = ((c10 - c00) * ofz + (c11 - c01) * fz) * L.inv_vs;
+        const float dz = (c1 - c0) * L.inv_vs;
+        const float qw = L.p0.w, qx = -L.p1.x, qy = -L.p1.y, qz = -L.p1.z;
+        const float tx = 2.0f * (qy * dz - qz * dy), ty = 2.0f * (qz * dx - qx * dz), tz = 2.0f * (qx * dy - qy * dx);
+        gx = dx + qw * tx + (qy * tz - qz * ty);
+        gy = dy + qw * ty + (qz * tx - qx * tz);
+        gz = dz + qw * tz + (qx * ty - qy * tx);
+    }
+};
+
 
 // ---------------------------------------------------------------------------
 // State resolution: flattened state index -> per-lane q in LDS
@@ -1002,17 +1130,14 @@ __device__ __forceinline__ void obb_argmin(const float4* __restrict__ s_obb, con
 // Hinge terms of one sphere at world position p given its OBB argmin (best
 // key; has_arg: there is one; rec(r0, r1, r2, r3) fetches the argmin OBB's
 // record, called only for the gradient of an active hinge): the summed hinge
-// (OBB + ESDF) and its point gradient d hinge / d p in g*; in clearance-only
-// mode the ESDF clearance with radius + margin.
-template <bool GRAD, class Rec>
-__device__ __forceinline__ float sphere_hinge_at(const CostArgs& a, bool has_arg, const Rec& rec, float best, float px,
+// (OBB + ESDF) and its point gradient d hinge / d p in g*.
+template <bool GRAD, bool ONE, class Rec>
+__device__ __forceinline__ float sphere_hinge_at(const CostArgs& a, const EsdfLayer& layer, bool has_arg, const Rec& rec, float best, float px,
                                                  float py, float pz, float r, int sph_id, bool use_obb, bool use_esdf,
                                                  float& gx, float& gy, float& gz) {
     const float m = a.P.world_margin;
     float world = 0.0f;
     gx = gy = gz = 0.0f;
-    // clearance mode is ESDF-only; no layer gives sphere_esdf_clearance's 1000
-    if (a.clearance_only && !use_esdf) return 1000.0f;
     if (use_obb) {
         const float clr = has_arg ? key_to_sdf(best) - r : 1000.0f;
         const float hh = m - clr;
@@ -1029,26 +1154,33 @@ __device__ __forceinline__ float sphere_hinge_at(const CostArgs& a, bool has_arg
     }
     if (use_esdf) {
         float dx, dy, dz;
-        const float rr = a.clearance_only ? r + a.margin : r;
-        const float c = esdf_clearance(a.S, px, py, pz, rr, sph_id, GRAD, dx, dy, dz);
-        if (a.clearance_only) return c;
-        const float hh = m - c;
-        if (hh > 0.0f) {
-            world += hh;
-            if (GRAD) { gx += dx; gy += dy; gz += dz; }
+        if (ONE) {
+            EsdfTap t;
+            t.load(layer, px, py, pz, true);
+            const float hh = m - t.value(r);
+            if (hh > 0.0f) {
+                world += hh;
+                if (GRAD && t.ok) {
+                    t.grad(layer, dx, dy, dz);
+                    gx += dx; gy += dy; gz += dz;
+                }
+            }
+        } else {
+            const float c = esdf_clearance(a.S, px, py, pz, r, sph_id, GRAD, dx, dy, dz);
+            const float hh = m - c;
+            if (hh > 0.0f) {
+                world += hh;
+                if (GRAD) { gx += dx; gy += dy; gz += dz; }
+            }
         }
     }
     return world;
 }
 
-// Sum / min over the G lanes of a state group (G a power of two <= 64; the
+// Sum over the G lanes of a state group (G a power of two <= 64; the
 // groups are aligned, so xor offsets below G stay inside the group).
 __device__ __forceinline__ float group_sum(float v, int G) {
     for (int o = 1; o < G; o <<= 1) v += __shfl_xor(v, o);
-    return v;
-}
-__device__ __forceinline__ float group_min(float v, int G) {
-    for (int o = 1; o < G; o <<= 1) v = fminf(v, __shfl_xor(v, o));
     return v;
 }
 
@@ -1070,8 +1202,8 @@ __global__ __launch_bounds__(64, 4) void k_cost(CostArgs a) {
     const int rs = rec_stride(J), ds = dq_stride(D);
     float* rec = s_q + (D + 2) * kWave + slot * rs;
     float* dqs = s_q + (D + 2) * kWave + (kWave / G) * rs + slot * ds;
-    const bool use_obb = a.P.use_obb != 0 && !a.clearance_only;
-    const bool use_esdf = (a.P.use_esdf != 0 || a.clearance_only) && a.S.n_voxel_layers > 0;
+    const bool use_obb = a.P.use_obb != 0;
+    const bool use_esdf = a.P.use_esdf != 0 && a.S.n_voxel_layers > 0;
     const float wt = a.P.weight;
     int cur_prob = -1, n_obb = 0;
     int4 ch;
@@ -1095,12 +1227,12 @@ __global__ __launch_bounds__(64, 4) void k_cost(CostArgs a) {
         // Self term from the self pass: hinge and its two point gradients.
         float self_h = 0.0f, snx = 0.0f, sny = 0.0f, snz = 0.0f;
         int si = -1, sj = -1;
-        if (a.self_in && active && !a.clearance_only) {
+        if (a.self_in && active) {
             const float* so = a.self_in + 8 * (size_t)ref.gs;
             self_h = fmaxf(a.P.self_margin - so[0], 0.0f);
             if (self_h > 0.0f) { si = __float_as_int(so[1]); sj = __float_as_int(so[2]); snx = so[3]; sny = so[4]; snz = so[5]; }
         }
-        float world = 0.0f, minclr = 1000.0f;
+        float world = 0.0f;
         Slots sl;
         for (int jj = 0; jj < J; ++jj) {
             float T[12];
@@ -1125,10 +1257,9 @@ __global__ __launch_bounds__(64, 4) void k_cost(CostArgs a) {
                     auto rec = [&](float4& r0, float4& r1, float4& r2, float4& r3) {
                         r0 = s_obb[4 * arg]; r1 = s_obb[4 * arg + 1]; r2 = s_obb[4 * arg + 2]; r3 = s_obb[4 * arg + 3];
                     };
-                    const float hs = sphere_hinge_at<GRAD>(a, arg >= 0, rec, best, px, py, pz, sp.w, R.sph_id[s],
+                    const float hs = sphere_hinge_at<GRAD, false>(a, EsdfLayer(), arg >= 0, rec, best, px, py, pz, sp.w, R.sph_id[s],
                                                            use_obb, use_esdf, gx, gy, gz);
-                    if (a.clearance_only) minclr = fminf(minclr, hs);
-                    else world += hs;
+                    world += hs;
                     if (GRAD) {
                         if (si >= 0) {
                             const int id = R.sph_id[s];
@@ -1144,7 +1275,7 @@ __global__ __launch_bounds__(64, 4) void k_cost(CostArgs a) {
                     }
                 }
             }
-            if (GRAD && !a.clearance_only) {
+            if (GRAD) {
                 const bool nz = fx != 0.0f || fy != 0.0f || fz != 0.0f || tx != 0.0f || ty != 0.0f || tz != 0.0f;
                 if (G > 1 && wave_any(nz)) {
                     fx = group_sum(fx, G); fy = group_sum(fy, G); fz = group_sum(fz, G);
@@ -1161,7 +1292,7 @@ __global__ __launch_bounds__(64, 4) void k_cost(CostArgs a) {
                 }
             }
         }
-        if (GRAD && !a.clearance_only && sub == 0 && active) {
+        if (GRAD && sub == 0 && active) {
             // Reverse DFS sweep: every joint's subtree wrench is complete once
             // its descendants (higher DFS positions) have been folded in.
             for (int d = 0; d < D; ++d) dqs[d] = 0.0f;
@@ -1192,13 +1323,8 @@ __global__ __launch_bounds__(64, 4) void k_cost(CostArgs a) {
             }
             for (int d = 0; d < D; ++d) a.grad_out[base + (size_t)d * stride] = endpoint ? 0.0f : wt * dqs[d];
         }
-        if (a.clearance_only) {
-            minclr = group_min(minclr, G);
-            if (active && sub == 0) a.cost_out[ref.gs] = minclr;
-        } else {
-            world = group_sum(world, G);
-            if (active && sub == 0 && a.cost_out) a.cost_out[ref.gs] = wt * (world + self_h);
-        }
+        world = group_sum(world, G);
+        if (active && sub == 0 && a.cost_out) a.cost_out[ref.gs] = wt * (world + self_h);
         __syncthreads();   // records and q of this chunk are dead before the next load_state
     }
 }
@@ -1335,7 +1461,7 @@ __device__ __forceinline__ void grp_masks(const DRobot& R, const float4* __restr
             q0 = s_obb[4 * lane]; q1 = s_obb[4 * lane + 1]; q2 = s_obb[4 * lane + 2]; qh = s_obb[4 * lane + 3];
         }
         for (int k = 0; k < nk; ++k) {
-            const float4 ce = R.clu_enc[c0 + k];
+            const float4 ce = uload4(R.clu_enc, c0 + k);
             ObbMask mk;
             const float c0x = read_lane(cx, k), c0y = read_lane(cy, k), c0z = read_lane(cz, k);
             const float reach = band + ce.w + sqrtf(read_lane(d2, k)) * 1.0001f + 1e-5f;
@@ -1414,7 +1540,8 @@ __device__ __forceinline__ void grp_argmin(const float4* __restrict__ s_obb, con
 // keeps the other path's registers out of the sphere pass. TILED: some
 // problem's OBBs pass through LDS in tiles (a variant of its own, so the
 // folding across tiles costs the one-staging kernels no registers).
-template <bool GRAD, int WORLD, bool TILED>
+// ONE: the scene is a single trilinear ESDF layer without masks (esdf_single).
+template <bool GRAD, int WORLD, bool TILED, bool ONE = false>
 __device__ __forceinline__ void cost_grp(const CostArgs& a) {
     extern __shared__ float4 s_lds[];
     const DRobot& R = a.R;
@@ -1438,11 +1565,11 @@ __device__ __forceinline__ void cost_grp(const CostArgs& a) {
     const int sub = lane & (kGrp - 1);
     const int slot = lane / kGrp;
     float* Ts = s_T + slot * fstride;
-    const bool use_obb = (WORLD & 1) && a.P.use_obb != 0 && !a.clearance_only;
-    const bool use_esdf = (WORLD & 2) && (a.P.use_esdf != 0 || a.clearance_only) && a.S.n_voxel_layers > 0;
-    const bool want_grad = GRAD && !a.clearance_only;
+    const bool use_obb = (WORLD & 1) && a.P.use_obb != 0;
+    const bool use_esdf = (WORLD & 2) && a.P.use_esdf != 0 && a.S.n_voxel_layers > 0;
     const float wt = a.P.weight;
     const int cap = a.C.obb_cap;
+    const EsdfLayer layer = ONE ? EsdfLayer(a.S) : EsdfLayer();
     int cur_prob = -1, n_obb = 0, o0 = 0, o1 = 0, n_tiles = 1;
     int4 ch;
     ChunkCursor cur = chunk_cursor();
@@ -1462,7 +1589,7 @@ __device__ __forceinline__ void cost_grp(const CostArgs& a) {
         const long g = (long)ch.y + slot;
         const bool active = g < ch.z;
         stage_unit_ends(a.X, ch.w, s_end);
-        if (want_grad)
+        if (GRAD)
             for (int i = lane; i < kGrpStates * (J * 6 + kMaxDof + 1); i += kWave) s_w[i] = 0.0f;
         __syncthreads();
         StateRef ref = load_state(a.X, D, g, active, s_q, ch.w, s_end, ch.x, slot, kGrpStates, sub == 0);
@@ -1507,7 +1634,7 @@ __device__ __forceinline__ void cost_grp(const CostArgs& a) {
         }
         float self_h = 0.0f, snx = 0.0f, sny = 0.0f, snz = 0.0f;
         int si = -1, sj = -1;
-        if (a.self_in && active && !a.clearance_only) {
+        if (a.self_in && active) {
             const float* so = a.self_in + 8 * (size_t)ref.gs;
             self_h = fmaxf(a.P.self_margin - so[0], 0.0f);
             if (self_h > 0.0f) { si = __float_as_int(so[1]); sj = __float_as_int(so[2]); snx = so[3]; sny = so[4]; snz = so[5]; }
@@ -1516,7 +1643,7 @@ __device__ __forceinline__ void cost_grp(const CostArgs& a) {
         // places its sphere with its joint's frame and walks its cluster's
         // candidate mask for the argmin box (tiled: reads the folded argmin
         // and rebuilds its record from the scene when the gradient needs it).
-        float world = 0.0f, minclr = 1000.0f;
+        float world = 0.0f;
         // In this pass lane = 4 * sphere slot + state: the four states of a
         // sphere walk its cluster's mask together, so each quarter-wave of an
         // LDS record read touches 4 records (broadcast) instead of 16 (bank
@@ -1581,21 +1708,17 @@ __device__ __forceinline__ void cost_grp(const CostArgs& a) {
             };
             float gx, gy, gz;
             const float hs =
-                sphere_hinge_at<GRAD>(a, arg >= 0, rec, best, px, py, pz, sp.w, sid, use_obb, use_esdf, gx, gy, gz);
-            if (a.clearance_only) minclr = fminf(minclr, hs);
-            else world += hs;
-            if (want_grad) add_wrench(jj, sid, px, py, pz, t0.w, t1.w, t2.w, gx, gy, gz);
+                sphere_hinge_at<GRAD, ONE>(a, layer, arg >= 0, rec, best, px, py, pz, sp.w, sid, use_obb,
+                                      use_esdf, gx, gy, gz);
+            world += hs;
+            if (GRAD) add_wrench(jj, sid, px, py, pz, t0.w, t1.w, t2.w, gx, gy, gz);
         }
         // each state's partial sums sit in the lanes with its lane & 3; the
         // pairwise tree matches a 16-lane group sum's
-        for (int o = kGrpStates; o < kWave; o <<= 1) {
-            world += __shfl_xor(world, o);
-            minclr = fminf(minclr, __shfl_xor(minclr, o));
-        }
+        for (int o = kGrpStates; o < kWave; o <<= 1) world += __shfl_xor(world, o);
         world = __shfl(world, slot);
-        minclr = __shfl(minclr, slot);
         // 3. adjoint: subtree wrench of joint `sub` -> d cost / d q
-        if (want_grad) {
+        if (GRAD) {
             __syncthreads();
             float* dq = s_dq + slot * (kMaxDof + 1);
             // Subtree sums by one prefix scan over the group's lanes: lane
@@ -1652,11 +1775,7 @@ __device__ __forceinline__ void cost_grp(const CostArgs& a) {
                 a.grad_out[base + (size_t)sub * stride] = endpoint ? 0.0f : wt * dq[sub];
             }
         }
-        if (a.clearance_only) {
-            if (active && sub == 0) a.cost_out[ref.gs] = minclr;
-        } else {
-            if (active && sub == 0 && a.cost_out) a.cost_out[ref.gs] = wt * (world + self_h);
-        }
+        if (active && sub == 0 && a.cost_out) a.cost_out[ref.gs] = wt * (world + self_h);
         __syncthreads();   // frames, masks and wrenches of this chunk are dead before the next one
     }
 }
@@ -1670,9 +1789,107 @@ __global__ __launch_bounds__(64, TILED ? 1 : 4) void k_cost_grp(CostArgs a) {
 
 // ESDF-only launches (no OBB path): five waves per SIMD fit in the register
 // budget, which the lookups' memory latency rewards.
-template <bool GRAD>
+template <bool GRAD, bool ONE>
 __global__ __launch_bounds__(64, 5) void k_cost_grp_esdf(CostArgs a) {
-    cost_grp<GRAD, 2, false>(a);
+    cost_grp<GRAD, 2, false, ONE>(a);
+}
+
+// ===========================================================================
+// Minimum ESDF clearance (radius + margin; 1000 without a layer) of every
+// state, scene_min_clearance_runtime semantics (scene_collision.cuh:339-384).
+//
+// Bound by latency: a lane per state is too few waves (782 of them for 50,001
+// Baxter configurations, 121.5 us a call, and 96 us for 256), each one chain of
+// 15 joints and 75 lookups. So G lanes share a state: they take its joints'
+// sines in turn, walk the tree in step (every frame has the same bits as a lane
+// on its own gives it), leave the frames in LDS and take every G-th sphere each,
+// two of them with their grid loads in flight together: 49 us, and 14 for 256.
+// ONE: the scene is a single trilinear layer without masks (esdf_single).
+// ===========================================================================
+template <int G, bool ONE>
+__global__ __launch_bounds__(64) void k_clear(ClearArgs a) {
+    extern __shared__ float s_clr[];
+    constexpr int kN = kWave / G;             // states of the wave
+    const DRobot& R = a.R;
+    const int lane = lane_id(), sub = lane & (G - 1), slot = lane / G;
+    const int J = R.n_joints, D = R.n_dof, S = R.n_sph;
+    const int fstride = J * 12;
+    // [slot][J][12] frames; a joint's first two floats hold its sine and cosine until its frame is there
+    float* s_T = s_clr + slot * fstride;
+    float* s_q = s_clr + kN * fstride;   // [D][kN]
+    const long n = a.X.n_states;
+    const EsdfLayer layer = ONE ? EsdfLayer(a.S) : EsdfLayer();
+    for (long base = (long)blockIdx.x * kN; base < n; base += (long)gridDim.x * kN) {
+        const long g = base + slot;
+        const bool active = g < n;
+        load_state(a.X, D, active ? g : base, true, s_q, -1, nullptr, 0, slot, kN, sub == 0);
+        __syncthreads();
+        float best = 1000.0f;
+        float gx, gy, gz;
+        Slots sl;
+        for (int jj = sub; jj < J; jj += G) {
+            const int4 meta = R.jmeta[jj];
+            float sn = 0.0f, cs = 1.0f;
+            if (meta.x >= kXRot) sincosf(meta.y >= 0 ? s_q[meta.y * kN + slot] : 0.0f, &sn, &cs);
+            *reinterpret_cast<float2*>(s_T + 12 * jj) = make_float2(sn, cs);
+        }
+        __syncthreads();
+        for (int jj = 0; jj < J; ++jj) {
+            float T[12];
+            const i4u meta = uload<i4u>(R.jmeta, jj);
+            if (jj == 0) {
+                aff_identity(T);
+            } else {
+                float P[12], A[12];
+                sl.load(meta.w, P);
+                const float2 sc = *reinterpret_cast<const float2*>(s_T + 12 * jj);
+                joint_step_u(R.ft, jj, meta.x, meta.y >= 0 ? s_q[meta.y * kN + slot] : 0.0f, sc.x, sc.y, A);
+                aff_compose(P, A, T);
+            }
+            sl.store(meta.z, T);
+            if (sub == (jj & (G - 1))) {
+                float4* d = reinterpret_cast<float4*>(s_T + 12 * jj);
+                d[0] = make_float4(T[0], T[1], T[2], T[3]);
+                d[1] = make_float4(T[4], T[5], T[6], T[7]);
+                d[2] = make_float4(T[8], T[9], T[10], T[11]);
+            }
+        }
+        __syncthreads();
+        auto place = [&](const float4& sp, int jj, float& px, float& py, float& pz) {
+            const float4* Tq = reinterpret_cast<const float4*>(s_T + 12 * jj);
+            const float4 t0 = Tq[0], t1 = Tq[1], t2 = Tq[2];
+            px = fmaf(t0.x, sp.x, fmaf(t0.y, sp.y, fmaf(t0.z, sp.z, t0.w)));
+            py = fmaf(t1.x, sp.x, fmaf(t1.y, sp.y, fmaf(t1.z, sp.z, t1.w)));
+            pz = fmaf(t2.x, sp.x, fmaf(t2.y, sp.y, fmaf(t2.z, sp.z, t2.w)));
+        };
+        if (ONE) {
+            for (int s = sub; s < S; s += 2 * G) {
+                const bool two = s + G < S;
+                const int s2 = two ? s + G : s;
+                const float4 spa = R.sph[s], spb = R.sph[s2];
+                const int ja = R.sph_jnt[s], jb = R.sph_jnt[s2];
+                EsdfTap ta, tb;
+                float px, py, pz;
+                place(spa, ja, px, py, pz);
+                ta.load(layer, px, py, pz, true);
+                place(spb, jb, px, py, pz);
+                tb.load(layer, px, py, pz, two);
+                best = fminf(best, ta.value(spa.w + a.margin));
+                best = fminf(best, tb.value(spb.w + a.margin));
+            }
+        } else {
+            for (int s = sub; s < S; s += G) {
+                const float4 sp = R.sph[s];
+                float px, py, pz;
+                place(sp, R.sph_jnt[s], px, py, pz);
+                best = fminf(best, esdf_clearance(a.S, px, py, pz, sp.w + a.margin, R.sph_id[s], false, gx, gy, gz));
+            }
+        }
+#pragma unroll
+        for (int o = 1; o < G; o <<= 1) best = fminf(best, __shfl_xor(best, o));
+        if (active && sub == 0) a.out[g] = best;
+        __syncthreads();   // q and the frames are read before the next round's
+    }
 }
 
 // ===========================================================================
@@ -2748,21 +2965,22 @@ size_t lds_bytes_grp(int obb_cap, int n_dof, int n_joints, int n_sph, int n_clu,
     return lds_floats_grp(obb_cap, n_dof, n_joints, n_sph, n_clu, grad, tiled) * sizeof(float);
 }
 
-// Variant table: [grad][world - 1][tiled] (ESDF-only launches stage no OBBs).
+// Variant table: [grad][world - 1][tiled] (ESDF-only launches stage no OBBs;
+// there the third index says whether the scene is a single layer, esdf_single).
 const void* grp_kernel(bool grad, int world, bool tiled) {
     static const void* const tab[2][3][2] = {
         {{(const void*)k_cost_grp<false, 1, false>, (const void*)k_cost_grp<false, 1, true>},
-         {(const void*)k_cost_grp_esdf<false>, (const void*)k_cost_grp_esdf<false>},
+         {(const void*)k_cost_grp_esdf<false, false>, (const void*)k_cost_grp_esdf<false, true>},
          {(const void*)k_cost_grp<false, 3, false>, (const void*)k_cost_grp<false, 3, true>}},
         {{(const void*)k_cost_grp<true, 1, false>, (const void*)k_cost_grp<true, 1, true>},
-         {(const void*)k_cost_grp_esdf<true>, (const void*)k_cost_grp_esdf<true>},
+         {(const void*)k_cost_grp_esdf<true, false>, (const void*)k_cost_grp_esdf<true, true>},
          {(const void*)k_cost_grp<true, 3, false>, (const void*)k_cost_grp<true, 3, true>}}};
     return tab[grad ? 1 : 0][world - 1][tiled ? 1 : 0];
 }
 
 int grp_world(const CostArgs& a) {
-    const bool obb = a.P.use_obb != 0 && !a.clearance_only && a.S.n_obbs > 0;
-    const bool esdf = (a.P.use_esdf != 0 || a.clearance_only) && a.S.n_voxel_layers > 0;
+    const bool obb = a.P.use_obb != 0 && a.S.n_obbs > 0;
+    const bool esdf = a.P.use_esdf != 0 && a.S.n_voxel_layers > 0;
     return obb && esdf ? 3 : esdf ? 2 : 1;
 }
 
@@ -2788,10 +3006,29 @@ hipError_t launch_cost_grp(const CostArgs& a, int grid, hipStream_t s, hipEvent_
     const size_t lds = lds_bytes_grp(a.C.obb_cap, a.R.n_dof, a.R.n_joints, a.R.n_sph, a.R.n_clu, a.grad != 0,
                                      a.C.tiled != 0);
     const int world = grp_world(a);
-    const bool tiled = a.C.tiled != 0 && world != 2;
+    const bool tiled = world == 2 ? esdf_single(a.S) : a.C.tiled != 0;   // the variant table's third index
     grid = std::max(1, std::min(grid, grid_cost_grp(a.grad != 0, world, tiled, lds)));   // persistent: occupancy x CUs
     CostArgs arg = a;
     return launch_args(grp_kernel(a.grad != 0, world, tiled), grid, lds, s, &arg, t0, t1);
+}
+
+// Lanes per state: 16 up to two waves a SIMD of them, else 8. Measured, us a call,
+// Baxter (Panda): 256 configurations 13.7 against 15.3 (11 and 11), 8,192 19.6
+// against 21.0 (14.3, 14.9), 20,000 35.8 against 26.6 (26.6, 21.9), 500,000 502
+// against 329 (367, 288); 4 lanes lie within 15% of 8 from 50,000 on, and one
+// lane needs 500,000 to be as fast (302, 318).
+hipError_t launch_clear(const ClearArgs& a, hipStream_t s) {
+    const long n = a.X.n_states;
+    if (n <= 0) return hipSuccess;
+    const int G = n * 16 <= (long)device_cus() * 4 * 2 * kWave ? 16 : 8;
+    const int kn = kWave / G;
+    const bool one = esdf_single(a.S);
+    const void* k = G == 8 ? (one ? (const void*)k_clear<8, true> : (const void*)k_clear<8, false>)
+                           : (one ? (const void*)k_clear<16, true> : (const void*)k_clear<16, false>);
+    const size_t lds = sizeof(float) * kn * ((size_t)a.R.n_dof + 12 * (size_t)a.R.n_joints);
+    const long blocks = std::min((n + kn - 1) / kn, (long)device_cus() * 32);
+    ClearArgs arg = a;
+    return launch_args(k, (int)blocks, lds, s, &arg, nullptr, nullptr);
 }
 
 hipError_t launch_self(const SelfArgs& a, hipStream_t s) {

@@ -167,11 +167,16 @@ struct CostArgs {
     DCostParams P;
     int group;                  // lanes per state (power of two <= kMaxGroup): a state's spheres are split over them
     int grad;                   // also compute d cost / d q
-    int clearance_only;         // write min ESDF clearance (+margin) instead of cost
-    float margin;               // clearance_only: radius margin
     const float* self_in;       // [n_states][8] self pass output (nullable)
-    float* cost_out;            // [n_states] weighted cost (or clearance)
+    float* cost_out;            // [n_states] weighted cost
     float* grad_out;            // layout of X (kSrcConfig: [n][D]; kSrcTraj: theta layout)
+};
+
+// Minimum ESDF clearance of states X in flat order (any source but waypoint-major).
+struct ClearArgs {
+    DRobot R; DScene S; DStates X;
+    float margin;               // added to every radius
+    float* out;                 // [n_states]
 };
 
 struct SelfArgs {
@@ -193,6 +198,7 @@ hipError_t launch_collide(const CollideArgs& a, int grid, hipStream_t s, hipEven
 hipError_t launch_cost(const CostArgs& a, int grid, hipStream_t s, hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr);
 hipError_t launch_cost_grp(const CostArgs& a, int grid, hipStream_t s, hipEvent_t t0 = nullptr,
                            hipEvent_t t1 = nullptr);
+hipError_t launch_clear(const ClearArgs& a, hipStream_t s);
 hipError_t launch_self(const SelfArgs& a, hipStream_t s);
 hipError_t launch_fill_i32(int* p, int v, long n, hipStream_t s);
 hipError_t launch_add_u32(unsigned* p, unsigned v, hipStream_t s);   // *p += v (one thread)

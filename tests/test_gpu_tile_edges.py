@@ -69,3 +69,28 @@ def test_esdf_brick_remainders(dims, boxes):
     ref = PO.esdf_from_obbs(obbs.obb_dims, obbs.obb_pose, prm, pose)
     assert got.shape == (dims[0] * dims[1] * dims[2],)
     assert np.max(np.abs(got - ref.reshape(-1)) / np.maximum(np.abs(ref.reshape(-1)), 0.05)) < 1e-5
+
+
+@pytest.mark.parametrize("name,n,layers,interp", [("panda", 1, 1, 1), ("panda", 5, 1, 0), ("baxter", 9, 1, 1),
+                                                  ("fetch", 8193, 1, 1), ("baxter", 8191, 2, 1), ("panda", 33000, 1, 1)])
+def test_clearance_lane_groups(robots, name, n, layers, interp):
+    """16 lanes a state up to two waves a SIMD, 8 above; odd state and sphere
+    counts; the single-layer lookup and the general one."""
+    from parity_common import assert_values, clearance_den
+    from prismplan_amd.planning_scene import HostScene
+    rob = robots[name]
+    rng = np.random.default_rng(n)
+    q = W.uniform_configs(rng, rob.arrays, n)
+    boxes = W.random_obbs(rng, 12, half_lo=0.02, half_hi=0.15)
+    prms, poses, feats = [], [], []
+    for k in range(layers):
+        prm, pose = W.esdf_grid(center=(0.5 + 0.1 * k, 0.0, 0.5), n=48, voxel=0.03)
+        prms.append(prm[0]); poses.append(pose[0])
+        feats.append(PO.esdf_from_obbs(boxes.obb_dims, boxes.obb_pose, prm[0], pose[0]).astype(np.float32))
+    hs = HostScene(voxel_params=np.stack(prms), voxel_pose=np.stack(poses), voxel_enable=np.ones(layers, np.uint8),
+                   voxel_features=np.stack(feats), esdf_interp=interp)
+    got = S.min_clearance_batched(S.Plan.configs(rob, n), S.DeviceScene.from_host(hs), torch.from_numpy(q).to(DEV),
+                                  collision_margin=0.01).cpu().numpy()
+    k = np.unique(np.linspace(0, n - 1, min(n, 3000)).astype(int))
+    ref, amb = PO.Oracle(rob.arrays, hs).min_clearance(q[k], margin=0.01, with_amb=True)
+    assert_values(got[k], ref, amb, clearance_den(ref), f"clearance {name} n={n}")
