@@ -310,8 +310,8 @@ ppl_status ppl_tune_cache_file(const char* path);
  * the plan's batched check on `stream` for each OBB staging tile (the largest
  * problem's OBBs in one staging, then 128, 64 and 32 records below that; the
  * stagings of a problem then pass through LDS in turn) and each grid form
- * (0: persistent at occupancy, 1: twice that, 2: one workgroup per 64-state
- * chunk), keeps the fastest for this plan's later any-collision calls and
+ * (0: up to eight times the workgroups the chip holds at once, 1: twice
+ * them, 2: one workgroup per 64-state chunk), keeps the fastest for this plan's later any-collision calls and
  * records it in the tuning cache under the robot's tables, the largest
  * problem's OBB count and the GPU architecture; when the cache already holds
  * a choice for that key it is adopted without timing (*best_ms: the time

@@ -233,7 +233,7 @@ ppl_status scene_from_view(const ppl_scene_view* v, DScene& S) {
     return PPL_OK;
 }
 
-enum KernelKind { kKCollide, kKCost, kKCostGrad, kKCostGrp, kKCostGrpGrad };
+enum KernelKind { kKCost, kKCostGrad, kKCostGrp, kKCostGrpGrad };
 
 // LDS OBB records of a launch whose largest problem has max_obbs OBBs: all of
 // them, or one tile of kMaxObbLds when they do not fit (tiled launch).
@@ -241,15 +241,13 @@ int obb_tile(int max_obbs) { return std::max(1, std::min(max_obbs, kMaxObbLds));
 
 // Persistent grid for a kernel family at the LDS footprint of this launch.
 int grid_for(KernelKind k, const DRobot& R, int obb_cap, int G) {
-    if (k == kKCollide) return grid_collide(lds_bytes(obb_cap, R.n_dof));
     if (k == kKCostGrp || k == kKCostGrpGrad) return INT_MAX;   // launch_cost_grp caps it per kernel variant
     const bool grad = k == kKCostGrad;
     return grid_cost(R.n_joints, grad, lds_bytes_cost(obb_cap, R.n_dof, R.n_joints, G, grad));
 }
 
 // max_obbs: OBBs of the largest problem of the launch.
-DChunks implicit_chunks(long n_states, KernelKind k, const DRobot& R, int max_obbs, int* grid_out, int G = 1) {
-    const int grid_cap = grid_for(k, R, obb_tile(max_obbs), G);
+DChunks implicit_chunks(long n_states, int grid_cap, int max_obbs, int* grid_out, int G = 1) {
     DChunks C{};
     C.obb_cap = obb_tile(max_obbs);
     C.tiled = max_obbs > kMaxObbLds;
@@ -259,6 +257,21 @@ DChunks implicit_chunks(long n_states, KernelKind k, const DRobot& R, int max_ob
     C.obb_off = nullptr;
     *grid_out = std::max(1, std::min(grid_cap, C.n_chunks));
     return C;
+}
+
+// Workgroups of an any-collision launch, in units of what the chip holds at
+// once. Chunks differ in cost by the joint their last state is decided at, so
+// a grid the chip holds at once ends with its unluckiest wave (16,384 edges
+// among 64 boxes: waves lived 121 us on average in a launch of 252); with more
+// the dispatcher evens them out (232 us at once, 214 twice, 184 from four times on,
+// one workgroup per chunk there).
+constexpr int kCollideWaves = 8;
+
+// Implicit chunks of an any-collision launch over a whole scene. n_states an
+// upper bound (counted on the device): the grid stays at what the chip holds.
+DChunks collide_chunks(long n_states, const DRobot& R, const DScene& S, int* grid_out, bool bound = false) {
+    return implicit_chunks(n_states, (bound ? 1 : kCollideWaves) * grid_collide(R, S, obb_tile(S.n_obbs)), S.n_obbs,
+                           grid_out);
 }
 
 // The cost kernel over n_states implicit chunks: k_cost with one lane per
@@ -299,7 +312,8 @@ hipError_t launch_cost_flat(CostArgs& a, long n_states, hipStream_t s) {
     int grid = 0;
     const bool tiled = a.S.n_obbs > kMaxObbLds;
     const KernelKind k = tiled ? (a.grad ? kKCostGrpGrad : kKCostGrp) : (a.grad ? kKCostGrad : kKCost);
-    a.C = implicit_chunks(n_states, k, a.R, a.S.n_obbs, &grid, tiled ? kGrp : 1);
+    const int G = tiled ? kGrp : 1;
+    a.C = implicit_chunks(n_states, grid_for(k, a.R, obb_tile(a.S.n_obbs), G), a.S.n_obbs, &grid, G);
     a.group = tiled ? kGrp : 1;
     return tiled ? launch_cost_grp(a, grid, s) : launch_cost(a, grid, s);
 }
@@ -451,9 +465,9 @@ DChunks plan_chunks(const ppl_plan_s* P, KernelKind k, int max_obbs, int G, int*
 // The any-collision launch shape of plan P for problems of up to max_obbs
 // OBBs: this plan's tuned or set shape, else the tuning cache's entry for the
 // robot, OBB count and GPU, else the built-in one (every OBB of a problem in
-// one staging, persistent grid at occupancy). tile: OBB records per LDS
-// staging; gmode 0 persistent grid at occupancy, 1 twice that, 2 one
-// workgroup per chunk.
+// one staging, grid form 0). tile: OBB records per LDS staging; gmode 0 up to
+// kCollideWaves times the workgroups the chip holds at once, 1 twice them, 2
+// one workgroup per chunk.
 void collide_shape(ppl_plan_s* P, int max_obbs, int* tile, int* gmode) {
     if (P->shape_src != 2 && P->shape_obbs != max_obbs) {
         P->shape_obbs = max_obbs;
@@ -471,7 +485,7 @@ void collide_shape(ppl_plan_s* P, int max_obbs, int* tile, int* gmode) {
     *gmode = P->cgrid;
 }
 
-DChunks plan_collide_chunks(ppl_plan_s* P, int max_obbs, int* grid_out) {
+DChunks plan_collide_chunks(ppl_plan_s* P, const DScene& S, int max_obbs, int* grid_out) {
     int tile = 0, gm = 0;
     collide_shape(P, max_obbs, &tile, &gm);
     DChunks C{};
@@ -481,8 +495,8 @@ DChunks plan_collide_chunks(ppl_plan_s* P, int max_obbs, int* grid_out) {
     C.n_chunks = P->n_chunks[0];
     C.chunk = kWave;
     C.obb_off = P->d_obb_off;
-    const int occ = grid_collide(lds_bytes(tile, P->robot->R.n_dof));
-    const int g = gm == 2 ? C.n_chunks : (gm == 1 ? 2 * occ : occ);
+    const int occ = grid_collide(P->robot->R, S, tile);
+    const int g = gm == 2 ? C.n_chunks : (gm == 1 ? 2 * occ : kCollideWaves * occ);
     *grid_out = std::max(1, std::min(g, C.n_chunks));
     return C;
 }
@@ -993,6 +1007,11 @@ ppl_status ppl_robot_create(const ppl_robot_desc* d, ppl_robot* out) try {
     R.sph_clu = reinterpret_cast<const int*>(b + o_sclu);
     R.clu_jnt = reinterpret_cast<const int*>(b + o_cjnt);
     R.scene_gate_fused = scene_gate_fused ? 1 : 0;
+    R.line = 1;
+    for (int k = 1; k < J; ++k) {
+        const int par = pos[parents[dfs[k]]];
+        if (par != 0 && par != k - 1) R.line = 0;
+    }
     R.self_gate_implied = self_gate_implied ? 1 : 0;
     R.n_cpb = (int)cpb.size();
     r->n_slots = n_slots;
@@ -1108,7 +1127,7 @@ ppl_status ppl_check_collision_scene(ppl_robot r, const ppl_scene_view* view, co
     a.X.cfg = r->d_cfg.as<float>();
     a.X.cfg_stride = D;
     int grid = 0;
-    a.C = implicit_chunks(n, kKCollide, r->R, S.n_obbs, &grid);
+    a.C = collide_chunks(n, r->R, S, &grid);
     a.margin = margin;
     a.mode = 0;
     a.out = r->d_out.as<uint8_t>();
@@ -1248,7 +1267,7 @@ ppl_status ppl_edge_eval_evaluate(ppl_edge_eval ev, const float* h_from, const f
         a.S = ev->S;
         a.X = X;
         int grid = 0;
-        a.C = implicit_chunks(total, kKCollide, r->R, ev->S.n_obbs, &grid);
+        a.C = collide_chunks(total, r->R, ev->S, &grid);
         a.margin = p->collision_margin;
         a.mode = 1;
         a.skip_resolved = 1;
@@ -1875,7 +1894,7 @@ ppl_status dense_check_setup(const ppl_plan_s* P, const DScene& S, float step, f
     dc.va.R = P->robot->R;
     dc.va.S = S;
     dc.va.X = dc.Xd;
-    dc.va.C = implicit_chunks((long)n_dense, kKCollide, P->robot->R, S.n_obbs, &dc.vgrid);
+    dc.va.C = collide_chunks((long)n_dense, P->robot->R, S, &dc.vgrid, true);
     dc.va.margin = margin;
     dc.va.mode = 1;
     dc.va.skip_resolved = 1;
@@ -2329,7 +2348,7 @@ ppl_status ppl_check_collision_batched(ppl_plan P, const ppl_scene_view* view, c
     a.S = S;
     a.X = X;
     int grid = 0;
-    a.C = plan_collide_chunks(P, plan_obb_cap(P, S), &grid);
+    a.C = plan_collide_chunks(P, S, plan_obb_cap(P, S), &grid);
     a.margin = margin;
     a.mode = 0;
     a.out = d_out;
@@ -2370,7 +2389,7 @@ ppl_status ppl_edge_check_batched(ppl_plan P, const ppl_scene_view* view, const 
     a.S = S;
     a.X = X;
     int grid = 0;
-    a.C = plan_collide_chunks(P, plan_obb_cap(P, S), &grid);
+    a.C = plan_collide_chunks(P, S, plan_obb_cap(P, S), &grid);
     a.margin = prm->collision_margin;
     a.mode = 1;
     a.skip_resolved = prm->skip_resolved;
@@ -2523,7 +2542,7 @@ ppl_status batch_cc_impl(ppl_robot r, const DScene& S, const float* d_samples, i
         a.self_hit = self;
     }
     int grid = 0;
-    a.C = implicit_chunks(n, kKCollide, r->R, S.n_obbs, &grid);
+    a.C = collide_chunks(n, r->R, S, &grid);
     a.margin = margin;
     a.mode = 0;
     a.out = d_cc;
@@ -2668,7 +2687,7 @@ ppl_status ppl_mitstar_edge_cc(ppl_robot r, const ppl_scene_view* view, const fl
         a.S = S;
         a.X = X;
         int grid = 0;
-        a.C = implicit_chunks((long)total, kKCollide, r->R, S.n_obbs, &grid);
+        a.C = collide_chunks((long)total, r->R, S, &grid);
         a.C.unit_hint = hint;
         a.margin = margin;
         a.mode = 1;

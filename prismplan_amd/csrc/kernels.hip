@@ -178,6 +178,42 @@ __device__ __forceinline__ void fk_joint(const DRobot& R, int jj, const float* s
     sl.store(meta.z, T);
 }
 
+// The same walk for a model whose joints each hang on the joint before them in
+// DFS order or on the root (DRobot::line; arms of a torso are such lines): the
+// parent's frame is the last one, or the root's identity, so T itself carries
+// the state from joint to joint and no slots are held. The compositions are
+// fk_joint's, so the frames have the same bits.
+template <bool LINE>
+struct FkWalk {
+    Slots sl;
+    __device__ __forceinline__ void step(const DRobot& R, int jj, const float* s_q, float* T, int4& meta) {
+        fk_joint(R, jj, s_q, sl, T, meta);
+    }
+};
+template <>
+struct FkWalk<true> {
+    __device__ __forceinline__ void step(const DRobot& R, int jj, const float* s_q, float* T, int4& meta) {
+        const i4u m = uload<i4u>(R.jmeta, jj);
+        meta = make_int4(m.x, m.y, m.z, m.w);
+        if (jj == 0) {
+            aff_identity(T);
+            return;
+        }
+        float P[12], S[12];
+        if (uload<int>(R.parent, jj) == 0) {
+            aff_identity(P);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 12; ++k) P[k] = T[k];
+        }
+        const float q = meta.y >= 0 ? s_q[meta.y * kWave] : 0.0f;
+        float s = 0.0f, c = 0.0f;
+        if (meta.x >= kXRot) sincosf(q, &s, &c);
+        joint_step_u(R.ft, jj, meta.x, q, s, c, S);
+        aff_compose(P, S, T);
+    }
+};
+
 // ---------------------------------------------------------------------------
 // OBB staging: enabled OBBs of [o0, o1) -> LDS records (see ppl_internal.hpp)
 // ---------------------------------------------------------------------------
@@ -201,7 +237,9 @@ __device__ __forceinline__ void obb_record(const DScene& S, int o, float4* rec) 
 }
 
 // Stages the enabled OBBs of [o0, o1) (at most cap of them: callers pass
-// ranges of at most cap OBBs) and returns their count.
+// ranges of at most cap OBBs) and returns their count. STRIDE: float4s from one
+// record to the next.
+template <int STRIDE = 4>
 __device__ int stage_obbs(const DScene& S, int o0, int o1, float4* s_obb, int cap) {
     const int lane = lane_id();
     int n = 0;
@@ -219,7 +257,7 @@ __device__ int stage_obbs(const DScene& S, int o0, int o1, float4* s_obb, int ca
         const unsigned long long m = __ballot(ok);
         if (ok) {
             const int pos = n + __popcll(m & ((1ull << lane) - 1ull));
-            if (pos < cap) obb_record(d4, p0, p1, o, s_obb + 4 * pos);
+            if (pos < cap) obb_record(d4, p0, p1, o, s_obb + STRIDE * pos);
         }
         n += __popcll(m);
     }
@@ -525,6 +563,19 @@ __device__ __forceinline__ int find_unit(const int* off, int n, long g, int u0, 
     return u;
 }
 
+// out(d, get(d)) for d < n, eight loads in flight at a time (a plain loop waits
+// for each one; past the end the last is loaded and written again).
+template <class Get, class Out>
+__device__ __forceinline__ void each_dof(int n, const Get& get, const Out& out) {
+    for (int d0 = 0; d0 < n; d0 += 8) {
+        float v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = get(min(d0 + k, n - 1));
+#pragma unroll
+        for (int k = 0; k < 8; ++k) out(min(d0 + k, n - 1), v[k]);
+    }
+}
+
 // Writes q_d into s_q[d * 64 + lane] for d < D (inactive lanes write nothing).
 // g is the chunk-order index; prob the chunk's problem (waypoint-major plans).
 // qcol / qstride: where q_d goes, s_q[d * qstride + qcol] (default: the
@@ -538,6 +589,7 @@ __device__ __forceinline__ StateRef load_state(const DStates& X, int D, long g, 
     const int lane = qcol >= 0 ? qcol : lane_id();
     const int nd = store ? D : 0;   // dimensions to write
     if (!active) return ref;
+    auto put = [&](int d, float v) { s_q[d * qstride + lane] = v; };
     if (X.source == kSrcDense) {
         int d0, d1;
         const int b = find_unit(X.dense_off, X.n_traj, g, u0, s_end, &d0, &d1);
@@ -550,14 +602,14 @@ __device__ __forceinline__ StateRef load_state(const DStates& X, int D, long g, 
         ref.u0 = d0;
         const float* th = X.theta + (size_t)t0 * D;
         if (f >= (T - 1) * ns) {
-            for (int d = 0; d < nd; ++d) s_q[d * qstride + lane] = th[(size_t)d * T + T - 1];
+            each_dof(nd, [&](int d) { return th[(size_t)d * T + T - 1]; }, put);
         } else {
             const int seg = f / ns, sub = f - seg * ns;
             const float frac = __fdiv_rn((float)sub, (float)ns);
-            for (int d = 0; d < nd; ++d) {
+            each_dof(nd, [&](int d) {
                 const float x0 = th[(size_t)d * T + seg], x1 = th[(size_t)d * T + seg + 1];
-                s_q[d * qstride + lane] = __fadd_rn(x0, __fmul_rn(__fsub_rn(x1, x0), frac));
-            }
+                return __fadd_rn(x0, __fmul_rn(__fsub_rn(x1, x0), frac));
+            }, put);
         }
         return ref;
     }
@@ -578,8 +630,7 @@ __device__ __forceinline__ StateRef load_state(const DStates& X, int D, long g, 
         const float t = __fdiv_rn((float)(2 * (kk - (1 << lvl)) + 1), (float)(1 << (lvl + 1)));
         const float* a = X.cfg + (size_t)X.node_src[e] * X.cfg_stride;
         const float* b = X.cfg + (size_t)X.node_dst[e] * X.cfg_stride;
-        for (int d = 0; d < nd; ++d)
-            s_q[d * qstride + lane] = __fadd_rn(__fmul_rn(a[d], 1.0f - t), __fmul_rn(b[d], t));
+        each_dof(nd, [&](int d) { return __fadd_rn(__fmul_rn(a[d], 1.0f - t), __fmul_rn(b[d], t)); }, put);
         return ref;
     }
     if (X.source == kSrcTraj && X.wmajor) {
@@ -592,14 +643,14 @@ __device__ __forceinline__ StateRef load_state(const DStates& X, int D, long g, 
         ref.u0 = (long)pr.w + (long)r * pr.z;
         ref.gs = ref.u0 + t;
         const float* th = X.theta + (size_t)ref.u0 * D;
-        for (int d = 0; d < nd; ++d) s_q[d * qstride + lane] = th[(size_t)d * pr.z + t];
+        each_dof(nd, [&](int d) { return th[(size_t)d * pr.z + t]; }, put);
         return ref;
     }
     if (X.source == kSrcConfig) {
         ref.unit = (int)g;
         ref.u0 = g;
         const float* q = X.cfg + (size_t)g * X.cfg_stride;
-        for (int d = 0; d < nd; ++d) s_q[d * qstride + lane] = q[d];
+        each_dof(nd, [&](int d) { return q[d]; }, put);
     } else if (X.source == kSrcEdge) {
         int b0, b1;
         const int e = find_unit(X.edge_off, X.n_edges, g, u0, s_end, &b0, &b1);
@@ -611,7 +662,7 @@ __device__ __forceinline__ StateRef load_state(const DStates& X, int D, long g, 
         const float t = ref.n > 1 ? (float)ref.k / (float)(ref.n - 1) : 0.0f;
         const float* a = X.from + (size_t)e * D;
         const float* b = X.to + (size_t)e * D;
-        for (int d = 0; d < nd; ++d) s_q[d * qstride + lane] = fmaf(t, b[d] - a[d], a[d]);
+        each_dof(nd, [&](int d) { return fmaf(t, b[d] - a[d], a[d]); }, put);
     } else {
         int t0, t1;
         const int b = find_unit(X.traj_off, X.n_traj, g, u0, s_end, &t0, &t1);
@@ -621,7 +672,7 @@ __device__ __forceinline__ StateRef load_state(const DStates& X, int D, long g, 
         ref.k = (int)(g - t0);
         ref.n = Tn;
         const float* th = X.theta + (size_t)t0 * D;
-        for (int d = 0; d < nd; ++d) s_q[d * qstride + lane] = th[(size_t)d * Tn + ref.k];
+        each_dof(nd, [&](int d) { return th[(size_t)d * Tn + ref.k]; }, put);
     }
     return ref;
 }
@@ -689,6 +740,30 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// Maximum over the 16 lanes of a row (lanes 16 k .. 16 k + 15), by row rotations.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+    const int i = __float_as_int(v);
+    return __int_as_float(__builtin_amdgcn_update_dpp(i, i, CTRL, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float row_max(float v) {
+    v = fmaxf(v, dpp<0x128>(v));
+    v = fmaxf(v, dpp<0x124>(v));
+    v = fmaxf(v, dpp<0x122>(v));
+    return fmaxf(v, dpp<0x121>(v));
+}
+
+// A row's 16 bits of a ballot (row: its first lane).
+__device__ __forceinline__ unsigned row_bits(unsigned long long m, int row) {
+    const unsigned w = row >= 32 ? (unsigned)(m >> 32) : (unsigned)m;
+    return (w >> (row & 16)) & 0xFFFFu;
+}
+
+// Lanes below this one set in a ballot.
+__device__ __forceinline__ int rank_below(unsigned long long m) {
+    return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
@@ -699,18 +774,46 @@ __device__ __forceinline__ float wave_sum(float v) {
 // Any-collision: two-phase gate semantics (two_phase_cc.cuh:57-138 with the
 // check kernel's environment pass, pRRTC.cu:2337-2386).
 // ===========================================================================
-// Five waves per SIMD (95 VGPRs, no spills): the chunk loads and the joint
-// loop's LDS reads leave half the wave time waiting, which a fifth resident
-// wave hides better than the register room four waves would give.
-__global__ __launch_bounds__(64, 5) void k_collide(CollideArgs a) {
+// A lane per state walks the joints; per joint, three steps narrow the (state,
+// box) pairs down to the exact sphere tests:
+//  1. each row of 16 lanes holds 16 consecutive states, whose approximate
+//     spheres lie within rw of a middle one's centre c0: every box one of them
+//     overlaps lies within rw + r of c0 (slack covers rounding). The row's
+//     lanes test 16 boxes at once;
+//  2. each lane tests its own approximate sphere against its row's candidates;
+//  3. the pairs that hit are queued in LDS and taken 64 at a time, one pair
+//     per lane (fewer pairs: several lanes share one, each a part of the
+//     joint's spheres), with the frame out of the state's own lane.
+// Bound by VALU and SALU issue. The whole wave used to share one candidate
+// set, and tested the exact spheres of a pair in all lanes as soon as one lane
+// had it: on 16,384 edges among 64 boxes a wave went through 100 candidates
+// and 12 exact boxes, of which its states needed 2.7 x 64 pairs; on uncorrelated
+// configurations (20 boxes) 89 and 31, needing 1.4 x 64. Together with the
+// scalar table loads and the grid (kCollideWaves): the edges 321 -> 179 us a
+// call, 262,144 configurations of 64 requests 135 -> 48 us, 11 densified
+// validity passes of 256 trajectories 258 -> 170 us each.
+// Records lie five float4s apart: the 16 boxes that a row's lanes read at once
+// then start in different LDS banks (four apart they shared four of them, and
+// conflicts took 53 us of the CU's LDS time on the edges above).
+constexpr int kObbRec = 5;
+
+// ESDF: the scene has voxel layers (a variant of its own: the lookups cost the
+// box-only kernel registers).
+// LINE: the model is a line of joints (FkWalk), which saves the slots' registers.
+template <bool ESDF, bool LINE>
+__global__ __launch_bounds__(64, 4) void k_collide(CollideArgs a) {
     extern __shared__ float4 s_lds[];
     float4* s_obb = s_lds;
-    float* s_q = reinterpret_cast<float*>(s_lds + 4 * a.C.obb_cap);
+    float4* s_sph = s_lds + kObbRec * a.C.obb_cap;                    // [S]
+    float* s_q = reinterpret_cast<float*>(s_sph + a.R.n_sph);
     const DRobot& R = a.R;
     const int lane = lane_id();
     const int J = R.n_joints, D = R.n_dof;
-    int* s_end = reinterpret_cast<int*>(s_q + D * kWave);
-    const bool has_esdf = a.S.n_voxel_layers > 0;
+    int* s_end = reinterpret_cast<int*>(s_q + D * kWave);       // [2][64] unit ends, then
+    int* s_queue = s_end;                                       // [128] pairs: lane | box << 8
+    int* s_hit = s_end + 2 * kWave;                             // [64] states hit in a flush
+    const int row = lane & 48;                                  // the lane's row of 16
+    for (int k = lane; k < R.n_sph; k += kWave) s_sph[k] = R.sph[k];
     const uint8_t* acm = a.S.sphere_obb_acm;
     const int cap = a.C.obb_cap;
     int cur_prob = -1, n_obb = 0, o0 = 0, o1 = 0, n_tiles = 1;
@@ -732,7 +835,7 @@ __global__ __launch_bounds__(64, 5) void k_collide(CollideArgs a) {
             n_tiles = uniform(obb_tiles(o0, o1, cap));
             if (n_tiles == 1) {
                 __syncthreads();
-                n_obb = uniform(stage_obbs(a.S, o0, o1, s_obb, cap));
+                n_obb = uniform(stage_obbs<kObbRec>(a.S, o0, o1, s_obb, cap));
             }
             cur_prob = ch.x;
         }
@@ -752,6 +855,7 @@ __global__ __launch_bounds__(64, 5) void k_collide(CollideArgs a) {
         }
         if (have_n) prefetch_unit_ends(a.X, chn.w, pf_end, pf_beg);
         __syncthreads();
+        s_hit[lane] = 0;
         // A problem with more OBBs than one staging holds is checked tile by
         // tile (FK redone per tile); bit jj of `flagged`: joint jj's
         // approximate spheres hit an OBB of an earlier tile, which the ESDF
@@ -762,115 +866,129 @@ __global__ __launch_bounds__(64, 5) void k_collide(CollideArgs a) {
             if (n_tiles > 1) {
                 const int t0 = o0 + t * cap;
                 __syncthreads();
-                n_obb = uniform(stage_obbs(a.S, t0, min(o1, t0 + cap), s_obb, cap));
+                n_obb = uniform(stage_obbs<kObbRec>(a.S, t0, min(o1, t0 + cap), s_obb, cap));
             }
-            Slots sl;
+            FkWalk<LINE> fk;
+            float T[12];
             for (int jj = 0; jj < J && wave_any(active); ++jj) {
-                float T[12];
                 int4 meta;
-                fk_joint(R, jj, s_q + lane, sl, T, meta);
-                const int s0 = R.sph_off[jj], s1 = R.sph_off[jj + 1];
-                const int a0 = R.apx_off[jj], a1 = R.apx_off[jj + 1];
+                fk.step(R, jj, s_q + lane, T, meta);
+                const int s0 = uload<int>(R.sph_off, jj), s1 = uload<int>(R.sph_off, jj + 1);
+                const int a0 = uload<int>(R.apx_off, jj), a1 = uload<int>(R.apx_off, jj + 1);
                 if (s1 == s0 || a1 == a0) continue;
-                // Approximate spheres of this joint in world coordinates (usually one).
-                float apx[3], apr2;
-                const float4 as0 = R.apx[a0];
-                aff_point(T, as0.x, as0.y, as0.z, apx[0], apx[1], apx[2]);
-                {
-                    const float rr = as0.w + a.margin;
-                    apr2 = rr * rr;
-                }
-                // Broad phase: the OBBs some active lane's approximate sphere can
-                // reach. The active lanes' centres lie within rw of the first
-                // active lane's centre c0, so every OBB an approximate sphere
-                // overlaps lies within rw + r of c0 (slack covers rounding).
-                const bool broad = a1 - a0 == 1;
-                float cx = 0.0f, cy = 0.0f, cz = 0.0f, reach2 = 0.0f;
-                if (broad) {
-                    const int l0 = __ffsll(__ballot(active)) - 1;
-                    cx = read_lane(apx[0], l0); cy = read_lane(apx[1], l0); cz = read_lane(apx[2], l0);
-                    const float dx = apx[0] - cx, dy = apx[1] - cy, dz = apx[2] - cz;
-                    const float d2 = wave_max(active ? fmaf(dz, dz, fmaf(dy, dy, dx * dx)) : 0.0f);
-                    const float reach = sqrtf(d2) * 1.0001f + fabsf(as0.w + a.margin) + 1e-5f;
-                    reach2 = uniform(reach * reach);
-                }
                 bool flag = false;
-                bool done = false;
-                for (int base = 0; base < n_obb && !done; base += kWave) {
-                    // candidates of this block of 64 OBBs: lane i tests OBB base + i
-                    unsigned long long bits;
-                    {
-                        const int o = base + lane;
-                        bool c = o < n_obb;
-                        if (broad && c) {
-                            float lx, ly, lz;
-                            to_box(s_obb[4 * o], s_obb[4 * o + 1], s_obb[4 * o + 2], cx, cy, cz, lx, ly, lz);
-                            c = box_hit(lx, ly, lz, s_obb[4 * o + 3], reach2);
-                        }
-                        bits = __ballot(c);
-                    }
-                    while (bits && !done) {
-                        const int o = base + (__ffsll(bits) - 1);
-                        bits &= bits - 1ull;
-                        const float4 r0 = s_obb[4 * o], r1 = s_obb[4 * o + 1], r2 = s_obb[4 * o + 2], h = s_obb[4 * o + 3];
-                        float lx, ly, lz;
-                        to_box(r0, r1, r2, apx[0], apx[1], apx[2], lx, ly, lz);
-                        bool ah = box_hit(lx, ly, lz, h, apr2);
-                        for (int ai = a0 + 1; ai < a1; ++ai) {
-                            const float4 as = R.apx[ai];
-                            float x, y, z;
-                            aff_point(T, as.x, as.y, as.z, x, y, z);
-                            to_box(r0, r1, r2, x, y, z, lx, ly, lz);
-                            const float rr = as.w + a.margin;
-                            ah = ah || box_hit(lx, ly, lz, h, rr * rr);
-                        }
-                        flag = flag || ah;
-                        if (!wave_any(ah && active)) continue;
+                int qn = 0;              // pairs queued
+                // 3. exact tests of the queued pairs; states found to collide leave `active`
+                auto flush = [&]() {
+                    __syncthreads();
+                    const int ns = s1 - s0;
+                    for (int q0 = 0; q0 < qn; q0 += kWave) {
+                        const int n = min(kWave, qn - q0);
+                        const int sh = n <= 8 ? 3 : n <= 16 ? 2 : n <= 32 ? 1 : 0;   // 2^sh lanes per pair
+                        const int i = lane >> sh, k0 = lane & ((1 << sh) - 1);
+                        const bool on = i < n;
+                        const int item = s_queue[q0 + (on ? i : 0)];
+                        const int l = item & 0xFF, o = item >> 8;
+                        const float4 r0 = s_obb[kObbRec * o], r1 = s_obb[kObbRec * o + 1], r2 = s_obb[kObbRec * o + 2], h = s_obb[kObbRec * o + 3];
+                        float Tl[12];   // the state's frame, from its own lane
+#pragma unroll
+                        for (int c = 0; c < 12; ++c) Tl[c] = __shfl(T[c], l);
                         // M = R_o * T_j: sphere-local -> box-local in one affine map.
                         float M[12];
-    #pragma unroll
+#pragma unroll
                         for (int rr = 0; rr < 3; ++rr) {
-                            const float4 row = rr == 0 ? r0 : (rr == 1 ? r1 : r2);
-    #pragma unroll
+                            const float4 rw = rr == 0 ? r0 : (rr == 1 ? r1 : r2);
+#pragma unroll
                             for (int c = 0; c < 4; ++c) {
-                                float v = fmaf(row.z, T[8 + c], fmaf(row.y, T[4 + c], row.x * T[c]));
-                                if (c == 3) v += row.w;
+                                float v = fmaf(rw.z, Tl[8 + c], fmaf(rw.y, Tl[4 + c], rw.x * Tl[c]));
+                                if (c == 3) v += rw.w;
                                 M[rr * 4 + c] = v;
                             }
                         }
-                        const int o_orig = __float_as_int(h.w);
                         bool h_any = false;
-                        for (int s = s0; s < s1; ++s) {
-                            const float4 sp = R.sph[s];
+                        for (int k = k0; k < ns; k += 1 << sh) {
+                            const float4 sp = s_sph[s0 + k];
                             float x, y, z;
                             aff_point(M, sp.x, sp.y, sp.z, x, y, z);
                             const float rr = sp.w + a.margin;
                             bool hs = box_hit(x, y, z, h, rr * rr);
-                            if (acm) hs = hs && acm[(size_t)R.sph_id[s] * a.S.n_obbs + o_orig] != 0;
+                            if (acm) hs = hs && acm[(size_t)R.sph_id[s0 + k] * a.S.n_obbs + __float_as_int(h.w)] != 0;
                             h_any = h_any || hs;
                         }
-                        hit = hit || (active && ah && h_any);
-                        active = active && !hit;
-                        done = !wave_any(active);
+                        if (on && h_any) s_hit[l] = 1;
+                    }
+                    __syncthreads();
+                    hit = hit || (active && s_hit[lane] != 0);
+                    active = active && !hit;
+                    qn = 0;
+                };
+                // each approximate sphere of the joint (usually one)
+                for (int ai = a0; ai < a1; ++ai) {
+                    const float4 as = uload4(R.apx, ai);
+                    float px, py, pz;
+                    aff_point(T, as.x, as.y, as.z, px, py, pz);
+                    const float rr = as.w + a.margin;
+                    const float apr2 = rr * rr;
+                    // 1. the row's centre state (a middle one) and its spread
+                    const unsigned in_row = row_bits(__ballot(active), row);
+                    const int l0 = row + (in_row >> 8 ? 7 + __ffs(in_row >> 8) : in_row ? __ffs(in_row) - 1 : 0);
+                    const float cx = __shfl(px, l0), cy = __shfl(py, l0), cz = __shfl(pz, l0);
+                    const float dx = px - cx, dy = py - cy, dz = pz - cz;
+                    const float d2 = row_max(active ? fmaf(dz, dz, fmaf(dy, dy, dx * dx)) : 0.0f);
+                    const float reach = __builtin_amdgcn_sqrtf(d2) * 1.0001f + fabsf(rr) + 1e-5f;
+                    const float reach2 = reach * reach;
+                    for (int base = 0; base < n_obb; base += kWave) {
+                        const int m = min(kWave, n_obb - base);
+                        unsigned long long todo = 0ull;   // the lane's candidates
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            if (16 * r >= m) break;
+                            // past the last box: its record again, masked off
+                            const int k = 16 * r + (lane & 15), o = base + min(k, m - 1);
+                            float lx, ly, lz;
+                            to_box(s_obb[kObbRec * o], s_obb[kObbRec * o + 1], s_obb[kObbRec * o + 2], cx, cy, cz, lx, ly, lz);
+                            const bool c = k < m && box_hit(lx, ly, lz, s_obb[kObbRec * o + 3], reach2);
+                            todo |= (unsigned long long)row_bits(__ballot(c), row) << (16 * r);
+                        }
+                        if (!active) todo = 0ull;
+                        while (wave_any(todo != 0ull)) {
+                            // 2. the lane's own approximate sphere against its next candidate
+                            const bool on = todo != 0ull;
+                            const int o = base + (on ? __ffsll(todo) - 1 : 0);
+                            todo &= todo - 1ull;
+                            float lx, ly, lz;
+                            to_box(s_obb[kObbRec * o], s_obb[kObbRec * o + 1], s_obb[kObbRec * o + 2], px, py, pz, lx, ly, lz);
+                            const bool ah = box_hit(lx, ly, lz, s_obb[kObbRec * o + 3], apr2) && on;
+                            flag = flag || ah;
+                            const unsigned long long push = __ballot(ah);
+                            if (push == 0ull) continue;
+                            if (ah) s_queue[qn + rank_below(push)] = lane | (o << 8);
+                            qn += __popcll(push);
+                            if (qn >= kWave) {
+                                flush();
+                                if (!active) todo = 0ull;
+                            }
+                        }
                     }
                 }
+                if (qn > 0) flush();
                 if (!last) {
                     if (flag) flagged |= 1u << jj;
                     continue;
                 }
                 flag = flag || ((flagged >> jj) & 1u) != 0u;
-                if (has_esdf) {
+                if (ESDF) {
                     // Approx ESDF pass (ACM disabled, scene_collision.cuh:574-582),
                     // then the joint's exact spheres when it is flagged.
                     for (int ai = a0; ai < a1; ++ai) {
-                        const float4 as = R.apx[ai];
+                        const float4 as = uload4(R.apx, ai);
                         float x, y, z;
                         aff_point(T, as.x, as.y, as.z, x, y, z);
                         flag = flag || (active && esdf_hit(a.S, x, y, z, as.w + a.margin, -1));
                     }
                     if (wave_any(flag && active)) {
                         for (int s = s0; s < s1; ++s) {
-                            const float4 sp = R.sph[s];
+                            const float4 sp = uload4(R.sph, s);
                             float x, y, z;
                             aff_point(T, sp.x, sp.y, sp.z, x, y, z);
                             const bool hs = flag && active && esdf_hit(a.S, x, y, z, sp.w + a.margin, R.sph_id[s]);
@@ -1807,7 +1925,7 @@ __global__ __launch_bounds__(64, 5) void k_cost_grp_esdf(CostArgs a) {
 // ONE: the scene is a single trilinear layer without masks (esdf_single).
 // ===========================================================================
 template <int G, bool ONE>
-__global__ __launch_bounds__(64) void k_clear(ClearArgs a) {
+__global__ __launch_bounds__(64, 4) void k_clear(ClearArgs a) {
     extern __shared__ float s_clr[];
     constexpr int kN = kWave / G;             // states of the wave
     const DRobot& R = a.R;
@@ -1902,7 +2020,7 @@ __global__ __launch_bounds__(64) void k_clear(ClearArgs a) {
 constexpr int kSelfStates = kWave / kSelfGroup;
 static_assert(kSelfGroup >= kMaxJoints, "the self pass composes frames with one joint per lane of a state group");
 
-__global__ __launch_bounds__(64) void k_self(SelfArgs a) {
+__global__ __launch_bounds__(64, 4) void k_self(SelfArgs a) {
     extern __shared__ float4 s_dyn4[];
     const DRobot& R = a.R;
     const int lane = lane_id();
@@ -2912,17 +3030,28 @@ size_t lds_bytes(int obb_cap, int n_dof) {
     return (size_t)obb_cap * 64 + (size_t)(n_dof + 2) * kWave * sizeof(float);
 }
 
+size_t lds_bytes_collide(int obb_cap, const DRobot& R) {
+    const size_t b = lds_bytes(obb_cap, R.n_dof);
+    // + record padding, sphere table, hit flags
+    return R.scene_gate_fused ? b + (size_t)obb_cap * 16 * (kObbRec - 4) + (size_t)R.n_sph * 16 + kWave * sizeof(int) : b;
+}
+
 size_t lds_bytes_cost(int obb_cap, int n_dof, int n_joints, int G, bool grad) {
     size_t b = lds_bytes(obb_cap, n_dof);
     if (grad) b += (size_t)(kWave / G) * (rec_stride(n_joints) + dq_stride(n_dof)) * sizeof(float);
     return b;
 }
 
-int grid_collide(size_t lds) {
-    static size_t last = (size_t)-1;
-    static int g = 0;
-    if (lds != last) { g = occupancy_grid((const void*)k_collide, lds); last = lds; }
-    return g;
+static const void* collide_kernel(const DRobot& R, const DScene& S) {
+    if (!R.scene_gate_fused) return (const void*)k_collide_gated;
+    if (S.n_voxel_layers > 0) return R.line ? (const void*)k_collide<true, true> : (const void*)k_collide<true, false>;
+    return R.line ? (const void*)k_collide<false, true> : (const void*)k_collide<false, false>;
+}
+
+int grid_collide(const DRobot& R, const DScene& S, int obb_cap) {
+    static GridCache cache[5];
+    const int i = !R.scene_gate_fused ? 4 : (S.n_voxel_layers > 0 ? 2 : 0) + (R.line ? 1 : 0);
+    return cache[i].get(collide_kernel(R, S), lds_bytes_collide(obb_cap, R));
 }
 
 int grid_cost(int n_joints, bool grad, size_t lds) {
@@ -2949,8 +3078,8 @@ static hipError_t launch_args(const void* k, int grid, size_t lds, hipStream_t s
 
 hipError_t launch_collide(const CollideArgs& a, int grid, hipStream_t s, hipEvent_t t0, hipEvent_t t1) {
     CollideArgs arg = a;
-    const void* k = a.R.scene_gate_fused ? (const void*)k_collide : (const void*)k_collide_gated;
-    return launch_args(k, grid, lds_bytes(a.C.obb_cap, a.R.n_dof), s, &arg, t0, t1);
+    const void* k = collide_kernel(a.R, a.S);
+    return launch_args(k, grid, lds_bytes_collide(a.C.obb_cap, a.R), s, &arg, t0, t1);
 }
 
 hipError_t launch_cost(const CostArgs& a, int grid, hipStream_t s, hipEvent_t t0, hipEvent_t t1) {

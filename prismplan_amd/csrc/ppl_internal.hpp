@@ -79,6 +79,8 @@ struct DRobot {
     const int* sph_clu;         // [S] cluster of emission slot k
     const int* clu_jnt;         // [C] DFS joint of cluster c
     int scene_gate_fused;
+    // 1: every joint's parent is the joint before it in DFS order, or the root
+    int line;
     // 1: an exact self hit implies an approximate one (every exact pair lies in
     // an approximate pair); 0: the self verdict needs the approximate pass too.
     int self_gate_implied;
@@ -270,13 +272,14 @@ hipError_t launch_esdf_build(const float* obb_dims, const float* obb_pose, int n
                              const float* voxel_params, const float* voxel_pose, float* out,
                              hipStream_t s);
 size_t lds_bytes(int obb_cap, int n_dof);
+size_t lds_bytes_collide(int obb_cap, const DRobot& R);
 // Cost kernel: OBB records + q + (grad) per-state adjoint records.
 size_t lds_bytes_cost(int obb_cap, int n_dof, int n_joints, int G, bool grad);
 // Floats per state of the adjoint records: 12 per joint (odd stride), d cost / d q per dof.
 __host__ __device__ inline int rec_stride(int n_joints) { return 12 * n_joints + 1; }
 __host__ __device__ inline int dq_stride(int n_dof) { return n_dof | 1; }
 int device_cus();
-int grid_collide(size_t lds);
+int grid_collide(const DRobot& R, const DScene& S, int obb_cap);   // workgroups the chip holds at once
 int grid_cost(int n_joints, bool grad, size_t lds);
 size_t lds_bytes_grp(int obb_cap, int n_dof, int n_joints, int n_sph, int n_clu, bool grad, bool tiled);
 int grid_cost_grp(bool grad, int world, bool tiled, size_t lds);
