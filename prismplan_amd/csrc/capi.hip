@@ -101,6 +101,7 @@ struct HBuf {
 struct ppl_robot_s {
     DRobot R{};
     void* blob = nullptr;
+    void* far_blob = nullptr;   // tables of the rough self tests
     int n_slots = 1;
     int n_pairs = 0;
     int n_revolute = 0, n_prismatic = 0;   // joints that move with a dof
@@ -562,12 +563,13 @@ ppl_status run_self(const ppl_robot_s* r, const DStates& X, int mode, uint8_t* h
     SelfArgs a{};
     a.R = r->R;
     a.X = X;
+    a.C.chunk = self_chunk(r->R, mode, X.source, X.n_states);
     if (P && X.source != kSrcDense) {
-        // the plan's 4-state chunks: unit hints, and waypoint-major order where the plan has it
-        HIP_TRY(ensure_table(P, kSelfGroup));
-        a.C.tab = P->d_tab[group_index(kSelfGroup)];
-        a.C.n_chunks = P->n_chunks[group_index(kSelfGroup)];
-        a.C.chunk = kWave / kSelfGroup;
+        // the plan's chunks: unit hints, and waypoint-major order where the plan has it
+        const int G = kWave / a.C.chunk;
+        HIP_TRY(ensure_table(P, G));
+        a.C.tab = P->d_tab[group_index(G)];
+        a.C.n_chunks = P->n_chunks[group_index(G)];
     } else {
         a.X.wmajor = 0;  // flat plan order
         a.C.unit_hint = unit_hint;
@@ -889,6 +891,64 @@ ppl_status ppl_robot_create(const ppl_robot_desc* d, ppl_robot* out) try {
             k = e;
         }
     }
+    // Tables of the self pass's rough tests, one entry per block (DRobot::far_blk).
+    // They measure B's spheres in A's link frame, so the transforms must be
+    // rigid; far_slack bounds the distance error of the deviation and of FP32
+    // over the model's reach.
+    std::vector<int4> far_blk;
+    std::vector<int> far_gate, far_mask;
+    std::vector<float4> far_sph((size_t)2 * S);
+    double far_slack = 0.0, far_scale = 0.0, far_rmax = 0.0;
+    bool far_ok = true;
+    {
+        double dev = 0.0, reach = 0.0;
+        for (int k = 0; k < J; ++k) {
+            const float* f = &ft[12 * k];
+            for (int x = 0; x < 3; ++x)
+                for (int y = 0; y < 3; ++y) {
+                    double dot = 0.0;
+                    for (int r = 0; r < 3; ++r) dot += (double)f[4 * r + x] * f[4 * r + y];
+                    dev = std::max(dev, std::fabs(dot - (x == y ? 1.0 : 0.0)));
+                }
+            reach += std::sqrt((double)f[3] * f[3] + (double)f[7] * f[7] + (double)f[11] * f[11]);
+            if (meta[k].x >= 0 && meta[k].x < 3 && meta[k].y >= 0)
+                reach += std::max(std::fabs(d->joint_lower[meta[k].y]), std::fabs(d->joint_upper[meta[k].y]));
+        }
+        for (int k = 0; k < S; ++k) {
+            const double x = sph[k].x, y = sph[k].y, z = sph[k].z, rr = sph[k].w, c2 = x * x + y * y + z * z;
+            far_sph[2 * k] = make_float4((float)(-2 * x), (float)(-2 * y), (float)(-2 * z), (float)(c2 - rr * rr));
+            far_sph[2 * k + 1] = make_float4((float)(-2 * rr), 0.0f, 0.0f, 0.0f);
+            far_scale = std::max(far_scale, std::sqrt(c2) + std::fabs(rr));
+            far_rmax = std::max(far_rmax, std::fabs(rr));
+            far_ok = far_ok && rr >= 0.0;
+        }
+        far_slack = 2e-5 + (reach + far_scale) * (2.0 * J * dev + 4e-6);
+        far_ok = far_ok && dev <= 1e-5 && far_slack < 1e-2;
+        for (const int4& blk : cpb) {
+            int ca = blk.x, cb = blk.y;
+            auto count = [&](int c) { return clu_beg[c + 1] - clu_beg[c]; };
+            const bool swap = count(cb) > count(ca);
+            if (swap) std::swap(ca, cb);
+            const int a0 = clu_beg[ca], na = count(ca), b0 = clu_beg[cb], nb = count(cb);
+            int off = -1;
+            if (blk.w != na * nb) {
+                off = (int)far_mask.size();
+                far_mask.resize(off + nb, 0);
+                for (int t = 0; t < blk.w; ++t) {
+                    const int u = (int)(cpl[blk.z + t] & 0xFFFFu), v = (int)(cpl[blk.z + t] >> 16);
+                    far_mask[off + (swap ? u : v) - b0] |= 1 << ((swap ? v : u) - a0);
+                }
+            }
+            int ja = 0, jb = 0;
+            for (int k = 0; k < J; ++k) {
+                if (ca >= clu_off[k] && ca < clu_off[k + 1]) ja = k;
+                if (cb >= clu_off[k] && cb < clu_off[k + 1]) jb = k;
+            }
+            far_ok = far_ok && na <= 16 && nb <= 16 && ca != cb;
+            far_blk.push_back(make_int4(a0 | (na << 16), b0 | (nb << 16), ja | (jb << 16), off));
+            far_gate.push_back(ca | (cb << 16));
+        }
+    }
     std::vector<float4> sph_orig(S), apx_orig(A);
     for (int s = 0; s < S; ++s) sph_orig[s] = make_float4(d->spheres[4 * s], d->spheres[4 * s + 1], d->spheres[4 * s + 2], d->spheres[4 * s + 3]);
     for (int a = 0; a < A; ++a)
@@ -969,6 +1029,16 @@ ppl_status ppl_robot_create(const ppl_robot_desc* d, ppl_robot* out) try {
         return fail(PPL_ERR_ALLOC, "hipMalloc of %zu bytes for robot tables failed", host.size());
     }
     hipError_t e = hipMemcpy(r->blob, host.data(), host.size(), hipMemcpyHostToDevice);
+    // the rough self tests' tables lie apart from the blob whose digest keys the tuning cache
+    const size_t o_fb = 0, o_fs = o_fb + far_blk.size() * 16, o_fg = o_fs + far_sph.size() * 16,
+                 o_fm = o_fg + far_gate.size() * 4;
+    std::vector<char> far_host(o_fm + far_mask.size() * 4 + 16, 0);
+    if (!far_blk.empty()) memcpy(far_host.data() + o_fb, far_blk.data(), far_blk.size() * 16);
+    if (!far_sph.empty()) memcpy(far_host.data() + o_fs, far_sph.data(), far_sph.size() * 16);
+    if (!far_gate.empty()) memcpy(far_host.data() + o_fg, far_gate.data(), far_gate.size() * 4);
+    if (!far_mask.empty()) memcpy(far_host.data() + o_fm, far_mask.data(), far_mask.size() * 4);
+    if (e == hipSuccess) e = hipMalloc(&r->far_blob, far_host.size());
+    if (e == hipSuccess) e = hipMemcpy(r->far_blob, far_host.data(), far_host.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
         ppl_robot_destroy(r);
@@ -1000,6 +1070,14 @@ ppl_status ppl_robot_create(const ppl_robot_desc* d, ppl_robot* out) try {
     R.aft = own_chain ? reinterpret_cast<const float*>(b + o_aft) : nullptr;
     R.atype = own_chain ? reinterpret_cast<const int*>(b + o_atype) : nullptr;
     R.apx_jnt = reinterpret_cast<const int*>(b + o_ajnt);
+    char* fb = static_cast<char*>(r->far_blob);
+    R.far_blk = far_ok && !far_blk.empty() ? reinterpret_cast<const int4*>(fb + o_fb) : nullptr;
+    R.far_sph = reinterpret_cast<const float4*>(fb + o_fs);
+    R.far_gate = reinterpret_cast<const int*>(fb + o_fg);
+    R.far_mask = reinterpret_cast<const int*>(fb + o_fm);
+    R.far_slack = (float)far_slack;
+    R.far_scale2 = (float)(far_scale * far_scale);
+    R.far_rmax = (float)far_rmax;
     R.n_clu = n_clu;
     R.clu_off = reinterpret_cast<const int*>(b + o_coff);
     R.clu_beg = reinterpret_cast<const int*>(b + o_cbeg);
@@ -1064,6 +1142,7 @@ ppl_status ppl_robot_destroy(ppl_robot r) try {
     r->traj_plans.clear();
     if (r->stream) (void)hipStreamSynchronize(r->stream);
     if (r->blob) (void)hipFree(r->blob);
+    if (r->far_blob) (void)hipFree(r->far_blob);
     r->d_cfg.release(); r->d_out.release(); r->d_off.release(); r->d_aux.release(); r->d_self.release();
     r->d_mit.release(); r->d_hint.release(); r->h_mit.release();
     r->h_stage.release();

@@ -2020,72 +2020,31 @@ __global__ __launch_bounds__(64, 4) void k_clear(ClearArgs a) {
 constexpr int kSelfStates = kWave / kSelfGroup;
 static_assert(kSelfGroup >= kMaxJoints, "the self pass composes frames with one joint per lane of a state group");
 
-__global__ __launch_bounds__(64, 4) void k_self(SelfArgs a) {
-    extern __shared__ float4 s_dyn4[];
-    const DRobot& R = a.R;
-    const int lane = lane_id();
-    const int sub = lane & (kSelfGroup - 1);
-    const int st = lane / kSelfGroup;
-    const int S = R.n_sph, D = R.n_dof, J = R.n_joints;
-    float4* s_pos = s_dyn4;                                          // [kSelfStates][S] (x, y, z, r)
-    const int NC = R.n_clu;
-    float4* s_cenc = s_dyn4 + kSelfStates * S;                        // [kSelfStates][NC] cluster enclosing spheres
-    const int fstride = J * 12 + 4;                                   // frame block per state, padded
-    float* s_T = reinterpret_cast<float*>(s_cenc + kSelfStates * NC); // [kSelfStates][J][12] joint frames
-    float* s_q = s_T + kSelfStates * fstride;                         // [kMaxDof][kSelfStates]
-    int* s_par = reinterpret_cast<int*>(s_q + kMaxDof * kSelfStates); // [kSelfStates][J] pointer-jumping links
-    int* s_end = s_par + kSelfStates * J;                             // [2][64] unit ends / starts of a chunk
-    float4* s_apos = reinterpret_cast<float4*>(s_end + 2 * kWave);    // gated mode 0: [kSelfStates][A] approx spheres
-    const bool gated = a.mode == 0 && !R.self_gate_implied;
-    const long n_states = state_count(a.X);
-    // With the plan's chunk table a chunk names its first unit (staged unit
-    // ends make the state -> unit lookup an LDS bisection) or, waypoint-major,
-    // its problem; without it states go in flat order.
-    const bool chunked = a.C.tab != nullptr;
-    const long n_work = chunked ? (long)a.C.n_chunks : (n_states + kSelfStates - 1) / kSelfStates;
-    for (long w = blockIdx.x; w < n_work; w += gridDim.x) {
-    long base, g;
-    bool active;
-    int u0 = -1, prob = 0;
-    if (chunked) {
-        const int4 ch = a.C.tab[w];
-        base = ch.y;
-        g = base + st;
-        active = g < ch.z;
-        u0 = ch.w;
-        prob = ch.x;
-        stage_unit_ends(a.X, u0, s_end);
-        __syncthreads();
-    } else {
-        base = w * kSelfStates;
-        g = base + st;
-        active = g < n_states;
-        if (a.C.unit_hint) {
-            u0 = uniform(a.C.unit_hint[base >> 6]);
-            stage_unit_ends(a.X, u0, s_end);
-            __syncthreads();
-        }
+// LDS of the exact pass over four states, 16 lanes each.
+struct SelfLds {
+    float4* pos;    // [kSelfStates][S] (x, y, z, r)
+    float4* cenc;   // [kSelfStates][NC] cluster enclosing spheres
+    float* T;       // [kSelfStates][J][12] joint frames, padded
+    int* par;       // [kSelfStates][J] pointer-jumping links
+    static __host__ __device__ size_t bytes(int S, int NC, int J) {
+        return kSelfStates * (sizeof(float4) * (size_t)(S + NC) + sizeof(float) * (size_t)(J * 12 + 4) +
+                              sizeof(int) * (size_t)J);
     }
-    // units already decided need no configuration, FK or pairs (the unit
-    // first-hit mode runs over densified trajectories and edge midpoints)
-    const bool by_unit = a.unit_first_hit && (a.X.source == kSrcDense || a.X.source == kSrcBfs);
-    if (by_unit) {
-        int b0, b1;
-        const int u = find_unit(a.X.dense_off, a.X.n_traj, active ? g : base, u0, s_end, &b0, &b1);
-        if (active && a.unit_first_hit[u] >= 0) active = false;
-        if (!wave_any(active)) continue;
+    __device__ __forceinline__ SelfLds(void* base, int S, int NC, int J) {
+        pos = static_cast<float4*>(base);
+        cenc = pos + kSelfStates * S;
+        T = reinterpret_cast<float*>(cenc + kSelfStates * NC);
+        par = reinterpret_cast<int*>(T + kSelfStates * (J * 12 + 4));
     }
-    // Every lane of a state group resolves the state; lane 0 stores its q.
-    const StateRef ref = load_state(a.X, D, active ? g : base, true, s_q, u0, s_end, prob, st, kSelfStates, sub == 0);
-    if (a.unit_first_hit && !by_unit) {
-        if (active && a.unit_first_hit[ref.unit] >= 0) active = false;
-        if (!wave_any(active)) continue;
-    }
-    __syncthreads();
-    float4* pos = s_pos + st * S;
-    float4* cenc = s_cenc + st * NC;
-    float* Ts = s_T + st * fstride;
-    group_frames(R, s_q + st, kSelfStates, Ts, s_par + st * J, sub);
+};
+
+// Sphere centres and cluster enclosing spheres of the four states from their
+// frames (whole wave).
+__device__ __forceinline__ void self_place(const DRobot& R, const SelfLds& L, int st, int sub) {
+    const int S = R.n_sph, NC = R.n_clu;
+    float4* pos = L.pos + st * S;
+    float4* cenc = L.cenc + st * NC;
+    const float* Ts = L.T + st * (R.n_joints * 12 + 4);
     // sphere centres (emission slot k: a joint's spheres are contiguous) and
     // each sphere cluster's enclosing sphere, from the frames
     for (int k = sub; k < S; k += kSelfGroup) {
@@ -2104,36 +2063,16 @@ __global__ __launch_bounds__(64, 4) void k_self(SelfArgs a) {
                               fmaf(t1.x, ce.x, fmaf(t1.y, ce.y, fmaf(t1.z, ce.z, t1.w))),
                               fmaf(t2.x, ce.x, fmaf(t2.y, ce.y, fmaf(t2.z, ce.z, t2.w))), ce.w);
     }
-    __syncthreads();
-    bool live = active;   // states whose pairs are checked (gated: an approximate pair collides)
-    if (gated) {
-        // Approximate pairs first (two_phase_cc.cuh:114-131): a state none of
-        // whose approximate pairs collide has no self collision. Their frames
-        // come from the approximate chain when the model has its own (the
-        // exact positions above no longer need the full chain's).
-        if (R.aft) {
-            group_frames<true>(R, s_q + st, kSelfStates, Ts, s_par + st * J, sub);
-        }
-        float4* apos = s_apos + st * R.n_apx;
-        for (int k = sub; k < R.n_apx; k += kSelfGroup) {
-            const float4 sp = R.apx_orig[k];
-            const float4* Tq = reinterpret_cast<const float4*>(Ts + 12 * R.apx_jnt[k]);
-            const float4 t0 = Tq[0], t1 = Tq[1], t2 = Tq[2];
-            apos[k] = make_float4(fmaf(t0.x, sp.x, fmaf(t0.y, sp.y, fmaf(t0.z, sp.z, t0.w))),
-                                  fmaf(t1.x, sp.x, fmaf(t1.y, sp.y, fmaf(t1.z, sp.z, t1.w))),
-                                  fmaf(t2.x, sp.x, fmaf(t2.y, sp.y, fmaf(t2.z, sp.z, t2.w))), sp.w);
-        }
-        __syncthreads();
-        bool ah = false;
-        for (int p = sub; p < R.n_apx_pairs && live; p += kSelfGroup) {
-            const int2 pr = R.apx_pairs[p];
-            const float4 u = apos[pr.x], v = apos[pr.y];
-            const float ux = u.x - v.x, uy = u.y - v.y, uz = u.z - v.z;
-            const float r2 = u.w + v.w;
-            ah = ah || fmaf(uz, uz, fmaf(uy, uy, ux * ux)) - r2 * r2 < 0.0f;
-        }
-        live = live && ((__ballot(ah) >> (st * kSelfGroup)) & 0xFFFFull) != 0ull;
-    }
+}
+
+// Exact self check of the four states (16 lanes each) from their sphere
+// centres: the pairs of every block whose clusters are near, the outputs of
+// states with `active`. live: states whose pairs are checked.
+__device__ __forceinline__ void self_pairs(const SelfArgs& a, const SelfLds& L, int st, int sub, bool active, bool live,
+                                           long gs, int unit, int kstate) {
+    const DRobot& R = a.R;
+    const float4* pos = L.pos + st * R.n_sph;
+    const float4* cenc = L.cenc + st * R.n_clu;
     // Pairs come in blocks by the sphere clusters of their two spheres; a
     // cluster's enclosing sphere contains all of its spheres, so a block
     // whose two enclosing spheres are at clearance >= band holds no pair
@@ -2197,9 +2136,9 @@ __global__ __launch_bounds__(64, 4) void k_self(SelfArgs a) {
     if (a.mode == 0) {
         if (active && sub == 0) {
             if (a.unit_first_hit) {
-                if (hit) atomicMin((unsigned*)&a.unit_first_hit[ref.unit], (unsigned)ref.k);
+                if (hit) atomicMin((unsigned*)&a.unit_first_hit[unit], (unsigned)kstate);
             } else {
-                a.hit_out[ref.gs] = hit ? 1 : 0;
+                a.hit_out[gs] = hit ? 1 : 0;
             }
         }
     } else {
@@ -2213,7 +2152,7 @@ __global__ __launch_bounds__(64, 4) void k_self(SelfArgs a) {
             }
         }
         if (active && sub == 0) {
-            float* o = a.out + 8 * (size_t)ref.gs;
+            float* o = a.out + 8 * (size_t)gs;
             o[0] = best;
             if (bkey != INT_MAX) {
                 const unsigned pr = R.cpl[R.cpb[bkey >> 16].z + (bkey & 0xFFFF)];
@@ -2230,7 +2169,374 @@ __global__ __launch_bounds__(64, 4) void k_self(SelfArgs a) {
             o[6] = o[7] = 0.0f;
         }
     }
+}
+
+// Whether a state can no longer change its unit's first hit: an edge's states
+// past its known hit, every state of another unit that has one.
+__device__ __forceinline__ bool unit_settled(const SelfArgs& a, const StateRef& ref) {
+    const int fh = a.unit_first_hit[ref.unit];
+    return a.X.source == kSrcEdge ? (unsigned)fh <= (unsigned)ref.k : fh >= 0;
+}
+
+__global__ __launch_bounds__(64, 4) void k_self(SelfArgs a) {
+    extern __shared__ float4 s_dyn4[];
+    const DRobot& R = a.R;
+    const int lane = lane_id();
+    const int sub = lane & (kSelfGroup - 1);
+    const int st = lane / kSelfGroup;
+    const int S = R.n_sph, D = R.n_dof, J = R.n_joints;
+    const SelfLds L(s_dyn4, S, R.n_clu, J);
+    const int fstride = J * 12 + 4;
+    float* s_q = reinterpret_cast<float*>(reinterpret_cast<char*>(s_dyn4) + SelfLds::bytes(S, R.n_clu, J));   // [kMaxDof][kSelfStates]
+    int* s_end = reinterpret_cast<int*>(s_q + kMaxDof * kSelfStates); // [2][64] unit ends / starts of a chunk
+    float4* s_apos = reinterpret_cast<float4*>(s_end + 2 * kWave);    // gated mode 0: [kSelfStates][A] approx spheres
+    const bool gated = a.mode == 0 && !R.self_gate_implied;
+    const long n_states = state_count(a.X);
+    // With the plan's chunk table a chunk names its first unit (staged unit
+    // ends make the state -> unit lookup an LDS bisection) or, waypoint-major,
+    // its problem; without it states go in flat order.
+    const bool chunked = a.C.tab != nullptr;
+    const long n_work = chunked ? (long)a.C.n_chunks : (n_states + kSelfStates - 1) / kSelfStates;
+    for (long w = blockIdx.x; w < n_work; w += gridDim.x) {
+    long base, g;
+    bool active;
+    int u0 = -1, prob = 0;
+    if (chunked) {
+        const int4 ch = a.C.tab[w];
+        base = ch.y;
+        g = base + st;
+        active = g < ch.z;
+        u0 = ch.w;
+        prob = ch.x;
+        stage_unit_ends(a.X, u0, s_end);
+        __syncthreads();
+    } else {
+        base = w * kSelfStates;
+        g = base + st;
+        active = g < n_states;
+        if (a.C.unit_hint) {
+            u0 = uniform(a.C.unit_hint[base >> 6]);
+            stage_unit_ends(a.X, u0, s_end);
+            __syncthreads();
+        }
+    }
+    // units already decided need no configuration, FK or pairs (the unit
+    // first-hit mode runs over densified trajectories and edge midpoints)
+    const bool by_unit = a.unit_first_hit && (a.X.source == kSrcDense || a.X.source == kSrcBfs);
+    if (by_unit) {
+        int b0, b1;
+        const int u = find_unit(a.X.dense_off, a.X.n_traj, active ? g : base, u0, s_end, &b0, &b1);
+        if (active && a.unit_first_hit[u] >= 0) active = false;
+        if (!wave_any(active)) continue;
+    }
+    // Every lane of a state group resolves the state; lane 0 stores its q.
+    const StateRef ref = load_state(a.X, D, active ? g : base, true, s_q, u0, s_end, prob, st, kSelfStates, sub == 0);
+    if (a.unit_first_hit && !by_unit) {
+        if (active && unit_settled(a, ref)) active = false;
+        if (!wave_any(active)) continue;
+    }
+    __syncthreads();
+    float* Ts = L.T + st * fstride;
+    group_frames(R, s_q + st, kSelfStates, Ts, L.par + st * J, sub);
+    self_place(R, L, st, sub);
+    __syncthreads();
+    bool live = active;   // states whose pairs are checked (gated: an approximate pair collides)
+    if (gated) {
+        // Approximate pairs first (two_phase_cc.cuh:114-131): a state none of
+        // whose approximate pairs collide has no self collision. Their frames
+        // come from the approximate chain when the model has its own (the
+        // exact positions above no longer need the full chain's).
+        if (R.aft) {
+            group_frames<true>(R, s_q + st, kSelfStates, Ts, L.par + st * J, sub);
+        }
+        float4* apos = s_apos + st * R.n_apx;
+        for (int k = sub; k < R.n_apx; k += kSelfGroup) {
+            const float4 sp = R.apx_orig[k];
+            const float4* Tq = reinterpret_cast<const float4*>(Ts + 12 * R.apx_jnt[k]);
+            const float4 t0 = Tq[0], t1 = Tq[1], t2 = Tq[2];
+            apos[k] = make_float4(fmaf(t0.x, sp.x, fmaf(t0.y, sp.y, fmaf(t0.z, sp.z, t0.w))),
+                                  fmaf(t1.x, sp.x, fmaf(t1.y, sp.y, fmaf(t1.z, sp.z, t1.w))),
+                                  fmaf(t2.x, sp.x, fmaf(t2.y, sp.y, fmaf(t2.z, sp.z, t2.w))), sp.w);
+        }
+        __syncthreads();
+        bool ah = false;
+        for (int p = sub; p < R.n_apx_pairs && live; p += kSelfGroup) {
+            const int2 pr = R.apx_pairs[p];
+            const float4 u = apos[pr.x], v = apos[pr.y];
+            const float ux = u.x - v.x, uy = u.y - v.y, uz = u.z - v.z;
+            const float r2 = u.w + v.w;
+            ah = ah || fmaf(uz, uz, fmaf(uy, uy, ux * ux)) - r2 * r2 < 0.0f;
+        }
+        live = live && ((__ballot(ah) >> (st * kSelfGroup)) & 0xFFFFull) != 0ull;
+    }
+    self_pairs(a, L, st, sub, active, live, ref.gs, ref.unit, ref.k);
     __syncthreads();   // positions of this round are dead before the next load
+    }
+}
+
+// ===========================================================================
+// Any-collision self pass in two steps, for models with rigid transforms
+// (DRobot::far_blk): rough distances settle nearly every state, and the few
+// they leave open go through the exact pass above, four at a time.
+//
+// kFar lanes share a state: they take its joints' sines in turn and walk the
+// tree in step (frames kept in LDS for the pairs), place the clusters' centres,
+// test every kFar-th block's two enclosing spheres each, and for the blocks
+// near in some state take every kFar-th sphere b of the smaller cluster, place it
+// in the larger cluster's link frame and measure it against that link's
+// constant spheres a, |b - a|^2 = |b|^2 + (-2a . b + |a|^2): four multiply-adds a
+// pair with a's constants in SGPRs. val = |b - a|^2 - (ra + rb + slack)^2 above
+// its rounding err for all pairs proves the state free (slack bounds the frames'
+// and the transforms' errors), val below -(4 rs slack + err) for one proves it
+// hit. What is open is decided by the exact pass, so the verdicts are its own.
+// Bound by VALU issue: frames once per state instead of in every group's rounds,
+// and 210 pairs of near blocks a wave of states where the exact pass spends about
+// 1,000 instructions on four states. Where it runs: see self_far.
+// ===========================================================================
+constexpr int kFar = 4;
+constexpr int kFarStates = kWave / kFar;
+
+struct FarLds {
+    size_t T, cen, enc, sph, gate, q, end, list, ref, bytes;
+    __host__ __device__ explicit FarLds(const DRobot& R) {
+        constexpr int kn = kFarStates;
+        size_t o = 0;
+        auto take = [&](size_t n) {
+            const size_t at = o;
+            o += (n + 15) & ~(size_t)15;
+            return at;
+        };
+        T = take((size_t)R.n_joints * kn * 48);
+        cen = take((size_t)R.n_clu * kn * 12);
+        const size_t exact = SelfLds::bytes(R.n_sph, R.n_clu, R.n_joints);   // takes T's and cen's place
+        if (o < exact) o = (exact + 15) & ~(size_t)15;
+        enc = take((size_t)R.n_clu * 16);
+        sph = take((size_t)R.n_sph * 16);
+        gate = take((size_t)R.n_cpb * 4);
+        q = take((size_t)R.n_dof * kn * 4);
+        end = take(2 * kWave * 4);
+        list = take((size_t)kn * 4);
+        ref = take((size_t)kn * 16);
+        bytes = o;
+    }
+};
+
+__global__ __launch_bounds__(64, 4) void k_self_far(SelfArgs a) {
+    extern __shared__ float4 s_dyn4[];
+    constexpr int G = kFar, kN = kFarStates;
+    const DRobot& R = a.R;
+    const int lane = lane_id(), sub = lane & (G - 1), slot = lane / G;
+    const int S = R.n_sph, D = R.n_dof, J = R.n_joints, NC = R.n_clu;
+    const FarLds lay(R);
+    char* base_lds = reinterpret_cast<char*>(s_dyn4);
+    float* s_T = reinterpret_cast<float*>(base_lds + lay.T);      // [J][kN][12]; a joint's sine and cosine first
+    float* s_cen = reinterpret_cast<float*>(base_lds + lay.cen);  // [NC][3][kN]
+    float4* s_enc = reinterpret_cast<float4*>(base_lds + lay.enc);
+    float4* s_sph = reinterpret_cast<float4*>(base_lds + lay.sph);
+    int* s_gate = reinterpret_cast<int*>(base_lds + lay.gate);
+    float* s_q = reinterpret_cast<float*>(base_lds + lay.q);      // [D][kN]
+    int* s_end = reinterpret_cast<int*>(base_lds + lay.end);
+    int* s_list = reinterpret_cast<int*>(base_lds + lay.list);    // states left open
+    int4* s_ref = reinterpret_cast<int4*>(base_lds + lay.ref);    // per state: plan index, unit, state of the unit
+    for (int k = lane; k < NC; k += kWave) s_enc[k] = R.clu_enc[k];
+    for (int k = lane; k < S; k += kWave) s_sph[k] = R.sph[k];
+    for (int k = lane; k < R.n_cpb; k += kWave) s_gate[k] = R.far_gate[k];
+    const float rsure = 8.0f * R.far_rmax;
+    const long n_states = state_count(a.X);
+    const bool chunked = a.C.tab != nullptr;
+    const long n_work = chunked ? (long)a.C.n_chunks : (n_states + kN - 1) / kN;
+    for (long w = blockIdx.x; w < n_work; w += gridDim.x) {
+        __syncthreads();   // the last round's LDS is read
+        long base, g;
+        bool active;
+        int u0 = -1, prob = 0;
+        if (chunked) {
+            const int4 ch = a.C.tab[w];
+            base = ch.y;
+            g = base + slot;
+            active = g < ch.z;
+            u0 = ch.w;
+            prob = ch.x;
+            stage_unit_ends(a.X, u0, s_end);
+        } else {
+            base = w * kN;
+            g = base + slot;
+            active = g < n_states;
+            if (a.C.unit_hint) {
+                u0 = uniform(a.C.unit_hint[base >> 6]);
+                stage_unit_ends(a.X, u0, s_end);
+            }
+        }
+        __syncthreads();
+        const bool by_unit = a.unit_first_hit && (a.X.source == kSrcDense || a.X.source == kSrcBfs);
+        if (by_unit) {
+            int b0, b1;
+            const int u = find_unit(a.X.dense_off, a.X.n_traj, active ? g : base, u0, s_end, &b0, &b1);
+            if (active && a.unit_first_hit[u] >= 0) active = false;
+            if (!wave_any(active)) continue;
+        }
+        const StateRef ref = load_state(a.X, D, active ? g : base, true, s_q, u0, s_end, prob, slot, kN, sub == 0);
+        if (a.unit_first_hit && !by_unit) {
+            if (active && unit_settled(a, ref)) active = false;
+            if (!wave_any(active)) continue;
+        }
+        if (sub == 0) s_ref[slot] = make_int4((int)ref.gs, ref.unit, ref.k, 0);
+        __syncthreads();
+        // frames and cluster centres
+        for (int jj = sub; jj < J; jj += G) {
+            const int4 meta = R.jmeta[jj];
+            float sn = 0.0f, cs = 1.0f;
+            if (meta.x >= kXRot) sincosf(meta.y >= 0 ? s_q[meta.y * kN + slot] : 0.0f, &sn, &cs);
+            *reinterpret_cast<float2*>(s_T + 12 * (jj * kN + slot)) = make_float2(sn, cs);
+        }
+        __syncthreads();
+        float T[12];
+        for (int jj = 0; jj < J; ++jj) {
+            const i4u meta = uload<i4u>(R.jmeta, jj);
+            float* Tj = s_T + 12 * (jj * kN + slot);
+            if (jj == 0) {
+                aff_identity(T);
+            } else {
+                float P[12], A[12];
+                const int par = uload<int>(R.parent, jj);
+                if (par == 0) {
+                    aff_identity(P);
+                } else if (par == jj - 1) {
+#pragma unroll
+                    for (int k = 0; k < 12; ++k) P[k] = T[k];
+                } else {
+                    const float* Tp = s_T + 12 * (par * kN + slot);
+#pragma unroll
+                    for (int k = 0; k < 12; ++k) P[k] = Tp[k];
+                }
+                const float2 sc = *reinterpret_cast<const float2*>(Tj);
+                joint_step_u(R.ft, jj, meta.x, meta.y >= 0 ? s_q[meta.y * kN + slot] : 0.0f, sc.x, sc.y, A);
+                aff_compose(P, A, T);
+            }
+            if (sub == (jj & (G - 1))) {
+                float4* d = reinterpret_cast<float4*>(Tj);
+                d[0] = make_float4(T[0], T[1], T[2], T[3]);
+                d[1] = make_float4(T[4], T[5], T[6], T[7]);
+                d[2] = make_float4(T[8], T[9], T[10], T[11]);
+            }
+            const int c1 = uload<int>(R.clu_off, jj + 1);
+            for (int c = uload<int>(R.clu_off, jj) + sub; c < c1; c += G) {
+                const float4 ce = s_enc[c];
+                float x, y, z;
+                aff_point(T, ce.x, ce.y, ce.z, x, y, z);
+                float* o = s_cen + 3 * c * kN + slot;
+                o[0] = x; o[kN] = y; o[2 * kN] = z;
+            }
+        }
+        __syncthreads();
+        const float far_t = 2e-6f * (fabsf(T[3]) + fabsf(T[7]) + fabsf(T[11]));   // a base moved far off its limits
+        const float slack = R.far_slack + far_t;
+        float open = 1.0f, sure = 1.0f;   // smallest margins: open < 0 not proven clear, sure < 0 proven hit
+        for (int b0 = 0; b0 < R.n_cpb; b0 += G) {
+            const int bb = b0 + sub;
+            bool near = active && bb < R.n_cpb;
+            if (near) {
+                const int ids = s_gate[bb], cA = ids & 0xFFFF, cB = ids >> 16;
+                const float* p = s_cen + 3 * cA * kN + slot;
+                const float* q = s_cen + 3 * cB * kN + slot;
+                const float dx = p[0] - q[0], dy = p[kN] - q[kN], dz = p[2 * kN] - q[2 * kN];
+                const float rs = s_enc[cA].w + s_enc[cB].w + slack;
+                near = fmaf(dz, dz, fmaf(dy, dy, dx * dx)) < rs * rs;
+            }
+            const unsigned long long bal = __ballot(near);
+            if (bal == 0ull) continue;
+            unsigned todo = 0u;   // bit p: block b0 + p is near in some state
+#pragma unroll
+            for (int p = 0; p < G; ++p) {
+                unsigned long long col = 1ull << p;
+#pragma unroll
+                for (int k = G; k < kWave; k <<= 1) col |= col << k;
+                todo |= (bal & col) ? 1u << p : 0u;
+            }
+            while (todo) {
+                const int p = __builtin_ctz(todo);
+                todo &= todo - 1u;
+                const i4u blk = uload<i4u>(R.far_blk, b0 + p);
+                const int a0 = blk.x & 0xFFFF, na = blk.x >> 16, s0 = blk.y & 0xFFFF, nb = blk.y >> 16;
+                const float4* A = reinterpret_cast<const float4*>(s_T + 12 * ((blk.z & 0xFFFF) * kN + slot));
+                const float4* B = reinterpret_cast<const float4*>(s_T + 12 * ((blk.z >> 16) * kN + slot));
+                // M: B's link frame to A's, rotation transposed
+                float M[12];
+                {
+                    const float4 a0r = A[0], a1r = A[1], a2r = A[2], b0r = B[0], b1r = B[1], b2r = B[2];
+                    const float tx = b0r.w - a0r.w, ty = b1r.w - a1r.w, tz = b2r.w - a2r.w;
+                    auto row = [&](float u, float v, float x, float* m) {
+                        m[0] = fmaf(x, b2r.x, fmaf(v, b1r.x, u * b0r.x));
+                        m[1] = fmaf(x, b2r.y, fmaf(v, b1r.y, u * b0r.y));
+                        m[2] = fmaf(x, b2r.z, fmaf(v, b1r.z, u * b0r.z));
+                        m[3] = fmaf(x, tz, fmaf(v, ty, u * tx));
+                    };
+                    row(a0r.x, a1r.x, a2r.x, M);
+                    row(a0r.y, a1r.y, a2r.y, M + 4);
+                    row(a0r.z, a1r.z, a2r.z, M + 8);
+                }
+                for (int k0 = 0; k0 < nb; k0 += G) {
+                    const int k = min(k0 + sub, nb - 1);   // past the end: the last one again
+                    const float4 sp = s_sph[s0 + k];
+                    float x, y, z;
+                    aff_point(M, sp.x, sp.y, sp.z, x, y, z);
+                    const float bbq = fmaf(z, z, fmaf(y, y, x * x));
+                    const float cb = sp.w + slack;
+                    float mn = INFINITY;
+                    if (blk.w < 0) {
+                        for (int i = 0; i < na; i += 4) {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                const int t = 2 * (a0 + min(i + e, na - 1));
+                                const f4u c = uload<f4u>(R.far_sph, t);
+                                const float r2 = uload<float>(R.far_sph, 4 * (t + 1));
+                                mn = fminf(mn, fmaf(x, c.x, fmaf(y, c.y, fmaf(z, c.z, fmaf(cb, r2, c.w)))));
+                            }
+                        }
+                    } else {
+                        const int mask = R.far_mask[blk.w + k];
+                        for (int i = 0; i < na; ++i) {
+                            const int t = 2 * (a0 + i);
+                            const f4u c = uload<f4u>(R.far_sph, t);
+                            const float r2 = uload<float>(R.far_sph, 4 * (t + 1));
+                            const float v = fmaf(x, c.x, fmaf(y, c.y, fmaf(z, c.z, fmaf(cb, r2, c.w))));
+                            mn = fminf(mn, (mask >> i) & 1 ? v : INFINITY);
+                        }
+                    }
+                    const float val = fmaf(-cb, cb, bbq) + mn, err = 1e-6f * (bbq + R.far_scale2 + cb * cb);
+                    open = fminf(open, val - err);
+                    sure = fminf(sure, val + err + rsure * slack);
+                }
+            }
+        }
+#pragma unroll
+        for (int o = 1; o < G; o <<= 1) {
+            open = fminf(open, __shfl_xor(open, o));
+            sure = fminf(sure, __shfl_xor(sure, o));
+        }
+        const bool is_hit = active && sure < 0.0f;
+        const bool is_open = active && open < 0.0f && !is_hit;
+        if (active && sub == 0 && !is_open) {
+            if (!a.unit_first_hit) a.hit_out[ref.gs] = is_hit ? 1 : 0;
+            else if (is_hit) atomicMin((unsigned*)&a.unit_first_hit[ref.unit], (unsigned)ref.k);
+        }
+        // what is open, four states at a time
+        const unsigned long long om = __ballot(is_open && sub == 0);
+        if (om == 0ull) continue;
+        if (is_open && sub == 0) s_list[rank_below(om)] = slot;
+        const int n_open = __popcll(om);
+        const int sub16 = lane & (kSelfGroup - 1), st = lane / kSelfGroup;
+        const SelfLds L(base_lds, S, NC, J);
+        for (int i0 = 0; i0 < n_open; i0 += kSelfStates) {
+            __syncthreads();
+            const bool on = i0 + st < n_open;
+            const int col = s_list[on ? i0 + st : i0];
+            const int4 rf = s_ref[col];
+            group_frames(R, s_q + col, kN, L.T + st * (J * 12 + 4), L.par + st * J, sub16);
+            self_place(R, L, st, sub16);
+            __syncthreads();
+            self_pairs(a, L, st, sub16, on, on, rf.x, rf.y, rf.z);
+        }
     }
 }
 
@@ -3160,16 +3466,38 @@ hipError_t launch_clear(const ClearArgs& a, hipStream_t s) {
     return launch_args(k, (int)blocks, lds, s, &arg, nullptr, nullptr);
 }
 
+// Whether a self pass takes the two steps of k_self_far: any-collision checks
+// whose exact pairs decide alone, over at least 65,536 states in an order that
+// keeps neighbours near (edges and trajectories; a wave's near blocks are then
+// few), of models of up to 64 blocks. Measured, edges of 10 boxes with the
+// self check, us a call with it and without: Panda (23 blocks) 51,132 states 67
+// and 66, 180,857 106 and 124, 736,240 290 and 416; Fetch (153 blocks) 174,587 219
+// and 222, 699,268 664 and 787, but 48,403 126 and 104; Baxter (150) 877 and 714.
+// Uncorrelated configurations: Panda 262,144 170 and 173, Fetch 605 and 371.
+static bool self_far(const DRobot& R, int mode, int source, long n_states) {
+    return mode == 0 && R.far_blk && R.self_gate_implied && R.n_cpb <= 64 && n_states >= 65536 && source != kSrcConfig &&
+           source != kSrcBfs && FarLds(R).bytes <= 65536;
+}
+
+int self_chunk(const DRobot& R, int mode, int source, long n_states) {
+    return self_far(R, mode, source, n_states) ? kFarStates : kSelfStates;
+}
+
 hipError_t launch_self(const SelfArgs& a, hipStream_t s) {
+    const bool far = self_far(a.R, a.mode, a.X.source, a.X.n_states);
+    const int kn = far ? kFarStates : kSelfStates;
+    if (a.C.chunk != kn) return hipErrorInvalidValue;   // the caller's chunks are another size
     // X.n_states bounds the state count (a device-side count may be smaller,
     // then a bounded grid strides over it)
-    long blocks = a.C.tab ? (long)a.C.n_chunks : (a.X.n_states + kSelfStates - 1) / kSelfStates;
+    long blocks = a.C.tab ? (long)a.C.n_chunks : (a.X.n_states + kn - 1) / kn;
     if (a.X.n_dyn && blocks > 16384) blocks = 16384;
     if (blocks <= 0) return hipSuccess;
+    if (far) {
+        SelfArgs arg = a;
+        return launch_args((const void*)k_self_far, (int)blocks, FarLds(a.R).bytes, s, &arg, nullptr, nullptr);
+    }
     const bool gate = a.mode == 0 && !a.R.self_gate_implied;   // approximate pair positions
-    const size_t smem = sizeof(float4) * (size_t)kSelfStates * (a.R.n_sph + a.R.n_clu) +
-                        sizeof(float) * (size_t)kSelfStates * (a.R.n_joints * 12 + 4) +
-                        sizeof(float) * (size_t)kMaxDof * kSelfStates + sizeof(int) * (size_t)kSelfStates * a.R.n_joints +
+    const size_t smem = SelfLds::bytes(a.R.n_sph, a.R.n_clu, a.R.n_joints) + sizeof(float) * (size_t)kMaxDof * kSelfStates +
                         sizeof(int) * 2 * kWave + (gate ? sizeof(float4) * (size_t)kSelfStates * a.R.n_apx : 0);
     hipLaunchKernelGGL(k_self, dim3((unsigned)blocks), dim3(64), smem, s, a);
     return hipGetLastError();

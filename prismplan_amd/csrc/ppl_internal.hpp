@@ -55,6 +55,17 @@ struct DRobot {
     const int4* cpb;            // [n_cpb] self-pair blocks: (cluster A, cluster B, first pair, pairs), A <= B
     const unsigned* cpl;        // [n_pairs] block pair lists: slot a | slot b << 16 (emission slots)
     int n_cpb;
+    // The self pass's rough tests (NULL: the model's transforms are not rigid
+    // enough for them), one entry per block of cpb, its smaller cluster as B:
+    // (slot a0 | spheres << 16, slot b0 | spheres << 16, joint a | joint b << 16,
+    // first of B's masks in far_mask or -1 when the block holds every pair)
+    const int4* far_blk;        // [n_cpb]
+    const int* far_gate;        // [n_cpb] cluster A | cluster B << 16
+    const int* far_mask;        // per sphere of B: bit i set when A's sphere i is its partner
+    const float4* far_sph;      // [S][2] (-2 c, |c|^2 - r^2), (-2 r, 0, 0, 0) of emission slot k (centre c, radius r)
+    float far_slack;            // m: bounds how far the rough distances are off
+    float far_scale2;           // max (|c| + r)^2
+    float far_rmax;             // largest radius
     const int2* apx_pairs;      // [n_apx_pairs] approx self pairs (approx original indices)
     const float4* apx_orig;     // [A] approx spheres by original index
     const int* sph_jnt;         // [S] DFS joint of emission slot k
@@ -190,7 +201,7 @@ struct SelfArgs {
     int* unit_first_hit;        // mode 0, nullable: per-unit first hit (-1 free); states of units with a
                                 // hit are skipped and a self collision lowers the unit's entry instead of hit_out
     float* out;                 // [n_states][8]: clr, i, j (as int bits), nx, ny, nz, -, -
-    DChunks C;                  // the plan's 4-state chunks (tab NULL: states in flat order); outputs are
+    DChunks C;                  // chunks of C.chunk states (tab NULL: states in flat order); outputs are
                                 // indexed by plan order either way
 };
 
@@ -202,6 +213,9 @@ hipError_t launch_cost_grp(const CostArgs& a, int grid, hipStream_t s, hipEvent_
                            hipEvent_t t1 = nullptr);
 hipError_t launch_clear(const ClearArgs& a, hipStream_t s);
 hipError_t launch_self(const SelfArgs& a, hipStream_t s);
+// States per chunk of a self pass over n_states states (a bound, if they are
+// counted on the device): what its chunk table must hold.
+int self_chunk(const DRobot& R, int mode, int source, long n_states);
 hipError_t launch_fill_i32(int* p, int v, long n, hipStream_t s);
 hipError_t launch_add_u32(unsigned* p, unsigned v, hipStream_t s);   // *p += v (one thread)
 // CHOMP optimiser pieces (trajectory plans, dim-major [D][T] blocks).

@@ -134,3 +134,36 @@ def test_collide_rows_and_queue(name, n, boxes):
     off = np.concatenate([[0], np.cumsum(ns)])
     first = np.array([(np.flatnonzero(hits[off[e]:off[e + 1]])[:1].tolist() or [-1])[0] for e in range(n)])
     np.testing.assert_array_equal(fh, first)
+
+
+@pytest.mark.parametrize("margin,skip", [(0.0, False), (0.0, True)])
+def test_rough_self_pass_equals_the_exact_one(robots, margin, skip):
+    """Edge plans of at least 65,536 states take the two-step self pass, smaller
+    ones the exact pass alone: the same edges give the same verdicts and first
+    hits bit for bit, and both agree with the oracle outside its band."""
+    from prismplan_amd.planning_scene import HostScene
+    rob = robots["panda"]
+    arr, n = rob.arrays, 2100
+    rng = np.random.default_rng(77)
+    q = W.uniform_configs(rng, arr, n)
+    to = np.clip(q + rng.uniform(-0.8, 0.8, q.shape), arr.joint_lower, arr.joint_upper).astype(np.float32)
+    ns = rng.integers(2, 64, n).astype(np.int32)
+    ns[:3] = (1, 65, 16)
+    ds = S.DeviceScene.from_host(HostScene())
+
+    def run(lo, hi):
+        plan = S.Plan.edges(rob, ns[lo:hi])
+        out = S.edge_check_batched(plan, ds, torch.from_numpy(q[lo:hi]).to(DEV), torch.from_numpy(to[lo:hi]).to(DEV),
+                                   collision_margin=margin, check_self=True, skip_resolved=skip, state_hits=not skip)
+        fh, hits = (out, None) if skip else out
+        return plan.n_states, fh.cpu().numpy(), None if skip else hits.cpu().numpy()
+
+    total, fh, hits = run(0, n)
+    assert total >= 65536
+    parts = [run(k, min(k + 700, n)) for k in range(0, n, 700)]
+    assert all(p[0] < 65536 for p in parts)
+    np.testing.assert_array_equal(fh, np.concatenate([p[1] for p in parts]))
+    if not skip:
+        np.testing.assert_array_equal(hits, np.concatenate([p[2] for p in parts]))
+        ref, clr = PO.Oracle(arr).check_collision(PO.edge_states(q, to, ns), check_self=True)
+        assert not np.any((hits != ref) & (np.abs(clr) >= 1e-5)) and 0.05 < ref.mean() < 0.5
