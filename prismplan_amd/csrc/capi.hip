@@ -120,7 +120,7 @@ struct ppl_edge_eval_s {
     hipStream_t stream = nullptr;
     // one call's inputs and first hits, packed [offsets][first hits][from][to]
     // (256-byte aligned parts) in one pinned block and one device block
-    DBuf d_io, d_clr_state, d_clr_edge, d_self;
+    DBuf d_io, d_clr_state, d_clr_edge;
     HBuf h_io, h_clr;
 };
 
@@ -1254,7 +1254,7 @@ ppl_status ppl_edge_eval_create(ppl_robot r, const ppl_scene_view* view, int dim
 ppl_status ppl_edge_eval_destroy(ppl_edge_eval ev) try {
     if (!ev) return PPL_OK;
     if (ev->stream) (void)hipStreamSynchronize(ev->stream);
-    ev->d_io.release(); ev->d_clr_state.release(); ev->d_clr_edge.release(); ev->d_self.release();
+    ev->d_io.release(); ev->d_clr_state.release(); ev->d_clr_edge.release();
     ev->h_io.release(); ev->h_clr.release();
     if (ev->stream) (void)hipStreamDestroy(ev->stream);
     delete ev;
@@ -1333,13 +1333,6 @@ ppl_status ppl_edge_eval_evaluate(ppl_edge_eval ev, const float* h_from, const f
     X.n_edges = n;
     X.k0 = 1;
     // With G = granularity <= 1 the +1 state count gives t = k/G as the reference.
-    const uint8_t* self_hit = nullptr;
-    if (total > 0 && p->check_self && r->n_pairs > 0) {
-        HIP_TRY(ev->d_self.ensure((size_t)total));
-        ppl_status st = run_self(r, X, 0, ev->d_self.as<uint8_t>(), nullptr, ev->stream);
-        if (st != PPL_OK) return st;
-        self_hit = ev->d_self.as<uint8_t>();
-    }
     if (total > 0) {
         CollideArgs a{};
         a.R = r->R;
@@ -1351,8 +1344,12 @@ ppl_status ppl_edge_eval_evaluate(ppl_edge_eval ev, const float* h_from, const f
         a.mode = 1;
         a.skip_resolved = 1;
         a.first_hit = d_fh;
-        a.self_hit = self_hit;
         HIP_TRY(launch_collide(a, grid, ev->stream));
+        // then the self check, on states below their edge's known hit
+        if (p->check_self && r->n_pairs > 0) {
+            ppl_status st = run_self(r, X, 0, nullptr, nullptr, ev->stream, FLT_MAX, d_fh);
+            if (st != PPL_OK) return st;
+        }
     }
     const bool want_clr = p->compute_clearance && h_clr;
     if (want_clr && total > 0) {
@@ -2457,7 +2454,13 @@ ppl_status ppl_edge_check_batched(ppl_plan P, const ppl_scene_view* view, const 
     X.from = d_from;
     X.to = d_to;
     const uint8_t* self_hit = nullptr;
-    if (prm->check_self && P->robot->n_pairs > 0) {
+    const bool self = prm->check_self && P->robot->n_pairs > 0;
+    // With skipping, the self pass follows the environment's and leaves out the
+    // states past a hit that is known by then; first hits are the same in either
+    // order. (48% of the edges among 10 boxes end that way: 736,240 states 297 ->
+    // 244 us a call.)
+    const bool self_after = self && prm->skip_resolved;
+    if (self && !self_after) {
         HIP_TRY(P->d_self.ensure((size_t)P->n_states));
         if ((st = run_self(P->robot, X, 0, P->d_self.as<uint8_t>(), nullptr, s, FLT_MAX, nullptr, P)) != PPL_OK)
             return st;
@@ -2479,6 +2482,7 @@ ppl_status ppl_edge_check_batched(ppl_plan P, const ppl_scene_view* view, const 
     if (timing_now(P, s)) HIP_TRY(timing_pair(P, &t0, &t1));
     HIP_TRY(launch_collide(a, grid, s, t0, t1));
     if (t0) ++P->kused;
+    if (self_after) return run_self(P->robot, X, 0, nullptr, nullptr, s, FLT_MAX, d_first_hit, P);
     return PPL_OK;
 } catch (const std::bad_alloc&) {
     return ppl::fail_msg(PPL_ERR_ALLOC, "out of host memory");
