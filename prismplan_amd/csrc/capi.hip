@@ -1974,6 +1974,13 @@ ppl_status dense_check_setup(const ppl_plan_s* P, const DScene& S, float step, f
     dc.va.margin = margin;
     dc.va.mode = 1;
     dc.va.skip_resolved = 1;
+    // Only whether a trajectory collides counts, and most of those that do
+    // collide early in any even sample of their states: the chunks are visited
+    // spread over all trajectories, so that a wave's later chunks are mostly of
+    // trajectories already decided (256 trajectories densified to 2.0 M states:
+    // 170 -> 80 us).
+    dc.va.any = 1;
+    dc.va.C.spread = 1;
     dc.va.first_hit = first_hit;
     dc.va.self_hit = nullptr;
     dc.va.C.unit_hint = hint;
@@ -2775,6 +2782,7 @@ ppl_status ppl_mitstar_edge_cc(ppl_robot r, const ppl_scene_view* view, const fl
         a.margin = margin;
         a.mode = 1;
         a.skip_resolved = 1;
+        a.any = 1;
         a.first_hit = first_hit;
         HIP_TRY(launch_collide(a, grid, s));
         // self after the environment, on the edges still free (two_phase_cc's order)

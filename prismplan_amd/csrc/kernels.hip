@@ -704,9 +704,21 @@ __device__ __forceinline__ int chunk_count(const DChunks& C, long n_states) {
 __device__ __forceinline__ long state_count(const DStates& X) { return X.n_dyn ? (long)uniform(*X.n_dyn) : X.n_states; }
 
 __device__ __forceinline__ bool next_chunk(const DChunks& C, long n_states, int n_chunks, ChunkCursor& cur, int4& ch) {
-    const int c = cur.next;
-    if (c >= n_chunks) return false;
-    cur.next += cur.stride;
+    int c = cur.next;
+    if (C.spread) {
+        // a bijection of [0, 2^m) >= n_chunks that sends neighbours far apart
+        // (odd multiplier near 2^32 over the golden ratio)
+        const unsigned mask = n_chunks > 1 ? 0xFFFFFFFFu >> __builtin_clz((unsigned)(n_chunks - 1)) : 0u;
+        for (;;) {
+            if ((unsigned)cur.next > mask || n_chunks <= 0) return false;
+            c = (int)(((unsigned)cur.next * 0x9E3779B1u) & mask);
+            cur.next += cur.stride;
+            if (c < n_chunks) break;
+        }
+    } else {
+        if (c >= n_chunks) return false;
+        cur.next += cur.stride;
+    }
     if (C.tab) {
         ch = C.tab[c];
         ch.x = uniform(ch.x); ch.y = uniform(ch.y); ch.z = uniform(ch.z); ch.w = uniform(ch.w);
@@ -830,6 +842,15 @@ __global__ __launch_bounds__(64, 4) void k_collide(CollideArgs a) {
     while (have) {
         int4 chn;
         const bool have_n = next_chunk(a.C, n_states, n_chunks, cur, chn);
+        // a chunk inside one unit that already has its hit (read past the
+        // caches, which would keep an old entry for the whole launch)
+        if (a.any && ch.w >= 0 && __builtin_amdgcn_readlane(pf_end, 0) >= ch.z &&
+            __hip_atomic_load(a.first_hit + ch.w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= 0) {
+            if (have_n) prefetch_unit_ends(a.X, chn.w, pf_end, pf_beg);
+            ch = chn;
+            have = have_n;
+            continue;
+        }
         if (ch.x != cur_prob) {
             problem_obbs(a.C, a.S, ch.x, o0, o1);
             n_tiles = uniform(obb_tiles(o0, o1, cap));
@@ -851,7 +872,7 @@ __global__ __launch_bounds__(64, 4) void k_collide(CollideArgs a) {
         if (active && a.self_hit && a.self_hit[ref.gs]) { hit = true; active = false; }
         if (active && a.mode == 1 && a.skip_resolved) {
             const unsigned fh = (unsigned)a.first_hit[ref.unit];
-            if (fh < (unsigned)ref.k) active = false;
+            if (a.any ? fh != ~0u : fh < (unsigned)ref.k) active = false;
         }
         if (have_n) prefetch_unit_ends(a.X, chn.w, pf_end, pf_beg);
         __syncthreads();
@@ -1062,7 +1083,7 @@ __global__ __launch_bounds__(64) void k_collide_gated(CollideArgs a) {
         if (active && a.self_hit && a.self_hit[ref.gs]) { hit = true; active = false; }
         if (active && a.mode == 1 && a.skip_resolved) {
             const unsigned fh = (unsigned)a.first_hit[ref.unit];
-            if (fh < (unsigned)ref.k) active = false;
+            if (a.any ? fh != ~0u : fh < (unsigned)ref.k) active = false;
         }
         __syncthreads();
         // 1. approximate pass: bit jj of `flagged` once an approximate sphere

@@ -157,6 +157,7 @@ struct DChunks {
     int tiled;                  // some problem has more OBBs than obb_cap: they pass through LDS in tiles
                                 // (k_collide, the grouped cost kernel; k_cost refuses such launches)
     const int* unit_hint;       // implicit chunks (tab NULL), nullable: unit holding state 64 k, for each k
+    int spread;                 // implicit chunks are visited spread over the whole range, not in order
 };
 
 struct DCostParams {
@@ -170,6 +171,8 @@ struct CollideArgs {
     float margin;
     int mode;                   // 0 per-state verdict, 1 edge first-hit
     int skip_resolved;          // first-hit mode: skip states past a known hit
+    int any;                    // first-hit mode: only whether a unit has a hit counts (its entry then is some hit's
+                                // state), so every state of a unit that has one is skipped
     uint8_t* out;               // [n_states] verdicts (nullable in mode 1)
     int* first_hit;             // [n_edges] (mode 1), -1 = free
     const uint8_t* self_hit;    // [n_states] precomputed self verdicts (nullable)
