@@ -1994,7 +1994,6 @@ ppl_status dense_check_setup(const ppl_plan_s* P, const DScene& S, float step, f
 ppl_status dense_check_run(const ppl_robot_s* r, const ChompArgs& a, DenseCheck& dc, hipStream_t s) {
     HIP_TRY(launch_chomp_nsub(a, s));
     HIP_TRY(launch_unit_hint(a.dense_off, (int)dc.n_traj, dc.hint, dc.n_hint, s));
-    HIP_TRY(launch_fill_i32(dc.first_hit, -1, dc.n_traj, s));
     HIP_TRY(launch_collide(dc.va, dc.vgrid, s));
     if (r->n_pairs > 0) return run_self(r, dc.Xd, 0, nullptr, nullptr, s, FLT_MAX, dc.first_hit, nullptr, dc.hint);
     return PPL_OK;
@@ -2199,10 +2198,11 @@ ppl_status ppl_chomp_optimize(ppl_plan P, const ppl_scene_view* view, const ppl_
     auto evaluate = [&](hipStream_t q) -> ppl_status {
         ppl_status e = cs->fd_gradient ? fd_impl(P, view, d_theta, &cp, cs->fd_eps, grad, q) : PPL_OK;
         if (e != PPL_OK) return e;
-        e = hinge_impl(P, view, d_theta, &cp, state, total, cs->fd_gradient ? nullptr : grad, q);
+        e = hinge_impl(P, view, d_theta, &cp, state, nullptr, cs->fd_gradient ? nullptr : grad, q);
         if (e != PPL_OK) return e;
-        HIP_TRY(launch_control_cost(d_theta, P->d_off, P->n_units, D, cs->dt, cs->smoothness_weight, total, 1, q,
-                                    P->t_max));
+        // totals: the state costs' sum and the control cost in one launch
+        HIP_TRY(launch_control_cost(d_theta, P->d_off, P->n_units, D, cs->dt, cs->smoothness_weight, total, 0, q,
+                                    P->t_max, state));
         return dense_check_run(r, a, dc, q);
     };
     auto iteration = [&](hipStream_t q) -> ppl_status {
@@ -2290,10 +2290,10 @@ ppl_status ppl_stomp_optimize(ppl_plan P, const ppl_scene_view* view, const ppl_
                                 z->dense_off, z->hint.as<int>(), a, dc)) != PPL_OK)
         return st;
     auto evaluate = [&](hipStream_t q) -> ppl_status {
-        ppl_status e = hinge_impl(P, view, d_theta, &cp, z->theta_cost, z->totals, nullptr, q);
+        ppl_status e = hinge_impl(P, view, d_theta, &cp, z->theta_cost, nullptr, nullptr, q);
         if (e != PPL_OK) return e;
-        HIP_TRY(launch_control_cost(d_theta, P->d_off, B, D, ss->dt, ss->control_cost_weight, z->totals, 1, q,
-                                    P->t_max));
+        HIP_TRY(launch_control_cost(d_theta, P->d_off, B, D, ss->dt, ss->control_cost_weight, z->totals, 0, q,
+                                    P->t_max, z->theta_cost));
         return dense_check_run(r, a, dc, q);
     };
     if (first_call) {

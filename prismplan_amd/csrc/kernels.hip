@@ -2385,6 +2385,10 @@ __global__ __launch_bounds__(64, 4) void k_self_far(SelfArgs a) {
             active = g < n_states;
             if (a.C.unit_hint) {
                 u0 = uniform(a.C.unit_hint[base >> 6]);
+                // a chunk inside one unit that has its hit
+                if (a.unit_first_hit && a.X.source != kSrcEdge && a.X.dense_off[u0 + 1] >= base + kN &&
+                    a.unit_first_hit[u0] >= 0)
+                    continue;
                 stage_unit_ends(a.X, u0, s_end);
             }
         }
@@ -2675,6 +2679,7 @@ __global__ __launch_bounds__(64) void k_chomp_nsub(ChompArgs a) {
         if (a.check_step > 0.0f && m > a.check_step)
             n = (int)fminf(ceilf(__fdiv_rn(m, a.check_step)), (float)a.nsub_max);
         a.nsub[b] = n;
+        a.first_hit[b] = -1;   // for the validity pass that follows
     }
 }
 

@@ -229,10 +229,10 @@ struct ChompArgs {
     int nsub_max;               // densification cap (joint-limit box diagonal / step)
     const float* const* ainv;   // [n_traj] A^-1 (T x T) of each trajectory's length
     float* theta; float* best; float* record; const float* grad; const float* total;
-    const int* first_hit;       // [n_traj] validity pass result, -1 = collision-free
+    int* first_hit;             // [n_traj] validity pass result, -1 = collision-free (launch_chomp_nsub resets it)
     int* nsub; int* dense_off;  // [n_traj], [n_traj + 1]
 };
-hipError_t launch_chomp_nsub(const ChompArgs& a, hipStream_t s);   // nsub + dense_off (scan)
+hipError_t launch_chomp_nsub(const ChompArgs& a, hipStream_t s);   // nsub + dense_off (scan), first_hit = -1
 hipError_t launch_chomp_book(const ChompArgs& a, int initial, hipStream_t s);
 hipError_t launch_chomp_update(const ChompArgs& a, int max_t, hipStream_t s);
 
