@@ -895,7 +895,7 @@ ppl_status ppl_robot_create(const ppl_robot_desc* d, ppl_robot* out) try {
     // They measure B's spheres in A's link frame, so the transforms must be
     // rigid; far_slack bounds the distance error of the deviation and of FP32
     // over the model's reach.
-    std::vector<int4> far_blk;
+    std::vector<int4> far_blk, cpx;
     std::vector<int> far_gate, far_mask;
     std::vector<float4> far_sph((size_t)2 * S);
     double far_slack = 0.0, far_scale = 0.0, far_rmax = 0.0;
@@ -924,6 +924,14 @@ ppl_status ppl_robot_create(const ppl_robot_desc* d, ppl_robot* out) try {
         }
         far_slack = 2e-5 + (reach + far_scale) * (2.0 * J * dev + 4e-6);
         far_ok = far_ok && dev <= 1e-5 && far_slack < 1e-2;
+        for (const int4& blk : cpb) {
+            const int a0 = clu_beg[blk.x], b0 = clu_beg[blk.y], na = clu_beg[blk.x + 1] - a0, nb = clu_beg[blk.y + 1] - b0;
+            bool all = blk.w == na * nb && blk.w <= 256;
+            for (int t = 0; t < blk.w && all; ++t)
+                all = cpl[blk.z + t] == ((unsigned)(a0 + t / nb) | ((unsigned)(b0 + t % nb) << 16));
+            cpx.push_back(make_int4(blk.x | (blk.y << 8) | ((all ? nb : 0) << 16), a0 | (b0 << 16), blk.z,
+                                    blk.w | ((all ? (4096 + nb - 1) / nb : 0) << 16)));
+        }
         for (const int4& blk : cpb) {
             int ca = blk.x, cb = blk.y;
             auto count = [&](int c) { return clu_beg[c + 1] - clu_beg[c]; };
@@ -1031,8 +1039,9 @@ ppl_status ppl_robot_create(const ppl_robot_desc* d, ppl_robot* out) try {
     hipError_t e = hipMemcpy(r->blob, host.data(), host.size(), hipMemcpyHostToDevice);
     // the rough self tests' tables lie apart from the blob whose digest keys the tuning cache
     const size_t o_fb = 0, o_fs = o_fb + far_blk.size() * 16, o_fg = o_fs + far_sph.size() * 16,
-                 o_fm = o_fg + far_gate.size() * 4;
-    std::vector<char> far_host(o_fm + far_mask.size() * 4 + 16, 0);
+                 o_fm = o_fg + far_gate.size() * 4, o_fx = (o_fm + far_mask.size() * 4 + 15) & ~(size_t)15;
+    std::vector<char> far_host(o_fx + cpx.size() * 16 + 16, 0);
+    if (!cpx.empty()) memcpy(far_host.data() + o_fx, cpx.data(), cpx.size() * 16);
     if (!far_blk.empty()) memcpy(far_host.data() + o_fb, far_blk.data(), far_blk.size() * 16);
     if (!far_sph.empty()) memcpy(far_host.data() + o_fs, far_sph.data(), far_sph.size() * 16);
     if (!far_gate.empty()) memcpy(far_host.data() + o_fg, far_gate.data(), far_gate.size() * 4);
@@ -1072,6 +1081,7 @@ ppl_status ppl_robot_create(const ppl_robot_desc* d, ppl_robot* out) try {
     R.apx_jnt = reinterpret_cast<const int*>(b + o_ajnt);
     char* fb = static_cast<char*>(r->far_blob);
     R.far_blk = far_ok && !far_blk.empty() ? reinterpret_cast<const int4*>(fb + o_fb) : nullptr;
+    R.cpx = reinterpret_cast<const int4*>(fb + o_fx);
     R.far_sph = reinterpret_cast<const float4*>(fb + o_fs);
     R.far_gate = reinterpret_cast<const int*>(fb + o_fg);
     R.far_mask = reinterpret_cast<const int*>(fb + o_fm);

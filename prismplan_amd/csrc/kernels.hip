@@ -61,30 +61,10 @@ __device__ __forceinline__ void aff_identity(float* T) {
     T[0] = T[5] = T[10] = 1.0f;
 }
 
-// S = FT * M(q), restating xrot_fn / yrot_fn / zrot_fn / prism_fn
-// (planning/utils.cuh:560-702). FIXED or unknown types move nothing.
-__device__ __forceinline__ void joint_step(const float* __restrict__ ft, int type, float q, float* S) {
-#pragma unroll
-    for (int i = 0; i < 12; ++i) S[i] = ft[i];
-    if (type >= kXRot) {
-        float s, c;
-        sincosf(q, &s, &c);
-        const int a = (type == kXRot) ? 1 : (type == kYRot ? 2 : 0);
-        const int b = (type == kXRot) ? 2 : (type == kYRot ? 0 : 1);
-#pragma unroll
-        for (int r = 0; r < 3; ++r) {
-            const float fa = ft[r * 4 + a], fb = ft[r * 4 + b];
-            S[r * 4 + a] = fmaf(fa, c, fb * s);
-            S[r * 4 + b] = fmaf(fb, c, -fa * s);
-        }
-    } else if (type >= kXPrism) {
-#pragma unroll
-        for (int r = 0; r < 3; ++r) S[r * 4 + 3] = fmaf(ft[r * 4 + type], q, ft[r * 4 + 3]);
-    }
-}
-
-// The same step for a joint that is the same in every lane (rows of the fixed
-// transform by scalar loads; the same operations, so the same bits).
+// S = FT * M(q) for a joint that is the same in every lane, restating xrot_fn /
+// yrot_fn / zrot_fn / prism_fn (planning/utils.cuh:560-702); FIXED or unknown
+// types move nothing. tab: [J][12] rows of the fixed transforms, by scalar
+// loads; s, c: sine and cosine of q (revolute joints).
 template <int A, int B>
 __device__ __forceinline__ void rot_cols(float s, float c, float* S) {
 #pragma unroll
@@ -1499,24 +1479,67 @@ __global__ __launch_bounds__(64, 4) void k_cost(CostArgs a) {
 // link, until P is the root. Then A is the product of the steps from the root
 // down to jj: the frame. ceil(log2(depth)) rounds through LDS. qs: the
 // state's q (q_d = qs[d * qstride]); par: J ints of LDS for the links.
-// APPROX: the approximate spheres' own chain (R.aft / R.atype).
 // Contains block barriers: every lane of the workgroup must call it.
-template <bool APPROX = false>
-__device__ __forceinline__ void group_frames(const DRobot& R, const float* qs, int qstride, float* F, int* par,
-                                             int sub) {
-    const int J = R.n_joints;
+// jt: the lane's joint (DFS position `sub`), in registers, so that a caller with
+// several rounds loads it once.
+struct JointRegs {
+    float ft[12];
+    int type, dof, parent;
+    template <bool APPROX = false>
+    __device__ __forceinline__ void load(const DRobot& R, int sub) {
+        type = dof = -1;
+        parent = 0;
+#pragma unroll
+        for (int k = 0; k < 12; ++k) ft[k] = 0.0f;
+        if (sub == 0) {
+            ft[0] = ft[5] = ft[10] = 1.0f;
+        } else if (sub < R.n_joints) {
+            const int4 meta = R.jmeta[sub];
+            const float4* f = reinterpret_cast<const float4*>((APPROX ? R.aft : R.ft) + 12 * sub);
+            const float4 f0 = f[0], f1 = f[1], f2 = f[2];
+            ft[0] = f0.x; ft[1] = f0.y; ft[2] = f0.z; ft[3] = f0.w;
+            ft[4] = f1.x; ft[5] = f1.y; ft[6] = f1.z; ft[7] = f1.w;
+            ft[8] = f2.x; ft[9] = f2.y; ft[10] = f2.z; ft[11] = f2.w;
+            type = APPROX ? R.atype[sub] : meta.x;
+            dof = meta.y;
+            parent = R.parent[sub];
+        }
+    }
+    // joint_step_u of the lane's joint, its columns picked by selects
+    __device__ __forceinline__ void step(float q, float* S) const {
+#pragma unroll
+        for (int k = 0; k < 12; ++k) S[k] = ft[k];
+        if (type >= kXRot) {
+            float s, c;
+            sincosf(q, &s, &c);
+            const bool x = type == kXRot, y = type == kYRot;
+#pragma unroll
+            for (int r = 0; r < 3; ++r) {
+                const float f0 = ft[r * 4], f1 = ft[r * 4 + 1], f2 = ft[r * 4 + 2];
+                const float fa = x ? f1 : y ? f2 : f0, fb = x ? f2 : y ? f0 : f1;
+                const float na = fmaf(fa, c, fb * s), nb = fmaf(fb, c, -fa * s);
+                S[r * 4] = x ? f0 : y ? nb : na;
+                S[r * 4 + 1] = x ? na : y ? f1 : nb;
+                S[r * 4 + 2] = x ? nb : y ? na : f2;
+            }
+        } else if (type >= kXPrism) {
+#pragma unroll
+            for (int r = 0; r < 3; ++r) {
+                const float f = type == kXPrism ? ft[r * 4] : type == kYPrism ? ft[r * 4 + 1] : ft[r * 4 + 2];
+                S[r * 4 + 3] = fmaf(f, q, ft[r * 4 + 3]);
+            }
+        }
+    }
+};
+
+__device__ __forceinline__ void group_frames(const JointRegs& jt, int J, const float* qs, int qstride, float* F,
+                                             int* par, int sub) {
     const bool own = sub < J;
     int P = 0;
     if (own) {
         float A[12];
-        if (sub == 0) {
-            aff_identity(A);
-        } else {
-            const int4 meta = R.jmeta[sub];
-            const float q = meta.y >= 0 ? qs[meta.y * qstride] : 0.0f;
-            joint_step(APPROX ? R.aft + 12 * sub : R.ft + 12 * sub, APPROX ? R.atype[sub] : meta.x, q, A);
-            P = R.parent[sub];
-        }
+        jt.step(jt.dof >= 0 ? qs[jt.dof * qstride] : 0.0f, A);
+        P = jt.parent;
         float4* d = reinterpret_cast<float4*>(F + 12 * sub);
         d[0] = make_float4(A[0], A[1], A[2], A[3]);
         d[1] = make_float4(A[4], A[5], A[6], A[7]);
@@ -1734,7 +1757,9 @@ __device__ __forceinline__ void cost_grp(const CostArgs& a) {
         StateRef ref = load_state(a.X, D, g, active, s_q, ch.w, s_end, ch.x, slot, kGrpStates, sub == 0);
         __syncthreads();
         // 1a. joint frames (pointer jumping over the DFS tree)
-        group_frames(R, s_q + slot, kGrpStates, Ts, s_par + slot * J, sub);
+        JointRegs jt;
+        jt.load(R, sub);
+        group_frames(jt, J, s_q + slot, kGrpStates, Ts, s_par + slot * J, sub);
         // 1b. candidate masks per sphere cluster; a tiled problem's OBBs pass through
         // LDS tile by tile, each tile's argmins folded into s_best / s_barg
         // (tiles in index order and a strict < keep the lowest index on ties)
@@ -2037,6 +2062,11 @@ __global__ __launch_bounds__(64, 4) void k_clear(ClearArgs a) {
 //         runtime_kinematics.cuh:248-283);
 // mode 1: min over pairs of |d| - ri - rj with argmin pair and unit normal
 //         (runtime_kinematics.cuh:294-329).
+// Bound by VALU and SALU issue and the chain of a chunk's loads. Per chunk of
+// four Fetch states: 1,850 VALU and 970 SALU instructions before, 1,445 and
+// 640 now, with the gates and the far pairs told without square roots, the
+// pairs of full blocks numbered instead of listed, the table entries in flight
+// together and one kernel per mode: 325,152 rollout states 394 -> 290 us.
 // ===========================================================================
 constexpr int kSelfStates = kWave / kSelfGroup;
 static_assert(kSelfGroup >= kMaxJoints, "the self pass composes frames with one joint per lane of a state group");
@@ -2068,27 +2098,34 @@ __device__ __forceinline__ void self_place(const DRobot& R, const SelfLds& L, in
     const float* Ts = L.T + st * (R.n_joints * 12 + 4);
     // sphere centres (emission slot k: a joint's spheres are contiguous) and
     // each sphere cluster's enclosing sphere, from the frames
-    for (int k = sub; k < S; k += kSelfGroup) {
-        const float4 sp = R.sph[k];
-        const float4* Tq = reinterpret_cast<const float4*>(Ts + 12 * R.sph_jnt[k]);
+    // (each lane's table entries four at a time, before the first is used)
+    auto put = [&](const float4& sp, int jj, float4* out) {
+        const float4* Tq = reinterpret_cast<const float4*>(Ts + 12 * jj);
         const float4 t0 = Tq[0], t1 = Tq[1], t2 = Tq[2];
-        pos[k] = make_float4(fmaf(t0.x, sp.x, fmaf(t0.y, sp.y, fmaf(t0.z, sp.z, t0.w))),
-                             fmaf(t1.x, sp.x, fmaf(t1.y, sp.y, fmaf(t1.z, sp.z, t1.w))),
-                             fmaf(t2.x, sp.x, fmaf(t2.y, sp.y, fmaf(t2.z, sp.z, t2.w))), sp.w);
+        *out = make_float4(fmaf(t0.x, sp.x, fmaf(t0.y, sp.y, fmaf(t0.z, sp.z, t0.w))),
+                           fmaf(t1.x, sp.x, fmaf(t1.y, sp.y, fmaf(t1.z, sp.z, t1.w))),
+                           fmaf(t2.x, sp.x, fmaf(t2.y, sp.y, fmaf(t2.z, sp.z, t2.w))), sp.w);
+    };
+    for (int k0 = sub; k0 < S; k0 += 4 * kSelfGroup) {
+        float4 sp[4];
+        int jj[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int k = min(k0 + e * kSelfGroup, S - 1);
+            sp[e] = R.sph[k];
+            jj[e] = R.sph_jnt[k];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (k0 + e * kSelfGroup < S) put(sp[e], jj[e], pos + k0 + e * kSelfGroup);
     }
-    for (int c = sub; c < NC; c += kSelfGroup) {
-        const float4 ce = R.clu_enc[c];
-        const float4* Tq = reinterpret_cast<const float4*>(Ts + 12 * R.clu_jnt[c]);
-        const float4 t0 = Tq[0], t1 = Tq[1], t2 = Tq[2];
-        cenc[c] = make_float4(fmaf(t0.x, ce.x, fmaf(t0.y, ce.y, fmaf(t0.z, ce.z, t0.w))),
-                              fmaf(t1.x, ce.x, fmaf(t1.y, ce.y, fmaf(t1.z, ce.z, t1.w))),
-                              fmaf(t2.x, ce.x, fmaf(t2.y, ce.y, fmaf(t2.z, ce.z, t2.w))), ce.w);
-    }
+    for (int c = sub; c < NC; c += kSelfGroup) put(R.clu_enc[c], R.clu_jnt[c], cenc + c);
 }
 
 // Exact self check of the four states (16 lanes each) from their sphere
 // centres: the pairs of every block whose clusters are near, the outputs of
-// states with `active`. live: states whose pairs are checked.
+// states with `active`. live: states whose pairs are checked. MODE: the pass's.
+template <int MODE>
 __device__ __forceinline__ void self_pairs(const SelfArgs& a, const SelfLds& L, int st, int sub, bool active, bool live,
                                            long gs, int unit, int kstate) {
     const DRobot& R = a.R;
@@ -2101,24 +2138,27 @@ __device__ __forceinline__ void self_pairs(const SelfArgs& a, const SelfLds& L, 
     // strict d^2 < (r_i + r_j)^2 test). The 16 lanes of a state test 16
     // blocks at once; then every block that passes for some state of the
     // wave has its pair list walked, 16 pairs per step.
-    const float band = a.mode == 0 ? 0.0f : a.band;
+    const float band = MODE == 0 ? 0.0f : a.band;
     auto near = [&](float4 e, float4 f) {
         const float dx = e.x - f.x, dy = e.y - f.y, dz = e.z - f.z;
         const float d2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-        const float rs = e.w + f.w;
-        return a.mode == 0 ? d2 < rs * rs : sqrtf(d2) - rs < band;
+        // (mode 1: |d| - rs < band, squared; the enclosing spheres' padding covers the rounding)
+        const float rs = MODE == 0 ? e.w + f.w : fmaxf(e.w + f.w + band, 0.0f);
+        return d2 < rs * rs;
     };
     float best = 1000.0f;
     int bkey = INT_MAX;   // (block << 16 | pair) of the best pair: ties go to the first
     bool hit = false;
-    // lane sub holds the entry of block b0 + sub, the next pass's loaded ahead;
-    // a walked block's list comes from its lane in the first state group
-    int4 nb4 = sub < R.n_cpb ? R.cpb[sub] : make_int4(0, 0, 0, 0);
+    // lane sub holds the entry of block b0 + sub (DRobot::cpx), the next pass's
+    // loaded ahead; a walked block's comes from its lane in the first state
+    // group. A block of all pairs of its clusters, nearly every one, gives pair k's
+    // slots by a division, without a look at the list.
+    int4 nb4 = sub < R.n_cpb ? R.cpx[sub] : make_int4(0, 0, 0, 0);
     for (int b0 = 0; b0 < R.n_cpb; b0 += kSelfGroup) {
         const int bb = b0 + sub;
         const int4 hb = nb4;
-        if (bb + kSelfGroup < R.n_cpb) nb4 = R.cpb[bb + kSelfGroup];
-        const bool g = live && !hit && bb < R.n_cpb && near(cenc[hb.x], cenc[hb.y]);
+        if (bb + kSelfGroup < R.n_cpb) nb4 = R.cpx[bb + kSelfGroup];
+        const bool g = live && !hit && bb < R.n_cpb && near(cenc[hb.x & 0xFF], cenc[(hb.x >> 8) & 0xFF]);
         const unsigned long long bal = __ballot(g);
         const unsigned mine = (unsigned)(bal >> (st * kSelfGroup)) & 0xFFFFu;
         unsigned todo = (unsigned)(bal | (bal >> 16) | (bal >> 32) | (bal >> 48)) & 0xFFFFu;   // wave-uniform
@@ -2126,35 +2166,51 @@ __device__ __forceinline__ void self_pairs(const SelfArgs& a, const SelfLds& L, 
             const int t = __builtin_ctz(todo);
             todo &= todo - 1u;
             const int b = b0 + t;
-            const int first = __builtin_amdgcn_readlane(hb.z, t), n = __builtin_amdgcn_readlane(hb.w, t);
+            const int first = __builtin_amdgcn_readlane(hb.z, t), nm = __builtin_amdgcn_readlane(hb.w, t);
+            const int n = nm & 0xFFFF, inv = nm >> 16;   // inv: ceil(4096 / spheres of B), exact below 256
+            const int nb = __builtin_amdgcn_readlane(hb.x, t) >> 16, ab = __builtin_amdgcn_readlane(hb.y, t);
             const bool on = ((mine >> t) & 1u) != 0u && !hit;
             for (int k0 = 0; k0 < n; k0 += kSelfGroup) {
-                const int k = k0 + sub;
-                if (!on || k >= n) continue;
-                const unsigned pr = R.cpl[first + k];
+                // (branch-free up to the rare pair that counts: lanes without
+                // one take the block's last pair along)
+                const int k = min(k0 + sub, n - 1);
+                const bool valid = on && k0 + sub < n;
+                unsigned pr;
+                if (nb) {
+                    const int i = (k * inv) >> 12;
+                    pr = (unsigned)(ab + i + ((k - i * nb) << 16));
+                } else {
+                    pr = R.cpl[first + k];
+                }
                 const float4 u = pos[pr & 0xFFFFu], v = pos[pr >> 16];
                 const float ux = u.x - v.x, uy = u.y - v.y, uz = u.z - v.z;
                 const float e2 = fmaf(uz, uz, fmaf(uy, uy, ux * ux));
-                if (a.mode == 0) {
-                    const float r2 = u.w + v.w;
-                    if (e2 - r2 * r2 < 0.0f) hit = true;
+                const float rs = u.w + v.w;
+                if (MODE == 0) {
+                    hit = hit || (valid && e2 - rs * rs < 0.0f);
                 } else {
-                    const float cl = sqrtf(e2) - (u.w + v.w);
-                    const int key = (b << 16) | k;
-                    if (cl < best || (cl == best && key < bkey)) {
-                        best = cl;
-                        bkey = key;
+                    // only a pair below the band and no farther than the best
+                    // so far counts: the others are told without the root
+                    // (with room for its rounding)
+                    const float lim = fmaxf(fminf(best, band) + rs, 0.0f);
+                    if (valid && e2 <= fmaf(lim * lim, 1.00001f, 1e-12f)) {
+                        const float cl = sqrtf(e2) - rs;
+                        const int key = (b << 16) | k;
+                        if (cl < best || (cl == best && key < bkey)) {
+                            best = cl;
+                            bkey = key;
+                        }
                     }
                 }
             }
-            if (a.mode == 0) {
+            if (MODE == 0) {
                 // share the state's verdict so its lanes stop
                 hit = ((__ballot(hit) >> (st * kSelfGroup)) & 0xFFFFull) != 0ull;
             }
         }
-        if (a.mode == 0 && __ballot(live && !hit) == 0ull) break;
+        if (MODE == 0 && __ballot(live && !hit) == 0ull) break;
     }
-    if (a.mode == 0) {
+    if (MODE == 0) {
         if (active && sub == 0) {
             if (a.unit_first_hit) {
                 if (hit) atomicMin((unsigned*)&a.unit_first_hit[unit], (unsigned)kstate);
@@ -2199,6 +2255,8 @@ __device__ __forceinline__ bool unit_settled(const SelfArgs& a, const StateRef& 
     return a.X.source == kSrcEdge ? (unsigned)fh <= (unsigned)ref.k : fh >= 0;
 }
 
+// GATED: mode 0 of a model whose exact pairs do not decide alone.
+template <int MODE, bool GATED>
 __global__ __launch_bounds__(64, 4) void k_self(SelfArgs a) {
     extern __shared__ float4 s_dyn4[];
     const DRobot& R = a.R;
@@ -2211,19 +2269,24 @@ __global__ __launch_bounds__(64, 4) void k_self(SelfArgs a) {
     float* s_q = reinterpret_cast<float*>(reinterpret_cast<char*>(s_dyn4) + SelfLds::bytes(S, R.n_clu, J));   // [kMaxDof][kSelfStates]
     int* s_end = reinterpret_cast<int*>(s_q + kMaxDof * kSelfStates); // [2][64] unit ends / starts of a chunk
     float4* s_apos = reinterpret_cast<float4*>(s_end + 2 * kWave);    // gated mode 0: [kSelfStates][A] approx spheres
-    const bool gated = a.mode == 0 && !R.self_gate_implied;
     const long n_states = state_count(a.X);
     // With the plan's chunk table a chunk names its first unit (staged unit
     // ends make the state -> unit lookup an LDS bisection) or, waypoint-major,
     // its problem; without it states go in flat order.
     const bool chunked = a.C.tab != nullptr;
     const long n_work = chunked ? (long)a.C.n_chunks : (n_states + kSelfStates - 1) / kSelfStates;
+    // the lane's joint once per wave, the next chunk's table entry a round ahead
+    JointRegs jt;
+    jt.load(R, sub);
+    int4 chn = make_int4(0, 0, 0, 0);
+    if (chunked && (long)blockIdx.x < n_work) chn = a.C.tab[blockIdx.x];
     for (long w = blockIdx.x; w < n_work; w += gridDim.x) {
     long base, g;
     bool active;
     int u0 = -1, prob = 0;
     if (chunked) {
-        const int4 ch = a.C.tab[w];
+        const int4 ch = chn;
+        if (w + gridDim.x < n_work) chn = a.C.tab[w + gridDim.x];
         base = ch.y;
         g = base + st;
         active = g < ch.z;
@@ -2258,17 +2321,19 @@ __global__ __launch_bounds__(64, 4) void k_self(SelfArgs a) {
     }
     __syncthreads();
     float* Ts = L.T + st * fstride;
-    group_frames(R, s_q + st, kSelfStates, Ts, L.par + st * J, sub);
+    group_frames(jt, J, s_q + st, kSelfStates, Ts, L.par + st * J, sub);
     self_place(R, L, st, sub);
     __syncthreads();
     bool live = active;   // states whose pairs are checked (gated: an approximate pair collides)
-    if (gated) {
+    if (GATED) {
         // Approximate pairs first (two_phase_cc.cuh:114-131): a state none of
         // whose approximate pairs collide has no self collision. Their frames
         // come from the approximate chain when the model has its own (the
         // exact positions above no longer need the full chain's).
         if (R.aft) {
-            group_frames<true>(R, s_q + st, kSelfStates, Ts, L.par + st * J, sub);
+            JointRegs ja;
+            ja.load<true>(R, sub);
+            group_frames(ja, J, s_q + st, kSelfStates, Ts, L.par + st * J, sub);
         }
         float4* apos = s_apos + st * R.n_apx;
         for (int k = sub; k < R.n_apx; k += kSelfGroup) {
@@ -2290,7 +2355,7 @@ __global__ __launch_bounds__(64, 4) void k_self(SelfArgs a) {
         }
         live = live && ((__ballot(ah) >> (st * kSelfGroup)) & 0xFFFFull) != 0ull;
     }
-    self_pairs(a, L, st, sub, active, live, ref.gs, ref.unit, ref.k);
+    self_pairs<MODE>(a, L, st, sub, active, live, ref.gs, ref.unit, ref.k);
     __syncthreads();   // positions of this round are dead before the next load
     }
 }
@@ -2557,10 +2622,12 @@ __global__ __launch_bounds__(64, 4) void k_self_far(SelfArgs a) {
             const bool on = i0 + st < n_open;
             const int col = s_list[on ? i0 + st : i0];
             const int4 rf = s_ref[col];
-            group_frames(R, s_q + col, kN, L.T + st * (J * 12 + 4), L.par + st * J, sub16);
+            JointRegs jt;
+            jt.load(R, sub16);
+            group_frames(jt, J, s_q + col, kN, L.T + st * (J * 12 + 4), L.par + st * J, sub16);
             self_place(R, L, st, sub16);
             __syncthreads();
-            self_pairs(a, L, st, sub16, on, on, rf.x, rf.y, rf.z);
+            self_pairs<0>(a, L, st, sub16, on, on, rf.x, rf.y, rf.z);
         }
     }
 }
@@ -2607,6 +2674,8 @@ __global__ __launch_bounds__(64) void k_fk_out(DRobot R, DStates X, float* frame
             o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
         }
     };
+    JointRegs jt;
+    jt.load(R, sub);
     float qn = fetch(base);
     // 4 J <= 64: lane i's frame column, lane & 3, of joint position fj
     int fj = 0;
@@ -2623,7 +2692,7 @@ __global__ __launch_bounds__(64) void k_fk_out(DRobot R, DStates X, float* frame
         if (lane < kGrpStates * D) s_q[lane] = qn;
         qn = fetch(base + step);
         __syncthreads();
-        group_frames(R, s_q + slot * D, 1, s_T + slot * fstride, s_par + slot * J, sub);
+        group_frames(jt, J, s_q + slot * D, 1, s_T + slot * fstride, s_par + slot * J, sub);
         for (int g = 0; g < m; ++g) {
             const float* Tg = s_T + g * fstride;
             if (frames && lane < 4 * J) {
@@ -3525,8 +3594,12 @@ hipError_t launch_self(const SelfArgs& a, hipStream_t s) {
     const bool gate = a.mode == 0 && !a.R.self_gate_implied;   // approximate pair positions
     const size_t smem = SelfLds::bytes(a.R.n_sph, a.R.n_clu, a.R.n_joints) + sizeof(float) * (size_t)kMaxDof * kSelfStates +
                         sizeof(int) * 2 * kWave + (gate ? sizeof(float4) * (size_t)kSelfStates * a.R.n_apx : 0);
-    hipLaunchKernelGGL(k_self, dim3((unsigned)blocks), dim3(64), smem, s, a);
-    return hipGetLastError();
+    // one chunk a wave: chunks differ in cost, and the dispatcher evens them out
+    // (STOMP's rollouts: 718 us a call, 731 with four times the waves the chip
+    // holds, 881 with as many)
+    const void* k = a.mode != 0 ? (const void*)k_self<1, false> : gate ? (const void*)k_self<0, true> : (const void*)k_self<0, false>;
+    SelfArgs arg = a;
+    return launch_args(k, (int)blocks, smem, s, &arg, nullptr, nullptr);
 }
 
 hipError_t launch_fk_out(const DRobot& R, const DStates& X, float* frames, float* spheres, hipStream_t s) {

@@ -55,6 +55,10 @@ struct DRobot {
     const int4* cpb;            // [n_cpb] self-pair blocks: (cluster A, cluster B, first pair, pairs), A <= B
     const unsigned* cpl;        // [n_pairs] block pair lists: slot a | slot b << 16 (emission slots)
     int n_cpb;
+    // the same blocks as the pair walk reads them: (A | B << 8 | nb << 16, a0 | b0 << 16, first pair, pairs | inv << 16),
+    // a0, b0 the clusters' first slots, nb B's spheres when the block holds every pair in order, else 0,
+    // inv = ceil(4096 / nb)
+    const int4* cpx;
     // The self pass's rough tests (NULL: the model's transforms are not rigid
     // enough for them), one entry per block of cpb, its smaller cluster as B:
     // (slot a0 | spheres << 16, slot b0 | spheres << 16, joint a | joint b << 16,
