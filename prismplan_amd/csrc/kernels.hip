@@ -735,14 +735,20 @@ __device__ __forceinline__ float wave_max(float v) {
 // Maximum over the 16 lanes of a row (lanes 16 k .. 16 k + 15), by row rotations.
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
-    const int i = __float_as_int(v);
-    return __int_as_float(__builtin_amdgcn_update_dpp(i, i, CTRL, 0xf, 0xf, false));
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
 }
 __device__ __forceinline__ float row_max(float v) {
     v = fmaxf(v, dpp<0x128>(v));
     v = fmaxf(v, dpp<0x124>(v));
     v = fmaxf(v, dpp<0x122>(v));
     return fmaxf(v, dpp<0x121>(v));
+}
+
+__device__ __forceinline__ float row_sum(float v) {
+    v += dpp<0x128>(v);
+    v += dpp<0x124>(v);
+    v += dpp<0x122>(v);
+    return v + dpp<0x121>(v);
 }
 
 // A row's 16 bits of a ballot (row: its first lane).
@@ -1160,39 +1166,37 @@ __global__ __launch_bounds__(64) void k_collide_gated(CollideArgs a) {
 // of the OBBs some active lane's spheres of the cluster can come within the
 // hinge band of. Every sphere s of the cluster lies inside its enclosing
 // sphere `as` (centre a, radius R; DRobot::clu_enc), so clr(s, o) >=
-// sdf_o(a) - R; the active lanes' centres lie within rw of the first active
-// lane's centre c0, so sdf_o(a) >= sdf_o(c0) - rw. An OBB with sdf_o(c0) >=
-// band + R + rw therefore has clearance >= band from every sphere: it cannot
-// change a hinge, its argmin or its gradient. One pass per 64 OBBs (lane i
-// tests OBB base + i).
+// sdf_o(a) - R; the active lanes' centres lie within rw of c0, about their
+// mean (of those at finite places; the others make rw large instead), so
+// sdf_o(a) >= sdf_o(c0) - rw. An OBB with sdf_o(c0) >= band + R + rw therefore
+// has clearance >= band from every sphere: it cannot change a hinge, its argmin
+// or its gradient. One pass per 64 OBBs (lane i tests OBB base + i).
+template <int STRIDE>
 __device__ __forceinline__ void near_obbs(const float4* __restrict__ s_obb, int n_obb, const float* T, const float4& as,
-                                          float band, bool active, ObbMask& mk) {
+                                          float band, bool active, unsigned long long* w) {
     float ax, ay, az;
     aff_point(T, as.x, as.y, as.z, ax, ay, az);
-    const int l0 = __ffsll(__ballot(active)) - 1;
-    if (l0 < 0) {
-#pragma unroll
-        for (int k = 0; k < kMaskWords; ++k) mk.w[k] = 0ull;
-        return;
-    }
-    const float cx = read_lane(ax, l0), cy = read_lane(ay, l0), cz = read_lane(az, l0);
+    auto wave = [](float v) {   // a row's value in each of its lanes -> the four rows'
+        return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
+    };
+    const bool in = active && fabsf(ax) + fabsf(ay) + fabsf(az) < 1e4f;
+    const float inv_n = __builtin_amdgcn_rcpf((float)__popcll(__ballot(in)));
+    const float cx = wave(row_sum(in ? ax : 0.0f)) * inv_n, cy = wave(row_sum(in ? ay : 0.0f)) * inv_n,
+                cz = wave(row_sum(in ? az : 0.0f)) * inv_n;
     const float dx = ax - cx, dy = ay - cy, dz = az - cz;
-    const float d2 = wave_max(active ? fmaf(dz, dz, fmaf(dy, dy, dx * dx)) : 0.0f);
+    const float v = row_max(active ? fmaf(dz, dz, fmaf(dy, dy, dx * dx)) : 0.0f);
+    const float d2 = fmaxf(fmaxf(read_lane(v, 0), read_lane(v, 16)), fmaxf(read_lane(v, 32), read_lane(v, 48)));
     // sdf(c0) < reach  <=>  key(c0) < reach * |reach|; slack covers rounding
-    const float reach = band + as.w + sqrtf(d2) * 1.0001f + 1e-5f;
-    const float thr = uniform(reach * fabsf(reach));
+    const float reach = band + as.w + __builtin_amdgcn_sqrtf(d2) * 1.0001f + 1e-5f;
+    const float thr = reach * fabsf(reach);
 #pragma unroll
     for (int k = 0; k < kMaskWords; ++k) {
-        bool c = false;
-        if (k * 64 < n_obb) {
-            const int o = k * 64 + lane_id();
-            if (o < n_obb) {
-                float lx, ly, lz;
-                to_box(s_obb[4 * o], s_obb[4 * o + 1], s_obb[4 * o + 2], cx, cy, cz, lx, ly, lz);
-                c = box_key(lx, ly, lz, s_obb[4 * o + 3]) < thr;
-            }
-        }
-        mk.w[k] = __ballot(c);
+        if (k * 64 >= n_obb) break;
+        // past the last OBB: its record again, masked off
+        const int o = min(k * 64 + lane_id(), n_obb - 1);
+        float lx, ly, lz;
+        to_box(s_obb[STRIDE * o], s_obb[STRIDE * o + 1], s_obb[STRIDE * o + 2], cx, cy, cz, lx, ly, lz);
+        w[k] = __ballot(k * 64 + lane_id() < n_obb && box_key(lx, ly, lz, s_obb[STRIDE * o + 3]) < thr);
     }
 }
 
@@ -1200,10 +1204,6 @@ __device__ __forceinline__ void near_obbs(const float4* __restrict__ s_obb, int 
 // OBB (LDS record index; -1 when there is none). Ties keep the lowest index.
 // A (sphere, OBB) pair the scene's ACM masks out is skipped
 // (collision/scene_collision.cuh:140-167: sphere_obb_clearance by sphere index).
-// PAIR: two candidates per step, both records read before either test, so
-// one record's LDS latency hides the other's (the cost-only kernel has the
-// registers for it; the adjoint instantiation would spill).
-template <bool PAIR>
 __device__ __forceinline__ void obb_argmin(const float4* __restrict__ s_obb, const ObbMask& mk, float px, float py,
                                            float pz, const uint8_t* __restrict__ acm_row, float& best, int& arg) {
     best = FLT_MAX;
@@ -1211,37 +1211,14 @@ __device__ __forceinline__ void obb_argmin(const float4* __restrict__ s_obb, con
 #pragma unroll
     for (int k = 0; k < kMaskWords; ++k) {
         unsigned long long bits = mk.w[k];
-        if (PAIR) {
-            while (bits) {
-                const int oa = k * 64 + (__ffsll(bits) - 1);
-                bits &= bits - 1ull;
-                const bool two = bits != 0ull;
-                const int ob = two ? k * 64 + (__ffsll(bits) - 1) : oa;
-                if (two) bits &= bits - 1ull;
-                const float4 a0 = s_obb[4 * oa], a1 = s_obb[4 * oa + 1], a2 = s_obb[4 * oa + 2], ah = s_obb[4 * oa + 3];
-                const float4 b0 = s_obb[4 * ob], b1 = s_obb[4 * ob + 1], b2 = s_obb[4 * ob + 2], bh = s_obb[4 * ob + 3];
-                float lx, ly, lz;
-                to_box(a0, a1, a2, px, py, pz, lx, ly, lz);
-                float ka = box_key(lx, ly, lz, ah);
-                to_box(b0, b1, b2, px, py, pz, lx, ly, lz);
-                float kb = box_key(lx, ly, lz, bh);
-                if (acm_row) {
-                    if (acm_row[__float_as_int(ah.w)] == 0) ka = FLT_MAX;
-                    if (acm_row[__float_as_int(bh.w)] == 0) kb = FLT_MAX;
-                }
-                if (ka < best) { best = ka; arg = oa; }   // oa < ob: ties keep the lower index
-                if (two && kb < best) { best = kb; arg = ob; }
-            }
-        } else {
-            while (bits) {
-                const int o = k * 64 + (__ffsll(bits) - 1);
-                bits &= bits - 1ull;
-                if (acm_row && acm_row[__float_as_int(s_obb[4 * o + 3].w)] == 0) continue;
-                float lx, ly, lz;
-                to_box(s_obb[4 * o], s_obb[4 * o + 1], s_obb[4 * o + 2], px, py, pz, lx, ly, lz);
-                const float key = box_key(lx, ly, lz, s_obb[4 * o + 3]);
-                if (key < best) { best = key; arg = o; }
-            }
+        while (bits) {
+            const int o = k * 64 + (__ffsll(bits) - 1);
+            bits &= bits - 1ull;
+            if (acm_row && acm_row[__float_as_int(s_obb[4 * o + 3].w)] == 0) continue;
+            float lx, ly, lz;
+            to_box(s_obb[4 * o], s_obb[4 * o + 1], s_obb[4 * o + 2], px, py, pz, lx, ly, lz);
+            const float key = box_key(lx, ly, lz, s_obb[4 * o + 3]);
+            if (key < best) { best = key; arg = o; }
         }
     }
 }
@@ -1303,8 +1280,11 @@ __device__ __forceinline__ float group_sum(float v, int G) {
     return v;
 }
 
-template <bool GRAD>
-__global__ __launch_bounds__(64, 4) void k_cost(CostArgs a) {
+// Spheres of a lane that k_state_cost takes through the boxes together.
+constexpr int kSphRun = 4;
+
+// Cost and adjoint, G lanes per state, joint by joint.
+__global__ __launch_bounds__(64, 4) void k_cost_grad(CostArgs a) {
     extern __shared__ float4 s_lds[];
     float4* s_obb = s_lds;
     float* s_q = reinterpret_cast<float*>(s_lds + 4 * a.C.obb_cap);
@@ -1314,7 +1294,7 @@ __global__ __launch_bounds__(64, 4) void k_cost(CostArgs a) {
     const int sub = lane & (G - 1);
     const int slot = lane / G;                // state slot of this lane group
     const int J = R.n_joints, D = R.n_dof;
-    // Adjoint records (GRAD): per state slot and joint, the joint origin o,
+    // Adjoint records: per state slot and joint, the joint origin o,
     // axis z, and the force f / moment tau (about o) of its own spheres'
     // hinge gradients; then d cost / d q per dof.
     int* s_end = reinterpret_cast<int*>(s_q + D * kWave);
@@ -1358,12 +1338,14 @@ __global__ __launch_bounds__(64, 4) void k_cost(CostArgs a) {
             int4 meta;
             fk_joint(R, jj, s_q + lane, sl, T, meta);
             float fx = 0.0f, fy = 0.0f, fz = 0.0f, tx = 0.0f, ty = 0.0f, tz = 0.0f;
-            const int s0 = R.sph_off[jj], s1 = R.sph_off[jj + 1];
+            const bool any = uload<int>(R.sph_off, jj + 1) > uload<int>(R.sph_off, jj);
+            const int c1 = any ? uload<int>(R.clu_off, jj + 1) : 0;
             // one candidate mask per sphere cluster of the joint
-            for (int c = (s1 > s0 ? R.clu_off[jj] : 0); c < (s1 > s0 ? R.clu_off[jj + 1] : 0); ++c) {
-                ObbMask mk;
-                if (use_obb) near_obbs(s_obb, n_obb, T, R.clu_enc[c], a.P.world_margin, active, mk);
-                for (int s = R.clu_beg[c] + sub; s < R.clu_beg[c + 1]; s += G) {
+            for (int c = any ? uload<int>(R.clu_off, jj) : 0; c < c1; ++c) {
+                ObbMask mk{};
+                if (use_obb) near_obbs<4>(s_obb, n_obb, T, uload4(R.clu_enc, c), a.P.world_margin, active, mk.w);
+                const int b1 = uload<int>(R.clu_beg, c + 1);
+                for (int s = uload<int>(R.clu_beg, c) + sub; s < b1; s += G) {
                     const float4 sp = R.sph[s];
                     float px, py, pz;
                     aff_point(T, sp.x, sp.y, sp.z, px, py, pz);
@@ -1371,47 +1353,43 @@ __global__ __launch_bounds__(64, 4) void k_cost(CostArgs a) {
                     int arg = -1;
                     const uint8_t* acm_row =
                         a.S.sphere_obb_acm ? a.S.sphere_obb_acm + (size_t)R.sph_id[s] * a.S.n_obbs : nullptr;
-                    if (use_obb) obb_argmin<!GRAD>(s_obb, mk, px, py, pz, acm_row, best, arg);
+                    if (use_obb) obb_argmin(s_obb, mk, px, py, pz, acm_row, best, arg);
                     float gx, gy, gz;
                     auto rec = [&](float4& r0, float4& r1, float4& r2, float4& r3) {
                         r0 = s_obb[4 * arg]; r1 = s_obb[4 * arg + 1]; r2 = s_obb[4 * arg + 2]; r3 = s_obb[4 * arg + 3];
                     };
-                    const float hs = sphere_hinge_at<GRAD, false>(a, EsdfLayer(), arg >= 0, rec, best, px, py, pz, sp.w, R.sph_id[s],
+                    const float hs = sphere_hinge_at<true, false>(a, EsdfLayer(), arg >= 0, rec, best, px, py, pz, sp.w, R.sph_id[s],
                                                            use_obb, use_esdf, gx, gy, gz);
                     world += hs;
-                    if (GRAD) {
-                        if (si >= 0) {
-                            const int id = R.sph_id[s];
-                            if (id == si) { gx -= snx; gy -= sny; gz -= snz; }
-                            if (id == sj) { gx += snx; gy += sny; gz += snz; }
-                        }
-                        // wrench about the joint origin: f += g, tau += (p - o) x g
-                        const float rx = px - T[3], ry = py - T[7], rz = pz - T[11];
-                        fx += gx; fy += gy; fz += gz;
-                        tx = fmaf(ry, gz, fmaf(-rz, gy, tx));
-                        ty = fmaf(rz, gx, fmaf(-rx, gz, ty));
-                        tz = fmaf(rx, gy, fmaf(-ry, gx, tz));
+                    if (si >= 0) {
+                        const int id = R.sph_id[s];
+                        if (id == si) { gx -= snx; gy -= sny; gz -= snz; }
+                        if (id == sj) { gx += snx; gy += sny; gz += snz; }
                     }
+                    // wrench about the joint origin: f += g, tau += (p - o) x g
+                    const float rx = px - T[3], ry = py - T[7], rz = pz - T[11];
+                    fx += gx; fy += gy; fz += gz;
+                    tx = fmaf(ry, gz, fmaf(-rz, gy, tx));
+                    ty = fmaf(rz, gx, fmaf(-rx, gz, ty));
+                    tz = fmaf(rx, gy, fmaf(-ry, gx, tz));
                 }
             }
-            if (GRAD) {
-                const bool nz = fx != 0.0f || fy != 0.0f || fz != 0.0f || tx != 0.0f || ty != 0.0f || tz != 0.0f;
-                if (G > 1 && wave_any(nz)) {
-                    fx = group_sum(fx, G); fy = group_sum(fy, G); fz = group_sum(fz, G);
-                    tx = group_sum(tx, G); ty = group_sum(ty, G); tz = group_sum(tz, G);
-                }
-                if (sub == 0) {
-                    const int type = meta.x;
-                    const int ax = type >= kXRot ? type - kXRot : (type >= 0 ? type : 0);
-                    float* r = rec + 12 * jj;
-                    r[0] = T[3]; r[1] = T[7]; r[2] = T[11];
-                    r[3] = T[ax]; r[4] = T[4 + ax]; r[5] = T[8 + ax];
-                    r[6] = fx; r[7] = fy; r[8] = fz;
-                    r[9] = tx; r[10] = ty; r[11] = tz;
-                }
+            const bool nz = fx != 0.0f || fy != 0.0f || fz != 0.0f || tx != 0.0f || ty != 0.0f || tz != 0.0f;
+            if (G > 1 && wave_any(nz)) {
+                fx = group_sum(fx, G); fy = group_sum(fy, G); fz = group_sum(fz, G);
+                tx = group_sum(tx, G); ty = group_sum(ty, G); tz = group_sum(tz, G);
+            }
+            if (sub == 0) {
+                const int type = meta.x;
+                const int ax = type >= kXRot ? type - kXRot : (type >= 0 ? type : 0);
+                float* r = rec + 12 * jj;
+                r[0] = T[3]; r[1] = T[7]; r[2] = T[11];
+                r[3] = T[ax]; r[4] = T[4 + ax]; r[5] = T[8 + ax];
+                r[6] = fx; r[7] = fy; r[8] = fz;
+                r[9] = tx; r[10] = ty; r[11] = tz;
             }
         }
-        if (GRAD && sub == 0 && active) {
+        if (sub == 0 && active) {
             // Reverse DFS sweep: every joint's subtree wrench is complete once
             // its descendants (higher DFS positions) have been folded in.
             for (int d = 0; d < D; ++d) dqs[d] = 0.0f;
@@ -1448,6 +1426,136 @@ __global__ __launch_bounds__(64, 4) void k_cost(CostArgs a) {
     }
 }
 
+// The cost alone: as above, but a cluster's spheres meet a candidate box
+// together, up to four of a lane at a time, so a record is read once for all of
+// them and their tests do not wait for one another; the bound on the cluster is
+// taken around the mean of the wave's centres. A cluster that no box comes near
+// adds nothing and is left; so is the exact distance of a sphere that no lane
+// has within the hinge band. Bound by VALU issue (16,000 instructions a wave of
+// 64 states), at 64 % of it; a wave takes long enough that the last ones of a
+// launch show. 325,152 Fetch rollout states, 30 to 80 boxes a problem: 396 us
+// -> 210 with one kernel for cost and adjoint before, box by box for each
+// sphere; 239 around the first lane's centre; runs of 4, 3 and 2 spheres 211,
+// 213 and 220; at the waves that the chip holds at once 268.
+template <bool ESDF, bool LINE>
+__global__ __launch_bounds__(64, 4) void k_state_cost(CostArgs a) {
+    extern __shared__ float4 s_lds[];
+    float4* s_obb = s_lds;
+    float* s_q = reinterpret_cast<float*>(s_lds + kObbRec * a.C.obb_cap);
+    const DRobot& R = a.R;
+    const int lane = lane_id();
+    const int G = a.group, sub = lane & (G - 1), slot = lane / G;
+    const int lg = __ffs(G) - 1;
+    const int J = R.n_joints, D = R.n_dof;
+    int* s_end = reinterpret_cast<int*>(s_q + D * kWave);
+    const bool use_obb = a.P.use_obb != 0;
+    const bool use_esdf = ESDF && a.P.use_esdf != 0;
+    const float wt = a.P.weight, m = a.P.world_margin;
+    const bool quiet = m <= 1000.0f;   // no box near (clearance 1000): no hinge
+    const uint8_t* acm = a.S.sphere_obb_acm;
+    int cur_prob = -1, n_obb = 0;
+    int4 ch;
+    ChunkCursor cur = chunk_cursor();
+    const long n_states = state_count(a.X);
+    const int n_chunks = chunk_count(a.C, n_states);
+    while (next_chunk(a.C, n_states, n_chunks, cur, ch)) {
+        if (ch.x != cur_prob) {
+            int o0, o1;
+            problem_obbs(a.C, a.S, ch.x, o0, o1);
+            __syncthreads();
+            n_obb = uniform(stage_obbs<kObbRec>(a.S, o0, o1, s_obb, a.C.obb_cap));
+            cur_prob = ch.x;
+        }
+        const long g = (long)ch.y + slot;
+        const bool active = g < ch.z;
+        stage_unit_ends(a.X, ch.w, s_end);
+        __syncthreads();
+        StateRef ref = load_state(a.X, D, g, active, s_q, ch.w, s_end, ch.x);
+        __syncthreads();
+        const float self_h =
+            a.self_in && active ? fmaxf(a.P.self_margin - a.self_in[8 * (size_t)ref.gs], 0.0f) : 0.0f;
+        float world = 0.0f;
+        FkWalk<LINE> fk;
+        float T[12];
+        for (int jj = 0; jj < J; ++jj) {
+            int4 meta;
+            fk.step(R, jj, s_q + lane, T, meta);
+            if (uload<int>(R.sph_off, jj) == uload<int>(R.sph_off, jj + 1)) continue;
+            const int c1 = uload<int>(R.clu_off, jj + 1);
+            for (int c = uload<int>(R.clu_off, jj); c < c1; ++c) {
+                unsigned long long w[kMaskWords] = {};
+                if (use_obb) near_obbs<kObbRec>(s_obb, n_obb, T, uload4(R.clu_enc, c), m, active, w);
+                if (!use_esdf && quiet && (w[0] | w[1] | w[2] | w[3]) == 0ull) continue;
+                const int b1 = uload<int>(R.clu_beg, c + 1);
+                for (int b = uload<int>(R.clu_beg, c); b < b1; b += kSphRun * G) {
+                    const int n = min(kSphRun, (b1 - b + G - 1) >> lg);   // rounds of this run
+                    float4 p[kSphRun];
+                    float best[kSphRun];
+                    int id[kSphRun];   // for the ACM
+#pragma unroll
+                    for (int k = 0; k < kSphRun; ++k) {
+                        // past the cluster's end: its last sphere again
+                        const int s = min(b + k * G + sub, b1 - 1);
+                        const float4 sp = G == 1 ? uload4(R.sph, min(b + k, b1 - 1)) : R.sph[s];
+                        aff_point(T, sp.x, sp.y, sp.z, p[k].x, p[k].y, p[k].z);
+                        p[k].w = sp.w;
+                        best[k] = FLT_MAX;
+                        id[k] = acm ? R.sph_id[s] : 0;
+                    }
+                    unsigned long long v[kMaskWords];
+#pragma unroll
+                    for (int k = 0; k < kMaskWords; ++k) v[k] = w[k];
+                    for (int o0 = 0; o0 < n_obb; o0 += 64) {
+                        while (v[0]) {
+                            const int o = o0 + __ffsll(v[0]) - 1;
+                            v[0] &= v[0] - 1ull;
+                            const float4 r0 = s_obb[kObbRec * o], r1 = s_obb[kObbRec * o + 1],
+                                         r2 = s_obb[kObbRec * o + 2], h = s_obb[kObbRec * o + 3];
+#pragma unroll
+                            for (int k = 0; k < kSphRun; ++k) {
+                                if (k >= n) break;
+                                float lx, ly, lz;
+                                to_box(r0, r1, r2, p[k].x, p[k].y, p[k].z, lx, ly, lz);
+                                float key = box_key(lx, ly, lz, h);
+                                if (acm && acm[(size_t)id[k] * a.S.n_obbs + __float_as_int(h.w)] == 0) key = FLT_MAX;
+                                best[k] = fminf(best[k], key);
+                            }
+                        }
+#pragma unroll
+                        for (int k = 0; k + 1 < kMaskWords; ++k) v[k] = v[k + 1];
+                    }
+#pragma unroll
+                    for (int k = 0; k < kSphRun; ++k) {
+                        if (k >= n) break;
+                        const int s = b + k * G + sub;
+                        const float r = p[k].w;
+                        float hs = 0.0f;
+                        if (use_obb) {
+                            // sdf < m + r <=> key < (m + r) |m + r|; slack covers rounding
+                            const float reach = fmaf(fabsf(m) + fabsf(r), 1e-5f, m + r) + 1e-6f;
+                            if (!quiet || wave_any(best[k] < reach * fabsf(reach))) {
+                                const float clr = best[k] < FLT_MAX ? key_to_sdf(best[k]) - r : 1000.0f;
+                                const float hh = m - clr;
+                                if (hh > 0.0f) hs += hh;
+                            }
+                        }
+                        if (ESDF && use_esdf) {
+                            float gx, gy, gz;
+                            const float hh = m - esdf_clearance(a.S, p[k].x, p[k].y, p[k].z, r,
+                                                                R.sph_id[min(s, b1 - 1)], false, gx, gy, gz);
+                            if (hh > 0.0f) hs += hh;
+                        }
+                        if (s < b1) world += hs;
+                    }
+                }
+            }
+        }
+        world = group_sum(world, G);
+        if (active && sub == 0 && a.cost_out) a.cost_out[ref.gs] = wt * (world + self_h);
+        __syncthreads();   // the states of this chunk are read
+    }
+}
+
 // ===========================================================================
 // Grouped summed-hinge cost (+ adjoint): one state per aligned group of
 // kGrp = 16 lanes, four states per wave, with the state's spheres spread over
@@ -1469,7 +1577,7 @@ __global__ __launch_bounds__(64, 4) void k_cost(CostArgs a) {
 //     sums each joint's DFS subtree -- a contiguous run of positions -- into a
 //     total wrench about o_jj, and lane jj reads d cost / d q = z . tau
 //     (revolute) or z . f (prismatic).
-// Results equal k_cost's up to FP32 summation order.
+// Results equal k_cost_grad's up to FP32 summation order.
 // ===========================================================================
 // Joint frames of the state of a 16-lane group (one state per group, a
 // 1-wave workgroup), DFS positions 0..J-1, into F (12 floats each, row-major
@@ -3439,6 +3547,7 @@ size_t lds_bytes_collide(int obb_cap, const DRobot& R) {
 
 size_t lds_bytes_cost(int obb_cap, int n_dof, int n_joints, int G, bool grad) {
     size_t b = lds_bytes(obb_cap, n_dof);
+    if (!grad) b += (size_t)obb_cap * 16 * (kObbRec - 4);   // record padding
     if (grad) b += (size_t)(kWave / G) * (rec_stride(n_joints) + dq_stride(n_dof)) * sizeof(float);
     return b;
 }
@@ -3455,16 +3564,15 @@ int grid_collide(const DRobot& R, const DScene& S, int obb_cap) {
     return cache[i].get(collide_kernel(R, S), lds_bytes_collide(obb_cap, R));
 }
 
-int grid_cost(int n_joints, bool grad, size_t lds) {
-    (void)n_joints;
-    static size_t last[2] = {(size_t)-1, (size_t)-1};
-    static int g[2] = {0, 0};
-    const int idx = grad ? 1 : 0;
-    if (lds != last[idx]) {
-        g[idx] = occupancy_grid(grad ? (const void*)k_cost<true> : (const void*)k_cost<false>, lds);
-        last[idx] = lds;
-    }
-    return g[idx];
+static const void* cost_kernel(const DRobot& R, bool esdf, bool grad) {
+    if (grad) return (const void*)k_cost_grad;
+    if (esdf) return R.line ? (const void*)k_state_cost<true, true> : (const void*)k_state_cost<true, false>;
+    return R.line ? (const void*)k_state_cost<false, true> : (const void*)k_state_cost<false, false>;
+}
+
+int grid_cost(const DRobot& R, bool grad, size_t lds) {
+    static GridCache cache[3];
+    return cache[grad ? 2 : R.line ? 1 : 0].get(cost_kernel(R, false, grad), lds);
 }
 
 // A launch with its argument block; with t0/t1 the runtime records the two
@@ -3484,10 +3592,10 @@ hipError_t launch_collide(const CollideArgs& a, int grid, hipStream_t s, hipEven
 }
 
 hipError_t launch_cost(const CostArgs& a, int grid, hipStream_t s, hipEvent_t t0, hipEvent_t t1) {
-    if (a.C.tiled) return hipErrorInvalidValue;   // k_cost stages one OBB tile: tiled problems take k_cost_grp
+    if (a.C.tiled) return hipErrorInvalidValue;   // these kernels stage one OBB tile: tiled problems take k_cost_grp
     const size_t lds = lds_bytes_cost(a.C.obb_cap, a.R.n_dof, a.R.n_joints, a.group, a.grad != 0);
     CostArgs arg = a;
-    const void* k = a.grad ? (const void*)k_cost<true> : (const void*)k_cost<false>;
+    const void* k = cost_kernel(a.R, a.P.use_esdf != 0 && a.S.n_voxel_layers > 0, a.grad != 0);
     return launch_args(k, grid, lds, s, &arg, t0, t1);
 }
 

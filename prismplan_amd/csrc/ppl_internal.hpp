@@ -159,7 +159,7 @@ struct DChunks {
     const int* obb_off;         // [P+1] OBB ranges per problem; NULL = single problem
     int obb_cap;                // OBB records one LDS staging holds (a tile; 1 .. kMaxObbLds)
     int tiled;                  // some problem has more OBBs than obb_cap: they pass through LDS in tiles
-                                // (k_collide, the grouped cost kernel; k_cost refuses such launches)
+                                // (k_collide, the grouped cost kernel; k_cost_grad and k_state_cost refuse such launches)
     const int* unit_hint;       // implicit chunks (tab NULL), nullable: unit holding state 64 k, for each k
     int spread;                 // implicit chunks are visited spread over the whole range, not in order
 };
@@ -301,7 +301,7 @@ __host__ __device__ inline int rec_stride(int n_joints) { return 12 * n_joints +
 __host__ __device__ inline int dq_stride(int n_dof) { return n_dof | 1; }
 int device_cus();
 int grid_collide(const DRobot& R, const DScene& S, int obb_cap);   // workgroups the chip holds at once
-int grid_cost(int n_joints, bool grad, size_t lds);
+int grid_cost(const DRobot& R, bool grad, size_t lds);
 size_t lds_bytes_grp(int obb_cap, int n_dof, int n_joints, int n_sph, int n_clu, bool grad, bool tiled);
 int grid_cost_grp(bool grad, int world, bool tiled, size_t lds);
 int grp_world(const CostArgs& a);

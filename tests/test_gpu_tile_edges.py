@@ -12,6 +12,7 @@ import pytest
 import torch
 
 import pyoracle as PO
+from parity_common import cost_den
 from prismplan_amd import _ppl
 from prismplan_amd import substrate as S
 from prismplan_amd import workloads as W
@@ -167,3 +168,28 @@ def test_rough_self_pass_equals_the_exact_one(robots, margin, skip):
         np.testing.assert_array_equal(hits, np.concatenate([p[2] for p in parts]))
         ref, clr = PO.Oracle(arr).check_collision(PO.edge_states(q, to, ns), check_self=True)
         assert not np.any((hits != ref) & (np.abs(clr) >= 1e-5)) and 0.05 < ref.mean() < 0.5
+
+
+@pytest.mark.parametrize("name,n,boxes,group,margin", [("panda", 1, 1, 16, 0.05), ("fetch", 65, 63, 1, 0.05),
+                                                       ("baxter", 63, 64, 2, 0.05), ("fetch", 33, 65, 4, 0.1),
+                                                       ("branched", 130, 20, 1, 0.05), ("panda", 40, 256, 8, 0.02),
+                                                       ("panda", 70, 40, 1, 1001.0), ("panda", 90, 0, 1, 0.05)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_state_cost_runs(name, n, boxes, group, margin, masked):
+    """State counts around a wave's slots, boxes around a mask word and up to a
+    whole staging, lane groups that leave remainders of a cluster's spheres, a
+    margin past the clearance of an empty world, masked pairs."""
+    from prismplan_amd.planning_scene import HostScene
+    rob = S.Robot(_branched_panda() if name == "branched" else name)
+    arr, rng = rob.arrays, np.random.default_rng(n + boxes)
+    scene = W.random_obbs(rng, boxes, half_hi=0.15) if boxes else HostScene()
+    if masked and boxes:
+        scene.sphere_obb_acm = (rng.random((arr.n_spheres, boxes)) < 0.8).astype(np.uint8)
+    q = W.uniform_configs(rng, arr, n)
+    plan = S.Plan.configs(rob, n)
+    plan.set_cost_group(group)
+    kw = dict(world_margin=margin, weight=2.0, use_self=False, use_esdf=False)
+    st = S.hinge_cost(plan, S.DeviceScene.from_host(scene), torch.from_numpy(q).to(DEV), S.cost_params(**kw))[0]
+    o, prm = PO.Oracle(arr, scene, nthreads=8), PO.cost_params(**kw)
+    ref = o.hinge_cost(q, prm)
+    np.testing.assert_array_less(np.abs(st.cpu().numpy() - ref) / cost_den(ref, 2.0, o.hinge_terms(q, prm)), 1e-5)
