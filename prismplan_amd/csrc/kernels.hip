@@ -1571,13 +1571,23 @@ __global__ __launch_bounds__(64, 4) void k_state_cost(CostArgs a) {
 //     frame and its cluster's mask from LDS,
 //     finds the argmin OBB and the hinge terms. Panda's 59 spheres take four
 //     rounds instead of one round per joint with most lanes idle.
-//  3. Adjoint: every sphere with a non-zero point gradient g adds its force g
-//     and moment (p - o_j) x g about its joint's origin o_j into the joint's
-//     wrench in LDS. A prefix scan over the group's lanes (one joint per lane)
+//  3. Adjoint: every sphere's point gradient g gives a force g and a moment
+//     (p - o_j) x g about its joint's origin o_j. Each round's 16 of them pass
+//     through LDS to the joints' lanes, which add up their own spheres' in
+//     emission order. A prefix scan over the group's lanes (one joint per lane)
 //     sums each joint's DFS subtree -- a contiguous run of positions -- into a
 //     total wrench about o_jj, and lane jj reads d cost / d q = z . tau
 //     (revolute) or z . f (prismatic).
 // Results equal k_cost_grad's up to FP32 summation order.
+// Bound by latency: 16,384 Panda states are 4,096 waves, one round of the chip,
+// each a chain of loads, frames, masks and four sphere rounds, with VALU issue
+// at 0.45. 256 trajectories of 64 waypoints among 40 boxes: 45.5 us -> 31.7, of
+// which 6 by the masks' reach about the states' mean instead of the first
+// state's place (fewer candidates) with the reaches computed a lane each, and by
+// loads that start together, and 8 by the wrenches: six LDS atomics a sphere, up
+// to sixteen to one address, kept the CU's LDS unit busy. The same in CHOMP's
+// iterations 60 -> 48, and over an ESDF (71,000 Baxter states) 82 -> 78; there
+// VALU issue is at 0.62.
 // ===========================================================================
 // Joint frames of the state of a 16-lane group (one state per group, a
 // 1-wave workgroup), DFS positions 0..J-1, into F (12 floats each, row-major
@@ -1689,10 +1699,14 @@ __device__ __forceinline__ void group_frames(const JointRegs& jt, int J, const f
 
 static_assert(kGrp >= kMaxJoints, "the grouped kernel gives every joint its own lane of the group");
 
+// Floats of a state's 16 sphere wrenches of one round (6 each; the four states'
+// start in different LDS banks).
+constexpr int kGrpWrench = kGrp * 6 + 4;
+
 size_t lds_floats_grp(int obb_cap, int n_dof, int n_joints, int n_sph, int n_clu, bool grad, bool tiled) {
     size_t f = (size_t)obb_cap * 16 + (size_t)n_clu * kMaskWords * 2 +
                (((size_t)n_dof * kGrpStates + 3) & ~(size_t)3) + 2 * kWave + (size_t)kGrpStates * (n_joints * 13 + 4);
-    if (grad) f += (size_t)kGrpStates * ((size_t)n_joints * 6 + kMaxDof + 1);
+    if (grad) f += (size_t)kGrpStates * (kGrpWrench + kMaxDof + 1);
     if (tiled) f += (size_t)kGrpStates * n_sph * 2;
     return f;
 }
@@ -1700,71 +1714,67 @@ size_t lds_floats_grp(int obb_cap, int n_dof, int n_joints, int n_sph, int n_clu
 // Candidate masks of every sphere cluster of the wave's four states over the
 // staged OBBs (the broad phase of near_obbs, all clusters' enclosing spheres
 // placed at once, 16 clusters per pass): lane k of each group places cluster
-// c0 + k's enclosing sphere; the four states' spread about state slot 0's
-// centre sets the cluster's reach; one pass of 64 lanes over the OBBs per
-// cluster gives its mask.
+// c0 + k's enclosing sphere; the four states' spread about their mean sets the
+// cluster's reach; one pass of 64 lanes over the OBBs per cluster gives its
+// mask (words past the staged OBBs are neither written nor read).
 __device__ __forceinline__ void grp_masks(const DRobot& R, const float4* __restrict__ s_obb, int n_obb, const float* Ts,
                                           float band, bool active, int sub, unsigned long long* s_mask) {
     const int C = R.n_clu, lane = lane_id();
+    auto slots = [](float v) {   // sum over the four states
+        v += __shfl_xor(v, 16);
+        return v + __shfl_xor(v, 32);
+    };
     for (int c0 = 0; c0 < C; c0 += kGrp) {
         const int cl = c0 + sub;
+        float4 ce = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         float ax = 0.0f, ay = 0.0f, az = 0.0f;
         if (cl < C && active) {
-            const float4 ce = R.clu_enc[cl];
+            ce = R.clu_enc[cl];
             const float4* t = reinterpret_cast<const float4*>(Ts + 12 * R.clu_jnt[cl]);
             const float4 t0 = t[0], t1 = t[1], t2 = t[2];
             ax = fmaf(t0.x, ce.x, fmaf(t0.y, ce.y, fmaf(t0.z, ce.z, t0.w)));
             ay = fmaf(t1.x, ce.x, fmaf(t1.y, ce.y, fmaf(t1.z, ce.z, t1.w)));
             az = fmaf(t2.x, ce.x, fmaf(t2.y, ce.y, fmaf(t2.z, ce.z, t2.w)));
         }
-        const float cx = __shfl(ax, sub), cy = __shfl(ay, sub), cz = __shfl(az, sub);   // slot 0's centre
+        const bool in = cl < C && active && fabsf(ax) + fabsf(ay) + fabsf(az) < 1e4f;
+        const float inv_n = __builtin_amdgcn_rcpf(slots(in ? 1.0f : 0.0f));
+        const float cx = slots(in ? ax : 0.0f) * inv_n, cy = slots(in ? ay : 0.0f) * inv_n,
+                    cz = slots(in ? az : 0.0f) * inv_n;
         const float dx = ax - cx, dy = ay - cy, dz = az - cz;
         float d2 = (cl < C && active) ? fmaf(dz, dz, fmaf(dy, dy, dx * dx)) : 0.0f;
         d2 = fmaxf(d2, __shfl_xor(d2, 16));
         d2 = fmaxf(d2, __shfl_xor(d2, 32));
+        const float reach = band + ce.w + __builtin_amdgcn_sqrtf(d2) * 1.0001f + 1e-5f;
+        const float thr = reach * fabsf(reach);
         const int nk = min(kGrp, C - c0);
-        // up to 64 staged boxes: each lane reads its box's record once for
-        // every cluster of the pass
-        float4 q0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), q1 = q0, q2 = q0, qh = q0;
-        const bool one_word = n_obb <= 64;
-        if (one_word && lane < n_obb) {
-            q0 = s_obb[4 * lane]; q1 = s_obb[4 * lane + 1]; q2 = s_obb[4 * lane + 2]; qh = s_obb[4 * lane + 3];
-        }
-        for (int k = 0; k < nk; ++k) {
-            const float4 ce = uload4(R.clu_enc, c0 + k);
-            ObbMask mk;
-            const float c0x = read_lane(cx, k), c0y = read_lane(cy, k), c0z = read_lane(cz, k);
-            const float reach = band + ce.w + sqrtf(read_lane(d2, k)) * 1.0001f + 1e-5f;
-            const float thr = uniform(reach * fabsf(reach));
-            if (one_word) {
-                bool c = false;
-                if (lane < n_obb) {
-                    float lx, ly, lz;
-                    to_box(q0, q1, q2, c0x, c0y, c0z, lx, ly, lz);
-                    c = box_key(lx, ly, lz, qh) < thr;
-                }
-                mk.w[0] = __ballot(c);
-#pragma unroll
-                for (int w = 1; w < kMaskWords; ++w) mk.w[w] = 0ull;
-            } else
-#pragma unroll
-            for (int w = 0; w < kMaskWords; ++w) {
-                bool c = false;
-                if (w * 64 < n_obb) {
+        if (n_obb <= 64) {
+            // each lane reads its box's record once for every cluster of the pass
+            float4 q0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), q1 = q0, q2 = q0, qh = q0;
+            if (lane < n_obb) {
+                q0 = s_obb[4 * lane]; q1 = s_obb[4 * lane + 1]; q2 = s_obb[4 * lane + 2]; qh = s_obb[4 * lane + 3];
+            }
+            unsigned long long mine = 0ull;   // cluster c0 + lane's
+            for (int k = 0; k < nk; ++k) {
+                float lx, ly, lz;
+                to_box(q0, q1, q2, read_lane(cx, k), read_lane(cy, k), read_lane(cz, k), lx, ly, lz);
+                const unsigned long long m = __ballot(lane < n_obb && box_key(lx, ly, lz, qh) < read_lane(thr, k));
+                if (lane == k) mine = m;
+            }
+            if (lane < nk) s_mask[(c0 + lane) * kMaskWords] = mine;
+        } else {
+            for (int k = 0; k < nk; ++k) {
+                const float c0x = read_lane(cx, k), c0y = read_lane(cy, k), c0z = read_lane(cz, k), t = read_lane(thr, k);
+                for (int w = 0; w * 64 < n_obb; ++w) {
                     const int o = w * 64 + lane;
+                    bool c = false;
                     if (o < n_obb) {
                         float lx, ly, lz;
                         to_box(s_obb[4 * o], s_obb[4 * o + 1], s_obb[4 * o + 2], c0x, c0y, c0z, lx, ly, lz);
-                        c = box_key(lx, ly, lz, s_obb[4 * o + 3]) < thr;
+                        c = box_key(lx, ly, lz, s_obb[4 * o + 3]) < t;
                     }
+                    const unsigned long long m = __ballot(c);
+                    if (lane == 0) s_mask[(c0 + k) * kMaskWords + w] = m;
                 }
-                mk.w[w] = __ballot(c);
-            }
-            if (lane < kMaskWords) {
-                unsigned long long v = 0ull;
-#pragma unroll
-                for (int w = 0; w < kMaskWords; ++w) if (w == lane) v = mk.w[w];
-                s_mask[(c0 + k) * kMaskWords + lane] = v;
             }
         }
     }
@@ -1774,13 +1784,12 @@ __device__ __forceinline__ void grp_masks(const DRobot& R, const float4* __restr
 // LDS) and its LDS record index (-1: none). Two candidates per step: both
 // records are read before either test, so the LDS latency of one hides the
 // other's. Ties keep the lower index.
-__device__ __forceinline__ void grp_argmin(const float4* __restrict__ s_obb, const unsigned long long* own, bool valid,
+__device__ __forceinline__ void grp_argmin(const float4* __restrict__ s_obb, int n_obb, const unsigned long long* own, bool valid,
                                            float px, float py, float pz, const uint8_t* __restrict__ acm_row,
                                            float& best, int& arg) {
     best = FLT_MAX;
     arg = -1;
-#pragma unroll
-    for (int k = 0; k < kMaskWords; ++k) {
+    for (int k = 0; k * 64 < n_obb; ++k) {
         unsigned long long bits = valid ? own[k] : 0ull;
         while (bits) {
             const int oa = k * 64 + (__ffsll(bits) - 1);
@@ -1825,8 +1834,8 @@ __device__ __forceinline__ void cost_grp(const CostArgs& a) {
     const int fstride = J * 12 + 4;
     float* s_T = reinterpret_cast<float*>(s_end + 2 * kWave);
     int* s_par = reinterpret_cast<int*>(s_T + kGrpStates * fstride);   // [slot][J] pointer-jumping links
-    float* s_w = reinterpret_cast<float*>(s_par + kGrpStates * J);    // GRAD: [slot][J][6] wrenches
-    float* s_dq = s_w + kGrpStates * J * 6;                       // GRAD: [slot][kMaxDof + 1]
+    float* s_w = reinterpret_cast<float*>(s_par + kGrpStates * J);    // GRAD: [slot][kGrpWrench]
+    float* s_dq = s_w + kGrpStates * kGrpWrench;                  // GRAD: [slot][kMaxDof + 1]
     // tiled problems: per state slot and emission slot, the smallest box key
     // over the tiles so far and its OBB (original index, -1: none)
     float* s_best = GRAD ? s_dq + kGrpStates * (kMaxDof + 1) : s_w;
@@ -1846,6 +1855,11 @@ __device__ __forceinline__ void cost_grp(const CostArgs& a) {
     const long n_states = state_count(a.X);
     const int n_chunks = chunk_count(a.C, n_states);
     while (next_chunk(a.C, n_states, n_chunks, cur, ch)) {
+        // loads that wait for nothing else, in flight together
+        int u_end = 0, u_beg = 0;
+        prefetch_unit_ends(a.X, ch.w, u_end, u_beg);
+        JointRegs jt;
+        if (WORLD & 1) jt.load(R, sub);
         if ((WORLD & 1) && ch.x != cur_prob) {
             problem_obbs(a.C, a.S, ch.x, o0, o1);
             n_tiles = TILED ? uniform(obb_tiles(o0, o1, cap)) : 1;
@@ -1858,15 +1872,15 @@ __device__ __forceinline__ void cost_grp(const CostArgs& a) {
         const bool tiled = TILED && use_obb && n_tiles > 1;
         const long g = (long)ch.y + slot;
         const bool active = g < ch.z;
-        stage_unit_ends(a.X, ch.w, s_end);
+        s_end[lane] = u_end;
+        s_end[kWave + lane] = u_beg;
         if (GRAD)
-            for (int i = lane; i < kGrpStates * (J * 6 + kMaxDof + 1); i += kWave) s_w[i] = 0.0f;
+            for (int i = lane; i < kGrpStates * (kMaxDof + 1); i += kWave) s_dq[i] = 0.0f;
         __syncthreads();
         StateRef ref = load_state(a.X, D, g, active, s_q, ch.w, s_end, ch.x, slot, kGrpStates, sub == 0);
         __syncthreads();
         // 1a. joint frames (pointer jumping over the DFS tree)
-        JointRegs jt;
-        jt.load(R, sub);
+        if (!(WORLD & 1)) jt.load(R, sub);   // no registers to hold it from the start
         group_frames(jt, J, s_q + slot, kGrpStates, Ts, s_par + slot * J, sub);
         // 1b. candidate masks per sphere cluster; a tiled problem's OBBs pass through
         // LDS tile by tile, each tile's argmins folded into s_best / s_barg
@@ -1893,7 +1907,7 @@ __device__ __forceinline__ void cost_grp(const CostArgs& a) {
                 const uint8_t* acm_row = a.S.sphere_obb_acm ? a.S.sphere_obb_acm + (size_t)sid * a.S.n_obbs : nullptr;
                 float best;
                 int arg;
-                grp_argmin(s_obb, s_mask + R.sph_clu[sc] * kMaskWords, valid, px, py, pz, acm_row, best, arg);
+                grp_argmin(s_obb, n_obb, s_mask + R.sph_clu[sc] * kMaskWords, valid, px, py, pz, acm_row, best, arg);
                 if (valid) {
                     float* bk = s_best + slot * S + s;
                     int* ba = s_barg + slot * S + s;
@@ -1927,24 +1941,10 @@ __device__ __forceinline__ void cost_grp(const CostArgs& a) {
         const float* Tr = s_T + rslot * fstride;
         const int r_si = __shfl(si, rslot * kGrp), r_sj = __shfl(sj, rslot * kGrp);
         const float r_snx = __shfl(snx, rslot * kGrp), r_sny = __shfl(sny, rslot * kGrp), r_snz = __shfl(snz, rslot * kGrp);
-        // wrench of a sphere's point gradient g at p about its joint's origin o
-        auto add_wrench = [&](int jj, int sid, float px, float py, float pz, float ox, float oy, float oz, float gx,
-                              float gy, float gz) {
-            if (r_si >= 0) {
-                if (sid == r_si) { gx -= r_snx; gy -= r_sny; gz -= r_snz; }
-                if (sid == r_sj) { gx += r_snx; gy += r_sny; gz += r_snz; }
-            }
-            if (gx != 0.0f || gy != 0.0f || gz != 0.0f) {
-                const float rx = px - ox, ry = py - oy, rz = pz - oz;
-                float* w = s_w + (rslot * J + jj) * 6;
-                atomicAdd(w + 0, gx);
-                atomicAdd(w + 1, gy);
-                atomicAdd(w + 2, gz);
-                atomicAdd(w + 3, ry * gz - rz * gy);
-                atomicAdd(w + 4, rz * gx - rx * gz);
-                atomicAdd(w + 5, rx * gy - ry * gx);
-            }
-        };
+        // Joint `sub` of state `slot`: the force and the moment about its
+        // origin of its spheres' point gradients so far (GRAD).
+        float f0 = 0.0f, f1 = 0.0f, f2 = 0.0f, m0 = 0.0f, m1 = 0.0f, m2 = 0.0f;
+        const int js0 = GRAD && sub < J ? R.sph_off[sub] : 0, js1 = GRAD && sub < J ? R.sph_off[sub + 1] : 0;
         for (int r0 = 0; r0 < S; r0 += kGrp) {
             const int s = r0 + rsub;
             const bool valid = ractive && s < S;
@@ -1966,9 +1966,8 @@ __device__ __forceinline__ void cost_grp(const CostArgs& a) {
                 }
             } else if (use_obb) {
                 const uint8_t* acm_row = a.S.sphere_obb_acm ? a.S.sphere_obb_acm + (size_t)sid * a.S.n_obbs : nullptr;
-                grp_argmin(s_obb, s_mask + R.sph_clu[sc] * kMaskWords, valid, px, py, pz, acm_row, best, arg);
+                grp_argmin(s_obb, n_obb, s_mask + R.sph_clu[sc] * kMaskWords, valid, px, py, pz, acm_row, best, arg);
             }
-            if (!valid) continue;
             auto rec = [&](float4& r0, float4& r1, float4& r2, float4& r3) {
                 if (tiled) {
                     float4 t[4];
@@ -1978,12 +1977,36 @@ __device__ __forceinline__ void cost_grp(const CostArgs& a) {
                     r0 = s_obb[4 * arg]; r1 = s_obb[4 * arg + 1]; r2 = s_obb[4 * arg + 2]; r3 = s_obb[4 * arg + 3];
                 }
             };
-            float gx, gy, gz;
-            const float hs =
-                sphere_hinge_at<GRAD, ONE>(a, layer, arg >= 0, rec, best, px, py, pz, sp.w, sid, use_obb,
-                                      use_esdf, gx, gy, gz);
-            world += hs;
-            if (GRAD) add_wrench(jj, sid, px, py, pz, t0.w, t1.w, t2.w, gx, gy, gz);
+            float gx = 0.0f, gy = 0.0f, gz = 0.0f;
+            if (valid)
+                world += sphere_hinge_at<GRAD, ONE>(a, layer, arg >= 0, rec, best, px, py, pz, sp.w, sid, use_obb,
+                                                    use_esdf, gx, gy, gz);
+            if (GRAD) {
+                if (valid && r_si >= 0) {
+                    if (sid == r_si) { gx -= r_snx; gy -= r_sny; gz -= r_snz; }
+                    if (sid == r_sj) { gx += r_snx; gy += r_sny; gz += r_snz; }
+                }
+                const bool nz = gx != 0.0f || gy != 0.0f || gz != 0.0f;
+                if (!wave_any(nz)) continue;
+                // The round's wrenches (g and (p - o) x g about the joint's origin
+                // o) through LDS to their joints' lanes, added in emission order.
+                __syncthreads();
+                const float rx = px - t0.w, ry = py - t1.w, rz = pz - t2.w;
+                float2* w = reinterpret_cast<float2*>(s_w + rslot * kGrpWrench + rsub * 6);
+                w[0] = make_float2(gx, gy);
+                w[1] = make_float2(gz, nz ? ry * gz - rz * gy : 0.0f);
+                w[2] = nz ? make_float2(rz * gx - rx * gz, rx * gy - ry * gx) : make_float2(0.0f, 0.0f);
+                __syncthreads();
+                const int k1 = min(js1 - r0, kGrp);
+                for (int k = max(js0 - r0, 0); k < k1; k += 2) {
+                    const float2* u = reinterpret_cast<const float2*>(s_w + slot * kGrpWrench + k * 6);
+                    const bool two = k + 1 < k1;
+                    const float2* v = two ? u + 3 : u;
+                    const float2 u0 = u[0], u1 = u[1], u2 = u[2], v0 = v[0], v1 = v[1], v2 = v[2];
+                    f0 += u0.x; f1 += u0.y; f2 += u1.x; m0 += u1.y; m1 += u2.x; m2 += u2.y;
+                    if (two) { f0 += v0.x; f1 += v0.y; f2 += v1.x; m0 += v1.y; m1 += v2.x; m2 += v2.y; }
+                }
+            }
         }
         // each state's partial sums sit in the lanes with its lane & 3; the
         // pairwise tree matches a 16-lane group sum's
@@ -1998,16 +2021,13 @@ __device__ __forceinline__ void cost_grp(const CostArgs& a) {
             // origin m_i = tau_i + o_i x f_i; DFS subtrees are contiguous, so
             // joint j's subtree force and moment are P(jend[j] - 1) -
             // P(j - 1), and its moment about o_j is M - o_j x F.
-            float f0 = 0.0f, f1 = 0.0f, f2 = 0.0f, m0 = 0.0f, m1 = 0.0f, m2 = 0.0f;
             float ox = 0.0f, oy = 0.0f, oz = 0.0f;
             if (sub < J) {
-                const float* w = s_w + (slot * J + sub) * 6;
                 const float* Tj = Ts + 12 * sub;
                 ox = Tj[3]; oy = Tj[7]; oz = Tj[11];
-                f0 = w[0]; f1 = w[1]; f2 = w[2];
-                m0 = w[3] + (oy * f2 - oz * f1);
-                m1 = w[4] + (oz * f0 - ox * f2);
-                m2 = w[5] + (ox * f1 - oy * f0);
+                m0 += oy * f2 - oz * f1;
+                m1 += oz * f0 - ox * f2;
+                m2 += ox * f1 - oy * f0;
             }
 #pragma unroll
             for (int off = 1; off < kGrp; off <<= 1) {

@@ -193,3 +193,22 @@ def test_state_cost_runs(name, n, boxes, group, margin, masked):
     o, prm = PO.Oracle(arr, scene, nthreads=8), PO.cost_params(**kw)
     ref = o.hinge_cost(q, prm)
     np.testing.assert_array_less(np.abs(st.cpu().numpy() - ref) / cost_den(ref, 2.0, o.hinge_terms(q, prm)), 1e-5)
+
+
+@pytest.mark.parametrize("name,n,boxes", [("panda", 1, 64), ("fetch", 3, 65), ("baxter", 5, 128), ("branched", 66, 30),
+                                          ("fetch", 130, 130), ("panda", 41, 256)])
+def test_adjoint_masks_and_wrenches(name, n, boxes):
+    """State counts that leave slots of a wave empty, boxes around one, two and
+    four mask words, joints whose spheres cross the rounds of sixteen."""
+    rob = S.Robot(_branched_panda() if name == "branched" else name)
+    arr, rng = rob.arrays, np.random.default_rng(3 * n + boxes)
+    scene = W.random_obbs(rng, boxes, half_hi=0.15)
+    q = W.uniform_configs(rng, arr, n)
+    kw = dict(world_margin=0.05, self_margin=0.02, weight=2.0)
+    c, _, g = S.hinge_cost(S.Plan.configs(rob, n), S.DeviceScene.from_host(scene), torch.from_numpy(q).to(DEV),
+                           S.cost_params(**kw), grad=True)
+    o, prm = PO.Oracle(arr, scene, nthreads=8), PO.cost_params(**kw)
+    ref, g_ref, kink = o.hinge_grad(q, prm)
+    np.testing.assert_array_less(np.abs(c.cpu().numpy() - ref) / cost_den(ref, 2.0, o.hinge_terms(q, prm)), 1e-5)
+    err = np.linalg.norm(g.cpu().numpy() - g_ref, axis=1) / np.maximum(np.linalg.norm(g_ref, axis=1), 2.0)
+    assert np.all(err[~kink.astype(bool)] < 1e-4)
