@@ -278,7 +278,7 @@ constexpr int kCollideWaves = 8;
 // upper bound (counted on the device): the grid stays at what the chip holds.
 DChunks collide_chunks(long n_states, const DRobot& R, const DScene& S, int* grid_out, bool bound = false) {
     return implicit_chunks(n_states, (bound ? 1 : kCollideWaves) * grid_collide(R, S, obb_tile(S.n_obbs)), S.n_obbs,
-                           grid_out);
+                           grid_out, bound ? 1 : collide_lanes(R, n_states));
 }
 
 // The cost kernel over n_states implicit chunks: k_state_cost or k_cost_grad with one lane per
@@ -498,9 +498,10 @@ DChunks plan_collide_chunks(ppl_plan_s* P, const DScene& S, int max_obbs, int* g
     DChunks C{};
     C.obb_cap = tile;
     C.tiled = max_obbs > tile;
-    C.tab = P->d_tab[0];
-    C.n_chunks = P->n_chunks[0];
-    C.chunk = kWave;
+    const int lanes = collide_lanes(P->robot->R, P->n_states), gi = group_index(lanes);
+    C.tab = P->d_tab[gi];   // made with the plan
+    C.n_chunks = P->n_chunks[gi];
+    C.chunk = kWave / lanes;
     C.obb_off = P->d_obb_off;
     const int occ = grid_collide(P->robot->R, S, tile);
     const int g = gm == 2 ? C.n_chunks : (gm == 1 ? 2 * occ : kCollideWaves * occ);
@@ -1481,6 +1482,7 @@ ppl_status ppl_plan_create(ppl_robot r, const ppl_plan_desc* d, ppl_plan* out) t
     for (size_t i = 0; i < uoff.size(); ++i) P->h_off[i] = (int)uoff[i];
     for (size_t i = 0; i + 1 < uoff.size(); ++i) P->t_max = std::max(P->t_max, (int)(uoff[i + 1] - uoff[i]));
     hipError_t e = ensure_table(P, 1);
+    if (e == hipSuccess) e = ensure_table(P, collide_lanes(P->robot->R, P->n_states));   // the any-collision pass's
     if (e == hipSuccess && !prob.empty()) {
         e = hipMalloc((void**)&P->d_prob, prob.size() * sizeof(int4));
         if (e == hipSuccess) e = hipMemcpy(P->d_prob, prob.data(), prob.size() * sizeof(int4), hipMemcpyHostToDevice);

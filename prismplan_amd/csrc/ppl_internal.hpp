@@ -213,6 +213,18 @@ struct SelfArgs {
 };
 
 // t0 / t1 (optional): events the runtime records at the kernel's start and end
+// Lanes per state of an any-collision launch of so many states (chunks hold 64
+// over that; models that need the gated form take one). A wave of 64 states is a
+// long chain when nothing else runs beside it, above all of box tests where the
+// states lie apart; past some waves a SIMD the frames computed four times cost
+// more than the shorter chains give. Configurations among 20 boxes from the host,
+// us a call with one lane and with four, Panda (Fetch): 256 54.8 and 40.6 (27.8,
+// 28.3), 4,096 63.4 and 48.9 (37.5, 37.1), 32,768 101 and 85.5 (85.6, 87.1), 65,536
+// 146 and 139 (131, 135), 131,072 208 and 218 (200, 206); 14 edges of 884 Panda
+// states 49.7 and 44.2, 512 of 33,809 70.8 and 56.7 (Fetch, 29,694 states, 56.5 and 50.1).
+constexpr int kCollideParts = 4;
+constexpr long kCollideSplit = 32768;
+int collide_lanes(const DRobot& R, long n_states);
 hipError_t launch_collide(const CollideArgs& a, int grid, hipStream_t s, hipEvent_t t0 = nullptr,
                           hipEvent_t t1 = nullptr);
 hipError_t launch_cost(const CostArgs& a, int grid, hipStream_t s, hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr);

@@ -212,3 +212,32 @@ def test_adjoint_masks_and_wrenches(name, n, boxes):
     np.testing.assert_array_less(np.abs(c.cpu().numpy() - ref) / cost_den(ref, 2.0, o.hinge_terms(q, prm)), 1e-5)
     err = np.linalg.norm(g.cpu().numpy() - g_ref, axis=1) / np.maximum(np.linalg.norm(g_ref, axis=1), 2.0)
     assert np.all(err[~kink.astype(bool)] < 1e-4)
+
+
+@pytest.mark.parametrize("name,n,boxes,layers", [("panda", 1, 1, 0), ("fetch", 17, 63, 0), ("branched", 95, 64, 1),
+                                                 ("panda", 33, 65, 1), ("baxter", 640, 20, 0), ("panda", 300, 257, 1)])
+def test_small_checks_equal_large_ones(name, n, boxes, layers):
+    """A small launch gives every state four lanes, each a fourth of the boxes:
+    states around a chunk of 16, boxes around a staging, layers after the boxes,
+    masked pairs. The same states among many more, past the limit of such
+    launches, have the same verdicts."""
+    rob = S.Robot(_branched_panda() if name == "branched" else name)
+    arr, rng = rob.arrays, np.random.default_rng(n + boxes)
+    scene = W.random_obbs(rng, boxes, half_hi=0.12)
+    if layers:
+        params, pose = W.esdf_grid(center=(0.45, 0.0, 0.45), n=48, voxel=0.03)
+        inside = W.random_obbs(rng, 3)
+        vals = PO.esdf_from_obbs(inside.obb_dims, inside.obb_pose, params, pose)
+        scene.voxel_params, scene.voxel_pose = params, pose
+        scene.voxel_features, scene.voxel_enable = vals.astype(np.float32).reshape(1, -1), np.ones(1, np.uint8)
+        scene.sphere_obb_acm = (rng.random((arr.n_spheres, boxes)) < 0.8).astype(np.uint8)
+    ds = S.DeviceScene.from_host(scene)
+    q = W.uniform_configs(rng, arr, 33000)
+    big = S.check_collision_batched(S.Plan.configs(rob, len(q)), ds, torch.from_numpy(q).to(DEV), check_self=False)
+    got = S.check_collision_batched(S.Plan.configs(rob, n), ds, torch.from_numpy(q[:n]).to(DEV), check_self=False)
+    np.testing.assert_array_equal(got.cpu().numpy(), big.cpu().numpy()[:n])
+    to = np.clip(q + rng.uniform(-0.6, 0.6, q.shape), arr.joint_lower, arr.joint_upper).astype(np.float32)
+    ns = rng.integers(2, 40, len(q)).astype(np.int32)
+    fh = [S.edge_check_batched(S.Plan.edges(rob, ns[:m]), ds, torch.from_numpy(q[:m]).to(DEV),
+                               torch.from_numpy(to[:m]).to(DEV)).cpu().numpy() for m in (n, len(q))]
+    np.testing.assert_array_equal(fh[0], fh[1][:n])
