@@ -258,12 +258,17 @@ __device__ __forceinline__ void to_box(const float4& r0, const float4& r1, const
     lz = fmaf(r2.x, px, fmaf(r2.y, py, fmaf(r2.z, pz, r2.w)));
 }
 
-// Collision iff squared distance to the box < r^2 (scene_collision.cuh:59-78).
-__device__ __forceinline__ bool box_hit(float lx, float ly, float lz, const float4& h, float r2) {
+// Squared distance to the box.
+__device__ __forceinline__ float box_dist2(float lx, float ly, float lz, const float4& h) {
     const float cx = fmaxf(fabsf(lx) - h.x, 0.0f);
     const float cy = fmaxf(fabsf(ly) - h.y, 0.0f);
     const float cz = fmaxf(fabsf(lz) - h.z, 0.0f);
-    return fmaf(cz, cz, fmaf(cy, cy, cx * cx)) < r2;
+    return fmaf(cz, cz, fmaf(cy, cy, cx * cx));
+}
+
+// Collision iff squared distance to the box < r^2 (scene_collision.cuh:59-78).
+__device__ __forceinline__ bool box_hit(float lx, float ly, float lz, const float4& h, float r2) {
+    return box_dist2(lx, ly, lz, h) < r2;
 }
 
 // Order-preserving key of the box signed distance (Quilez form,
@@ -751,6 +756,13 @@ __device__ __forceinline__ float row_sum(float v) {
     return v + dpp<0x121>(v);
 }
 
+// |d|^2 for a bound over several lanes: infinite where d is no number, which
+// a maximum would pass over.
+__device__ __forceinline__ float spread2(float dx, float dy, float dz) {
+    const float v = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+    return v >= 0.0f ? v : INFINITY;
+}
+
 // A row's 16 bits of a ballot (row: its first lane).
 __device__ __forceinline__ unsigned row_bits(unsigned long long m, int row) {
     const unsigned w = row >= 32 ? (unsigned)(m >> 32) : (unsigned)m;
@@ -949,7 +961,9 @@ __global__ __launch_bounds__(64, 4) void k_collide(CollideArgs a) {
                     const int l0 = row + (in_row >> 8 ? 7 + __ffs(in_row >> 8) : in_row ? __ffs(in_row) - 1 : 0);
                     const float cx = __shfl(px, l0), cy = __shfl(py, l0), cz = __shfl(pz, l0);
                     const float dx = px - cx, dy = py - cy, dz = pz - cz;
-                    const float d2 = row_max(active ? fmaf(dz, dz, fmaf(dy, dy, dx * dx)) : 0.0f);
+                    // (a state that is not finite, at the centre or beside it,
+                    // makes the spread infinite and every box a candidate)
+                    const float d2 = row_max(active ? spread2(dx, dy, dz) : 0.0f);
                     const float reach = __builtin_amdgcn_sqrtf(d2) * 1.0001f + fabsf(rr) + 1e-5f;
                     const float reach2 = reach * reach;
                     for (int base = 0; base < n_obb; base += kWave) {
@@ -962,7 +976,7 @@ __global__ __launch_bounds__(64, 4) void k_collide(CollideArgs a) {
                             const int k = SPLIT ? 4 * (lane & 15) + part : 16 * r + (lane & 15), o = base + min(k, m - 1);
                             float lx, ly, lz;
                             to_box(s_obb[kObbRec * o], s_obb[kObbRec * o + 1], s_obb[kObbRec * o + 2], cx, cy, cz, lx, ly, lz);
-                            const bool c = k < m && box_hit(lx, ly, lz, s_obb[kObbRec * o + 3], reach2);
+                            const bool c = k < m && !(box_dist2(lx, ly, lz, s_obb[kObbRec * o + 3]) > reach2);
                             todo |= (unsigned long long)row_bits(__ballot(c), row) << (16 * r);
                         }
                         if (!active) todo = 0ull;
