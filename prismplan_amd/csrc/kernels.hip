@@ -737,18 +737,11 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
-// Maximum over the 16 lanes of a row (lanes 16 k .. 16 k + 15), by row rotations.
+// Over the 16 lanes of a row (lanes 16 k .. 16 k + 15), by row rotations.
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
 }
-__device__ __forceinline__ float row_max(float v) {
-    v = fmaxf(v, dpp<0x128>(v));
-    v = fmaxf(v, dpp<0x124>(v));
-    v = fmaxf(v, dpp<0x122>(v));
-    return fmaxf(v, dpp<0x121>(v));
-}
-
 __device__ __forceinline__ float row_sum(float v) {
     v += dpp<0x128>(v);
     v += dpp<0x124>(v);
@@ -756,11 +749,24 @@ __device__ __forceinline__ float row_sum(float v) {
     return v + dpp<0x121>(v);
 }
 
-// |d|^2 for a bound over several lanes: infinite where d is no number, which
-// a maximum would pass over.
-__device__ __forceinline__ float spread2(float dx, float dy, float dz) {
-    const float v = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-    return v >= 0.0f ? v : INFINITY;
+// Maximum of values that are not negative, in which a NaN stays (fmaxf drops
+// it): their bits order as unsigned numbers, NaN above infinity. For bounds that
+// a lane which is no number must not pass; a test against one keeps what it
+// cannot rule out.
+__device__ __forceinline__ float max_nan(float a, float b) {
+    return __uint_as_float(max(__float_as_uint(a), __float_as_uint(b)));
+}
+__device__ __forceinline__ float row_max_nan(float v) {
+    v = max_nan(v, dpp<0x128>(v));
+    v = max_nan(v, dpp<0x124>(v));
+    v = max_nan(v, dpp<0x122>(v));
+    return max_nan(v, dpp<0x121>(v));
+}
+
+// Whether a place may enter a mean: finite, and 64 of them sum and square
+// within FP32. (With none, the mean is NaN.)
+__device__ __forceinline__ bool usable(float x, float y, float z) {
+    return fabsf(x) + fabsf(y) + fabsf(z) < 1e16f;
 }
 
 // A row's 16 bits of a ballot (row: its first lane).
@@ -962,8 +968,8 @@ __global__ __launch_bounds__(64, 4) void k_collide(CollideArgs a) {
                     const float cx = __shfl(px, l0), cy = __shfl(py, l0), cz = __shfl(pz, l0);
                     const float dx = px - cx, dy = py - cy, dz = pz - cz;
                     // (a state that is not finite, at the centre or beside it,
-                    // makes the spread infinite and every box a candidate)
-                    const float d2 = row_max(active ? spread2(dx, dy, dz) : 0.0f);
+                    // makes the spread no number or infinite, and every box a candidate)
+                    const float d2 = row_max_nan(active ? fmaf(dz, dz, fmaf(dy, dy, dx * dx)) : 0.0f);
                     const float reach = __builtin_amdgcn_sqrtf(d2) * 1.0001f + fabsf(rr) + 1e-5f;
                     const float reach2 = reach * reach;
                     for (int base = 0; base < n_obb; base += kWave) {
@@ -1192,8 +1198,8 @@ __global__ __launch_bounds__(64) void k_collide_gated(CollideArgs a) {
 // of the OBBs some active lane's spheres of the cluster can come within the
 // hinge band of. Every sphere s of the cluster lies inside its enclosing
 // sphere `as` (centre a, radius R; DRobot::clu_enc), so clr(s, o) >=
-// sdf_o(a) - R; the active lanes' centres lie within rw of c0, about their
-// mean (of those at finite places; the others make rw large instead), so
+// sdf_o(a) - R; the active lanes' centres lie within rw of c0, the mean of
+// those at usable places (another one makes rw infinite or no number), so
 // sdf_o(a) >= sdf_o(c0) - rw. An OBB with sdf_o(c0) >= band + R + rw therefore
 // has clearance >= band from every sphere: it cannot change a hinge, its argmin
 // or its gradient. One pass per 64 OBBs (lane i tests OBB base + i).
@@ -1205,13 +1211,13 @@ __device__ __forceinline__ void near_obbs(const float4* __restrict__ s_obb, int 
     auto wave = [](float v) {   // a row's value in each of its lanes -> the four rows'
         return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
     };
-    const bool in = active && fabsf(ax) + fabsf(ay) + fabsf(az) < 1e4f;
+    const bool in = active && usable(ax, ay, az);
     const float inv_n = __builtin_amdgcn_rcpf((float)__popcll(__ballot(in)));
     const float cx = wave(row_sum(in ? ax : 0.0f)) * inv_n, cy = wave(row_sum(in ? ay : 0.0f)) * inv_n,
                 cz = wave(row_sum(in ? az : 0.0f)) * inv_n;
     const float dx = ax - cx, dy = ay - cy, dz = az - cz;
-    const float v = row_max(active ? fmaf(dz, dz, fmaf(dy, dy, dx * dx)) : 0.0f);
-    const float d2 = fmaxf(fmaxf(read_lane(v, 0), read_lane(v, 16)), fmaxf(read_lane(v, 32), read_lane(v, 48)));
+    const float v = row_max_nan(active ? fmaf(dz, dz, fmaf(dy, dy, dx * dx)) : 0.0f);
+    const float d2 = max_nan(max_nan(read_lane(v, 0), read_lane(v, 16)), max_nan(read_lane(v, 32), read_lane(v, 48)));
     // sdf(c0) < reach  <=>  key(c0) < reach * |reach|; slack covers rounding
     const float reach = band + as.w + __builtin_amdgcn_sqrtf(d2) * 1.0001f + 1e-5f;
     const float thr = reach * fabsf(reach);
@@ -1222,7 +1228,7 @@ __device__ __forceinline__ void near_obbs(const float4* __restrict__ s_obb, int 
         const int o = min(k * 64 + lane_id(), n_obb - 1);
         float lx, ly, lz;
         to_box(s_obb[STRIDE * o], s_obb[STRIDE * o + 1], s_obb[STRIDE * o + 2], cx, cy, cz, lx, ly, lz);
-        w[k] = __ballot(k * 64 + lane_id() < n_obb && box_key(lx, ly, lz, s_obb[STRIDE * o + 3]) < thr);
+        w[k] = __ballot(k * 64 + lane_id() < n_obb && !(box_key(lx, ly, lz, s_obb[STRIDE * o + 3]) >= thr));
     }
 }
 
@@ -1762,14 +1768,14 @@ __device__ __forceinline__ void grp_masks(const DRobot& R, const float4* __restr
             ay = fmaf(t1.x, ce.x, fmaf(t1.y, ce.y, fmaf(t1.z, ce.z, t1.w)));
             az = fmaf(t2.x, ce.x, fmaf(t2.y, ce.y, fmaf(t2.z, ce.z, t2.w)));
         }
-        const bool in = cl < C && active && fabsf(ax) + fabsf(ay) + fabsf(az) < 1e4f;
+        const bool in = cl < C && active && usable(ax, ay, az);
         const float inv_n = __builtin_amdgcn_rcpf(slots(in ? 1.0f : 0.0f));
         const float cx = slots(in ? ax : 0.0f) * inv_n, cy = slots(in ? ay : 0.0f) * inv_n,
                     cz = slots(in ? az : 0.0f) * inv_n;
         const float dx = ax - cx, dy = ay - cy, dz = az - cz;
         float d2 = (cl < C && active) ? fmaf(dz, dz, fmaf(dy, dy, dx * dx)) : 0.0f;
-        d2 = fmaxf(d2, __shfl_xor(d2, 16));
-        d2 = fmaxf(d2, __shfl_xor(d2, 32));
+        d2 = max_nan(d2, __shfl_xor(d2, 16));
+        d2 = max_nan(d2, __shfl_xor(d2, 32));
         const float reach = band + ce.w + __builtin_amdgcn_sqrtf(d2) * 1.0001f + 1e-5f;
         const float thr = reach * fabsf(reach);
         const int nk = min(kGrp, C - c0);
@@ -1783,7 +1789,7 @@ __device__ __forceinline__ void grp_masks(const DRobot& R, const float4* __restr
             for (int k = 0; k < nk; ++k) {
                 float lx, ly, lz;
                 to_box(q0, q1, q2, read_lane(cx, k), read_lane(cy, k), read_lane(cz, k), lx, ly, lz);
-                const unsigned long long m = __ballot(lane < n_obb && box_key(lx, ly, lz, qh) < read_lane(thr, k));
+                const unsigned long long m = __ballot(lane < n_obb && !(box_key(lx, ly, lz, qh) >= read_lane(thr, k)));
                 if (lane == k) mine = m;
             }
             if (lane < nk) s_mask[(c0 + lane) * kMaskWords] = mine;
@@ -1796,7 +1802,7 @@ __device__ __forceinline__ void grp_masks(const DRobot& R, const float4* __restr
                     if (o < n_obb) {
                         float lx, ly, lz;
                         to_box(s_obb[4 * o], s_obb[4 * o + 1], s_obb[4 * o + 2], c0x, c0y, c0z, lx, ly, lz);
-                        c = box_key(lx, ly, lz, s_obb[4 * o + 3]) < t;
+                        c = !(box_key(lx, ly, lz, s_obb[4 * o + 3]) >= t);
                     }
                     const unsigned long long m = __ballot(c);
                     if (lane == 0) s_mask[(c0 + k) * kMaskWords + w] = m;

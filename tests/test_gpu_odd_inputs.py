@@ -70,3 +70,78 @@ def test_edges_beside_one_without_an_end(n):
     np.testing.assert_array_equal(fh1[~bad], fh0[~bad])
     ok = ~np.repeat(bad, ns)
     np.testing.assert_array_equal(hits1[ok], hits0[ok])
+
+
+def _millimetres(shift):
+    """Panda in millimetres, its first moving link `shift` mm from the origin."""
+    a = load_robot_asset("panda")
+    ft = np.array(a["fixed_transforms"], np.float64).reshape(-1, 4, 4)
+    ft[:, :3, 3] *= 1000.0
+    ft[1, :3, 3] += shift
+    a["fixed_transforms"] = ft.reshape(-1).tolist()
+    for k in ("spheres_flat", "approx_spheres_flat"):
+        a[k] = (1000.0 * np.array(a[k])).tolist()
+    return a
+
+
+@pytest.mark.parametrize("n,boxes", [(1, 12), (70, 20), (203, 70)])
+@pytest.mark.parametrize("group", [1, 4, _ppl.PPL_COST_GROUPED])
+def test_costs_far_from_the_origin(n, boxes, group):
+    """Every state's links lie past 10 m in millimetres: boxes are found there
+    as anywhere. FP32 places a sphere at 16,000 mm within 16,000 x 4.6e-7 =
+    0.0074 mm of FP64 (parity_common's ratio), a box's face within as much
+    again, so a hinge term is within 0.015 mm; weight 2. A gradient's direction
+    turns by about 0.015 mm over the distance to the box, which is small for
+    most states but has no bound at an edge of a box."""
+    shift = np.array([16000.0, -300.0, 200.0])
+    rob = S.Robot(_millimetres(shift))
+    arr, rng = rob.arrays, np.random.default_rng(n + boxes)
+    m = W.random_obbs(rng, boxes, half_hi=0.2)
+    scene = W.random_obbs(np.random.default_rng(n + boxes), boxes, lo=1000 * np.array(W.PANDA_BOX_LO) + shift,
+                          hi=1000 * np.array(W.PANDA_BOX_HI) + shift, half_lo=20.0, half_hi=200.0)
+    assert m.n_obbs == scene.n_obbs
+    q = W.uniform_configs(rng, arr, n)
+    ds, plan = S.DeviceScene.from_host(scene), S.Plan.configs(rob, n)
+    kw = dict(world_margin=50.0, weight=2.0, use_self=False, use_esdf=False)
+    o, prm = PO.Oracle(arr, scene, nthreads=8), PO.cost_params(**kw)
+    ref, g_ref, kink = o.hinge_grad(q, prm, tol=0.03)
+    bar = 1e-5 * np.abs(ref) + 2.0 * 0.015 * np.maximum(o.hinge_terms(q, prm), 1)
+    plan.set_cost_group(group)
+    c0 = S.hinge_cost(plan, ds, up(q), S.cost_params(**kw))[0].cpu().numpy()
+    assert np.all(np.abs(c0 - ref) < bar) and (n == 1 or (ref > 0).mean() > 0.5)
+    plan.set_cost_group(group, grad=True)
+    c1, _, g = S.hinge_cost(plan, ds, up(q), S.cost_params(**kw), grad=True)
+    assert np.all(np.abs(c1.cpu().numpy() - ref) < bar)
+    err = np.linalg.norm(g.cpu().numpy() - g_ref, axis=1) / np.maximum(np.linalg.norm(g_ref, axis=1), 1.0)
+    assert np.mean(err[~kink] < 1e-2) > 0.95 or n == 1
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, 3e38])
+@pytest.mark.parametrize("group", [1, 4, _ppl.PPL_COST_GROUPED])
+def test_costs_beside_non_finite_states(bad, group):
+    """Costs, gradients, clearances and frames of the other states of a wave
+    stay what they are without the bad ones (a prismatic joint, so that its
+    place and not only its turn is lost)."""
+    rob, n = S.Robot("fetch"), 130
+    rng = np.random.default_rng(11)
+    q = W.uniform_configs(rng, rob.arrays, n)
+    ds = S.DeviceScene.from_host(W.random_obbs(rng, 40, W.FETCH_BOX_LO, W.FETCH_BOX_HI, half_hi=0.15))
+    prm, pose = W.esdf_grid(center=(0.6, 0.0, 0.8), n=48, voxel=0.03)
+    grid = S.DeviceScene.from_host(HostScene(voxel_params=prm, voxel_pose=pose, voxel_enable=np.ones(1, np.uint8), esdf_interp=1,
+                                             voxel_features=rng.normal(0, 0.2, (1, 48 ** 3)).astype(np.float32)))
+    plan = S.Plan.configs(rob, n)
+    plan.set_cost_group(group)
+    plan.set_cost_group(group, grad=True)
+    cp = S.cost_params(world_margin=0.05, self_margin=0.05, weight=2.0)
+
+    def run(x):
+        x = up(x)
+        out = [S.hinge_cost(plan, ds, x, cp)[0]] + [o for s in (ds, grid) for o in S.hinge_cost(plan, s, x, cp, grad=True)[::2]]
+        out += [S.min_clearance_batched(plan, grid, x), *S.fk_batched(plan, x)]
+        return [o.cpu().numpy() for o in out]
+
+    is_bad = (np.arange(n) % 5 == 0) | (np.arange(n) >= 126)
+    ref, keep = run(q), ~is_bad
+    q[is_bad, 0] = bad
+    for x, y in zip(run(q), ref):
+        np.testing.assert_array_equal(x[keep], y[keep])
