@@ -889,7 +889,10 @@ ppl_status ppl_robot_create(const ppl_robot_desc* d, ppl_robot* out) try {
             if (clu_of_slot[u] > clu_of_slot[v] || (clu_of_slot[u] == clu_of_slot[v] && u > v)) std::swap(u, v);
             ent.push_back({clu_of_slot[u], clu_of_slot[v], u, v});
         }
+        // (a pair may be named more than once, either way round; a block's
+        // count says whether it holds all pairs of its clusters)
         std::sort(ent.begin(), ent.end());
+        ent.erase(std::unique(ent.begin(), ent.end()), ent.end());
         for (size_t k = 0; k < ent.size();) {
             size_t e = k;
             while (e < ent.size() && ent[e][0] == ent[k][0] && ent[e][1] == ent[k][1]) ++e;

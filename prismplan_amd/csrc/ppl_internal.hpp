@@ -53,7 +53,7 @@ struct DRobot {
     const float4* sph_orig;     // [S] spheres by original index
     const int2* pairs;          // [n_pairs] exact self pairs (original indices), grouped by joint pair
     const int4* cpb;            // [n_cpb] self-pair blocks: (cluster A, cluster B, first pair, pairs), A <= B
-    const unsigned* cpl;        // [n_pairs] block pair lists: slot a | slot b << 16 (emission slots)
+    const unsigned* cpl;        // block pair lists, each pair once: slot a | slot b << 16 (emission slots)
     int n_cpb;
     // the same blocks as the pair walk reads them: (A | B << 8 | nb << 16, a0 | b0 << 16, first pair, pairs | inv << 16),
     // a0, b0 the clusters' first slots, nb B's spheres when the block holds every pair in order, else 0,

@@ -145,3 +145,47 @@ def test_costs_beside_non_finite_states(bad, group):
     q[is_bad, 0] = bad
     for x, y in zip(run(q), ref):
         np.testing.assert_array_equal(x[keep], y[keep])
+
+
+def _repeated_pairs():
+    """Panda with every other self pair left out and the others named twice,
+    as (i, j) and as (j, i)."""
+    a = load_robot_asset("panda")
+    r = np.array(a["self_cc_ranges_flat"], np.int64).reshape(-1, 3)
+    pairs = [(i, j) for i, lo, hi in r.tolist() for j in range(lo, hi + 1) if (i + j) % 2 == 0]
+    a["self_cc_ranges_flat"] = [v for i, j in pairs for v in (i, j, j, j, i, i)]
+    return a
+
+
+def _self_edges(rob, n, seed, skip, bad=0.0):
+    """The same edges in one plan of at least 65,536 states and in plans below
+    that: (first hits, state verdicts) of either, and the states."""
+    arr, rng = rob.arrays, np.random.default_rng(seed)
+    a = W.uniform_configs(rng, arr, n)
+    b = np.clip(a + rng.uniform(-0.8, 0.8, a.shape), arr.joint_lower, arr.joint_upper).astype(np.float32)
+    b[rng.random(n) < bad, 5] = np.nan
+    ns = rng.integers(20, 64, n).astype(np.int32)
+    ds = S.DeviceScene.from_host(HostScene())
+
+    def run(lo, hi):
+        plan = S.Plan.edges(rob, ns[lo:hi])
+        out = S.edge_check_batched(plan, ds, up(a[lo:hi]), up(b[lo:hi]), check_self=True, skip_resolved=skip,
+                                   state_hits=not skip)
+        return (plan.n_states, *[x.cpu().numpy() for x in ((out,) if skip else out)])
+
+    large, parts = run(0, n), [run(k, min(k + 700, n)) for k in range(0, n, 700)]
+    assert large[0] >= 65536 and all(p[0] < 65536 for p in parts)
+    return large[1:], [np.concatenate(x) for x in list(zip(*parts))[1:]], PO.edge_states(a, b, ns)
+
+
+@pytest.mark.parametrize("skip", [False, True])
+def test_self_pairs_named_twice(skip):
+    """A pair counts once however often it is named: large and small edge sets
+    agree with each other and with the oracle."""
+    rob = S.Robot(_repeated_pairs())
+    large, small, states = _self_edges(rob, 2000, 5, skip)
+    for x, y in zip(large, small):
+        np.testing.assert_array_equal(x, y)
+    if not skip:
+        ref, clr = PO.Oracle(rob.arrays).check_collision(states, check_self=True)
+        assert not np.any((large[1] != ref) & (np.abs(clr) >= 1e-5)) and 0.02 < ref.mean() < 0.6
