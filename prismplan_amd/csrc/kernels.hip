@@ -3460,18 +3460,22 @@ __global__ __launch_bounds__(64) void k_control(const float* theta, const int* t
 // exceeds the smallest (d + L rho) by more than L rho is nowhere the nearest;
 // a few are left, and only they are walked: 17.4 us (20.5 a call). Rounding is covered
 // by a slack of some 1e-6 of the coordinates. Boxes pass through LDS in tiles
-// of 64; a tile's bound takes in the earlier tiles'.
+// of 64; a tile's bound takes in the earlier tiles'. first: the launch's first run
+// (a launch takes fewer than 2^32 threads, and a grid may have more).
 constexpr int kEsdfRun = 4;
+constexpr long kEsdfLaunch = 1L << 25;   // runs of a launch
 
 __global__ __launch_bounds__(64) void k_esdf_build(const float* __restrict__ obb_dims, const float* __restrict__ obb_pose,
                                                    int n_obbs, float4 prm, float4 gp0, float4 gp1, int nx, int ny, int nz,
-                                                   float* __restrict__ out) {
+                                                   long first, float* __restrict__ out) {
     __shared__ float4 s_obb[4 * kWave];
     const float gpose[8] = {gp0.x, gp0.y, gp0.z, gp0.w, gp1.x, gp1.y, gp1.z, gp1.w};
     const int lane = lane_id();
     const int nbz = (nz + 4 * kEsdfRun - 1) / (4 * kEsdfRun), nby = (ny + 3) / 4;
-    const int bz = (int)(blockIdx.x % (unsigned)nbz), bxy = (int)(blockIdx.x / (unsigned)nbz);
-    const int ix = 4 * (bxy / nby) + (lane >> 4), iy = 4 * (bxy % nby) + ((lane >> 2) & 3);
+    const long run = first + blockIdx.x;
+    const long bxy = run / nbz;
+    const int bz = (int)(run - bxy * nbz), bx = (int)(bxy / nby), by = (int)(bxy - (long)bx * nby);
+    const int ix = 4 * bx + (lane >> 4), iy = 4 * by + ((lane >> 2) & 3);
     // node coordinates (may lie past the grid's end: such lanes store nothing)
     auto world = [&](float fx, float fy, float fz, float& px, float& py, float& pz) {
         const float lx = fx * prm.w - 0.5f * prm.x - gpose[0];
@@ -3520,7 +3524,7 @@ __global__ __launch_bounds__(64) void k_esdf_build(const float* __restrict__ obb
             const int z0 = 4 * (bz * kEsdfRun + r);
             if (z0 >= nz) break;
             float px, py, pz, lx, ly, lz;
-            world((float)(4 * (bxy / nby)) + 1.5f, (float)(4 * (bxy % nby)) + 1.5f, (float)z0 + 1.5f, px, py, pz);
+            world((float)(4 * bx) + 1.5f, (float)(4 * by) + 1.5f, (float)z0 + 1.5f, px, py, pz);
             to_box(rec[0], rec[1], rec[2], px, py, pz, lx, ly, lz);
             const float d = key_to_sdf(box_key(lx, ly, lz, rec[3]));
             const float slack = 1e-5f + 4e-6f * (mag + lip * (fabsf(px) + fabsf(py) + fabsf(pz)));
@@ -3909,12 +3913,12 @@ hipError_t launch_esdf_build(const float* obb_dims, const float* obb_pose, int n
     };
     const int nx = rf(voxel_params[0] * inv) + 1, ny = rf(voxel_params[1] * inv) + 1, nz = rf(voxel_params[2] * inv) + 1;
     if (nx <= 0 || ny <= 0 || nz <= 0) return hipSuccess;
-    const long blocks = (long)((nx + 3) / 4) * ((ny + 3) / 4) * ((nz + 4 * kEsdfRun - 1) / (4 * kEsdfRun));
-    if (blocks > INT_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_esdf_build, dim3((unsigned)blocks), dim3(64), 0, s, obb_dims, obb_pose, n_obbs,
-                       make_float4(voxel_params[0], voxel_params[1], voxel_params[2], voxel_params[3]),
-                       make_float4(voxel_pose[0], voxel_pose[1], voxel_pose[2], voxel_pose[3]),
-                       make_float4(voxel_pose[4], voxel_pose[5], voxel_pose[6], voxel_pose[7]), nx, ny, nz, out);
+    const long runs = (((long)nx + 3) / 4) * (((long)ny + 3) / 4) * (((long)nz + 4 * kEsdfRun - 1) / (4 * kEsdfRun));
+    for (long first = 0; first < runs; first += kEsdfLaunch)
+        hipLaunchKernelGGL(k_esdf_build, dim3((unsigned)std::min(kEsdfLaunch, runs - first)), dim3(64), 0, s, obb_dims,
+                           obb_pose, n_obbs, make_float4(voxel_params[0], voxel_params[1], voxel_params[2], voxel_params[3]),
+                           make_float4(voxel_pose[0], voxel_pose[1], voxel_pose[2], voxel_pose[3]),
+                           make_float4(voxel_pose[4], voxel_pose[5], voxel_pose[6], voxel_pose[7]), nx, ny, nz, first, out);
     return hipGetLastError();
 }
 

@@ -189,3 +189,29 @@ def test_self_pairs_named_twice(skip):
     if not skip:
         ref, clr = PO.Oracle(rob.arrays).check_collision(states, check_self=True)
         assert not np.any((large[1] != ref) & (np.abs(clr) >= 1e-5)) and 0.02 < ref.mean() < 0.6
+
+
+def test_esdf_grid_of_2_to_the_30_nodes():
+    """A wide flat grid has more 64-lane workgroups than one launch takes: every
+    node up to the last has its value."""
+    n, voxel = 32768, 1.0 / 128
+    box = HostScene.from_boxes(np.array([[3.0, 40.0, 2.0], [5.0, 5.0, 5.0]]),
+                               np.array([[10.0, -20.0, 0.5], [-127.0, 125.0, 0.0]]),
+                               np.array([[1.0, 0.0, 0.0, 0.0], [0.8, 0.0, 0.0, 0.6]]))
+    prm = np.array([voxel * (n - 1), voxel * (n - 1), 0.0, voxel], np.float32)
+    pose = np.array([0, 0, 0, 1, 0, 0, 0, 0], np.float32)
+    got = S.esdf_from_obbs(S.DeviceScene.from_host(box), prm, pose)
+    assert got.numel() == n * n
+    k = np.unique(np.concatenate([np.random.default_rng(0).integers(0, n * n, 20000), [0, n - 1, n * n - n, n * n - 1]]))
+    ix, iy = k // n, k % n
+    p = np.stack([ix * voxel - 0.5 * float(prm[0]), iy * voxel - 0.5 * float(prm[1]), 0.0 * ix], 1)
+    d = np.min([_box_distance(box, b, p) for b in range(2)], axis=0)
+    # coordinates up to 128 m: FP32 resolves 1.5e-5 m there, the map to a box sums three such products
+    assert np.abs(got[torch.from_numpy(k).to(DEV)].cpu().numpy() + d).max() < 2e-4
+
+
+def _box_distance(scene, b, p):
+    t, w, u = scene.obb_pose[b, :3].astype(float), float(scene.obb_pose[b, 3]), scene.obb_pose[b, 4:7].astype(float)
+    s = 2.0 * np.cross(u, p)
+    e = np.abs(p + w * s + np.cross(u, s) + t) - 0.5 * scene.obb_dims[b, :3]
+    return np.linalg.norm(np.maximum(e, 0.0), axis=1) + np.minimum(e.max(1), 0.0)
