@@ -3912,7 +3912,7 @@ hipError_t launch_esdf_build(const float* obb_dims, const float* obb_pose, int n
         return (int)nearest;
     };
     const int nx = rf(voxel_params[0] * inv) + 1, ny = rf(voxel_params[1] * inv) + 1, nz = rf(voxel_params[2] * inv) + 1;
-    if (nx <= 0 || ny <= 0 || nz <= 0) return hipSuccess;
+    if (nx <= 0 || ny <= 0 || nz <= 0) return hipErrorInvalidValue;   // no nodes
     const long runs = (((long)nx + 3) / 4) * (((long)ny + 3) / 4) * (((long)nz + 4 * kEsdfRun - 1) / (4 * kEsdfRun));
     for (long first = 0; first < runs; first += kEsdfLaunch)
         hipLaunchKernelGGL(k_esdf_build, dim3((unsigned)std::min(kEsdfLaunch, runs - first)), dim3(64), 0, s, obb_dims,
