@@ -2655,6 +2655,7 @@ __global__ __launch_bounds__(64, 4) void k_self_far(SelfArgs a) {
 #pragma unroll
                     for (int k = 0; k < 12; ++k) P[k] = T[k];
                 } else {
+                    __syncthreads();   // another lane of the state stored it
                     const float* Tp = s_T + 12 * (par * kN + slot);
 #pragma unroll
                     for (int k = 0; k < 12; ++k) P[k] = Tp[k];

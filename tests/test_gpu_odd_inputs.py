@@ -215,3 +215,61 @@ def _box_distance(scene, b, p):
     s = 2.0 * np.cross(u, p)
     e = np.abs(p + w * s + np.cross(u, s) + t) - 0.5 * scene.obb_dims[b, :3]
     return np.linalg.norm(np.maximum(e, 0.0), axis=1) + np.minimum(e.max(1), 0.0)
+
+
+def _branched():
+    """Panda with link 5 hung on link 3: not a line of joints."""
+    a = load_robot_asset("panda")
+    a["joint_parents"] = [0, 0, 1, 2, 3, 3, 5, 6]
+    a["t_memory_idx"] = [0, 1, 1, 1, 0, 1, 1, 1]
+    return a
+
+
+@pytest.mark.parametrize("skip", [False, True])
+def test_rough_self_pass_of_a_tree(skip):
+    """A joint whose parent is neither the root nor the joint before it: its
+    parent's frame is read back from LDS. Large and small edge sets agree, and
+    both with the oracle."""
+    rob = S.Robot(_branched())
+    large, small, states = _self_edges(rob, 2000, 8, skip)
+    for x, y in zip(large, small):
+        np.testing.assert_array_equal(x, y)
+    if not skip:
+        ref, clr = PO.Oracle(rob.arrays).check_collision(states, check_self=True)
+        assert not np.any((large[1] != ref) & (np.abs(clr) >= 1e-5)) and 0.005 < ref.mean() < 0.9
+
+
+def _solved(rob, ds, theta, T, step):
+    """Validity of each of len(theta) trajectories of T waypoints, in one call."""
+    plan = S.Plan.trajectories(rob, np.full(len(theta), T))
+    opt = S.ChompOptimizer(plan, ds, up(theta.reshape(-1)), S.chomp_settings(collision_check_step=step)).step(0)
+    return opt.solved().cpu().numpy()
+
+
+@pytest.mark.parametrize("name,boxes", [("panda", 3), ("branched", 3), ("panda", 0)])
+def test_densified_validity_alone_and_in_a_batch(name, boxes):
+    """Forty trajectories at once take the two-step self pass over up to 600,000
+    densified states, one alone the exact pass: the same verdicts."""
+    rob = S.Robot(_branched() if name == "branched" else name)
+    w = W.chomp(n_traj=40, n_wp=64, n_obbs=max(boxes, 1), seed=3 + boxes)
+    ds = S.DeviceScene.from_host(w.scene if boxes else HostScene())
+    theta = w.theta.reshape(40, -1)
+    batch = _solved(rob, ds, theta, 64, 0.05)
+    np.testing.assert_array_equal(batch, np.concatenate([_solved(rob, ds, theta[k:k + 1], 64, 0.05) for k in range(40)]))
+    assert 0 < batch.sum() < 40
+
+
+@pytest.mark.parametrize("n", [1, 2, 4, 5, 63, 65, 1100])
+def test_spread_visit_reaches_every_chunk(n):
+    """64 waypoints a trajectory and one state a segment: n chunks of 64 states,
+    one to a trajectory, visited in spread order. Chunk counts of one, powers of
+    two and one past and short of them; 1,100 take the two-step self pass."""
+    rob = S.Robot("panda")
+    w = W.chomp(n_traj=n, n_wp=64, n_obbs=3, seed=n)
+    got = _solved(rob, S.DeviceScene.from_host(w.scene), w.theta.reshape(n, -1), 64, 100.0)
+    D = rob.n_dof
+    q = w.theta.reshape(n, D, 64).transpose(0, 2, 1).reshape(-1, D)
+    hit, clr = PO.Oracle(rob.arrays, w.scene, nthreads=8).check_collision(q, check_self=True)
+    sure = ~(np.abs(clr) < 1e-5).reshape(n, 64).any(1)
+    np.testing.assert_array_equal(got[sure], ~hit.reshape(n, 64).any(1)[sure])
+    assert n < 60 or 0.02 < got.mean() < 0.98
