@@ -2641,6 +2641,7 @@ __global__ __launch_bounds__(64, 4) void k_self_far(SelfArgs a) {
         }
         __syncthreads();
         float T[12];
+        float far_at = 0.0f;   // the joint farthest from the origin
         for (int jj = 0; jj < J; ++jj) {
             const i4u meta = uload<i4u>(R.jmeta, jj);
             float* Tj = s_T + 12 * (jj * kN + slot);
@@ -2664,6 +2665,7 @@ __global__ __launch_bounds__(64, 4) void k_self_far(SelfArgs a) {
                 joint_step_u(R.ft, jj, meta.x, meta.y >= 0 ? s_q[meta.y * kN + slot] : 0.0f, sc.x, sc.y, A);
                 aff_compose(P, A, T);
             }
+            far_at = max_nan(far_at, fabsf(T[3]) + fabsf(T[7]) + fabsf(T[11]));
             if (sub == (jj & (G - 1))) {
                 float4* d = reinterpret_cast<float4*>(Tj);
                 d[0] = make_float4(T[0], T[1], T[2], T[3]);
@@ -2680,12 +2682,15 @@ __global__ __launch_bounds__(64, 4) void k_self_far(SelfArgs a) {
             }
         }
         __syncthreads();
-        const float far_t = 2e-6f * (fabsf(T[3]) + fabsf(T[7]) + fabsf(T[11]));   // a base moved far off its limits
-        const float slack = R.far_slack + far_t;
+        // A joint far off its limits adds its place's rounding. The proofs need a
+        // slack below the radii: a place beyond that, or that is no number, is
+        // left to the exact pass.
+        const float slack = R.far_slack + 4e-6f * far_at;
+        const bool lost = !(slack <= R.far_rmax);
         float open = 1.0f, sure = 1.0f;   // smallest margins: open < 0 not proven clear, sure < 0 proven hit
         for (int b0 = 0; b0 < R.n_cpb; b0 += G) {
             const int bb = b0 + sub;
-            bool near = active && bb < R.n_cpb;
+            bool near = active && !lost && bb < R.n_cpb;
             if (near) {
                 const int ids = s_gate[bb], cA = ids & 0xFFFF, cB = ids >> 16;
                 const float* p = s_cen + 3 * cA * kN + slot;
@@ -2765,8 +2770,8 @@ __global__ __launch_bounds__(64, 4) void k_self_far(SelfArgs a) {
             open = fminf(open, __shfl_xor(open, o));
             sure = fminf(sure, __shfl_xor(sure, o));
         }
-        const bool is_hit = active && sure < 0.0f;
-        const bool is_open = active && open < 0.0f && !is_hit;
+        const bool is_hit = active && sure < 0.0f && !lost;
+        const bool is_open = active && (open < 0.0f || lost) && !is_hit;
         if (active && sub == 0 && !is_open) {
             if (!a.unit_first_hit) a.hit_out[ref.gs] = is_hit ? 1 : 0;
             else if (is_hit) atomicMin((unsigned*)&a.unit_first_hit[ref.unit], (unsigned)ref.k);

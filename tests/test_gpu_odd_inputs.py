@@ -157,13 +157,15 @@ def _repeated_pairs():
     return a
 
 
-def _self_edges(rob, n, seed, skip, bad=0.0):
+def _self_edges(rob, n, seed, skip, change=None):
     """The same edges in one plan of at least 65,536 states and in plans below
-    that: (first hits, state verdicts) of either, and the states."""
+    that: (first hits, state verdicts) of either, and the states. change: applied
+    to the edges' ends (start, end, random numbers)."""
     arr, rng = rob.arrays, np.random.default_rng(seed)
     a = W.uniform_configs(rng, arr, n)
     b = np.clip(a + rng.uniform(-0.8, 0.8, a.shape), arr.joint_lower, arr.joint_upper).astype(np.float32)
-    b[rng.random(n) < bad, 5] = np.nan
+    if change:
+        change(a, b, rng)
     ns = rng.integers(20, 64, n).astype(np.int32)
     ds = S.DeviceScene.from_host(HostScene())
 
@@ -273,3 +275,39 @@ def test_spread_visit_reaches_every_chunk(n):
     sure = ~(np.abs(clr) < 1e-5).reshape(n, 64).any(1)
     np.testing.assert_array_equal(got[sure], ~hit.reshape(n, 64).any(1)[sure])
     assert n < 60 or 0.02 < got.mean() < 0.98
+
+
+@pytest.mark.parametrize("skip", [False, True])
+def test_self_check_of_edges_without_an_end(skip):
+    """Edges with a NaN joint in the middle of the arm: the finite links' pairs
+    decide, in large edge sets as in small ones."""
+    rob = S.Robot("panda")
+
+    def change(a, b, rng):
+        b[rng.random(len(b)) < 0.3, 5] = np.nan
+
+    large, small, states = _self_edges(rob, 2000, 6, skip, change)
+    for x, y in zip(large, small):
+        np.testing.assert_array_equal(x, y)
+    if not skip:
+        bad = np.isnan(states).any(1)
+        assert large[1][bad].mean() > 0.001 and large[1][~bad].mean() > 0.02
+
+
+@pytest.mark.parametrize("place", [300.0, 3e5, 1e30])
+def test_self_check_far_off_the_limits(place):
+    """A base rail run far off its limits, where FP32 resolves a sphere's place
+    by less and less: the rough pass leaves to the exact one what it cannot
+    prove there."""
+    a = load_robot_asset("panda")
+    a["joint_types"] = [3, 0] + a["joint_types"][2:]
+    rob = S.Robot(a)
+
+    def change(a, b, rng):
+        a[rng.random(len(a)) < 0.5, 0] = place
+        b[:, 0] = a[:, 0]
+
+    large, small, _ = _self_edges(rob, 2000, 7, False, change)
+    for x, y in zip(large, small):
+        np.testing.assert_array_equal(x, y)
+    assert 0.01 < large[1].mean() < 0.99
