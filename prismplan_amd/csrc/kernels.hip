@@ -461,7 +461,7 @@ struct EsdfTap {
         const float c = -d - r;
         return c < 1000.0f ? c : 1000.0f;
     }
-    // d dist / d p (world) where value() came from the grid
+    // d dist / d p (world); only where value() is below its 1000
     __device__ __forceinline__ void grad(const EsdfLayer& L, float& gx, float& gy, float& gz) const {
         const float c00 = fmaf(c100 - c000, fx, c000), c01 = fmaf(c101 - c001, fx, c001);
         const float c10 = fmaf(c110 - c010, fx, c010), c11 = fmaf(c111 - c011, fx, c011);
@@ -1285,10 +1285,10 @@ __device__ __forceinline__ float sphere_hinge_at(const CostArgs& a, const EsdfLa
         if (ONE) {
             EsdfTap t;
             t.load(layer, px, py, pz, true);
-            const float hh = m - t.value(r);
+            const float c = t.value(r), hh = m - c;
             if (hh > 0.0f) {
                 world += hh;
-                if (GRAD && t.ok) {
+                if (GRAD && c < 1000.0f) {   // 1000: not from the grid, no gradient
                     t.grad(layer, dx, dy, dz);
                     gx += dx; gy += dy; gz += dz;
                 }

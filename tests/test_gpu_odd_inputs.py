@@ -311,3 +311,29 @@ def test_self_check_far_off_the_limits(place):
     for x, y in zip(large, small):
         np.testing.assert_array_equal(x, y)
     assert 0.01 < large[1].mean() < 0.99
+
+
+@pytest.mark.parametrize("name", ["panda", "baxter"])
+def test_unobserved_grid_has_no_gradient(name):
+    """A margin above the 1000 m of a sphere that no grid value applies to
+    (outside, or beside an unobserved node): the hinge is margin - 1000 and has
+    no gradient. The single-layer lookups equal the general ones, which a mask
+    that masks nothing selects."""
+    rob = S.Robot(name)
+    arr, rng, n = rob.arrays, np.random.default_rng(9), 300
+    prm, pose = W.esdf_grid(center=(0.5, 0.0, 0.5), n=48, voxel=0.03)
+    src = W.random_obbs(rng, 8, half_hi=0.15)
+    vals = PO.esdf_from_obbs(src.obb_dims, src.obb_pose, prm, pose).astype(np.float32).reshape(-1)
+    vals[rng.random(vals.size) < 0.05] = -1000.0
+    hs = lambda acm: HostScene(voxel_params=prm, voxel_pose=pose, voxel_enable=np.ones(1, np.uint8),
+                               voxel_features=vals.reshape(1, -1), esdf_interp=1, sphere_acm=acm)
+    q = up(W.uniform_configs(rng, arr, n))
+    cp = S.cost_params(world_margin=1001.0, weight=1.0, use_self=False, use_obb=False)
+    out = []
+    for acm in (None, np.ones((arr.n_spheres, 1), np.uint8)):
+        c, _, g = S.hinge_cost(S.Plan.configs(rob, n), S.DeviceScene.from_host(hs(acm)), q, cp, grad=True)
+        out.append((c.cpu().numpy(), g.cpu().numpy()))
+    np.testing.assert_allclose(out[0][0], out[1][0], rtol=5e-6)   # sums of up to 75 FP32 terms
+    # sums of unit point gradients times arms of metres, over the model's spheres
+    np.testing.assert_allclose(out[0][1], out[1][1], rtol=0, atol=1e-5 * arr.n_spheres)
+    assert np.abs(out[0][1]).max() > 0.1
