@@ -42,13 +42,15 @@ __device__ __forceinline__ float uniform(float v) {
 // into SGPRs. A plain read after a barrier or an LDS write is a vector load
 // per lane instead, since the compiler cannot tell that the table stays.
 typedef float f4u __attribute__((ext_vector_type(4)));
+typedef float f4s __attribute__((ext_vector_type(4), aligned(4)));   // of a caller's floats, which lie at any float
 typedef int i4u __attribute__((ext_vector_type(4)));
 template <typename T>
 __device__ __forceinline__ T uload(const void* p, int i) {
     return reinterpret_cast<const __attribute__((address_space(4))) T*>(reinterpret_cast<uintptr_t>(p))[i];
 }
+template <typename V = f4u>
 __device__ __forceinline__ float4 uload4(const void* p, int i) {
-    const f4u v = uload<f4u>(p, i);
+    const V v = uload<V>(p, i);
     return make_float4(v.x, v.y, v.z, v.w);
 }
 
@@ -418,7 +420,7 @@ struct EsdfLayer {
     const float* feat;
     EsdfLayer() = default;
     __device__ __forceinline__ explicit EsdfLayer(const DScene& S)
-        : prm(uload4(S.voxel_params, 0)), p0(uload4(S.voxel_pose, 0)), p1(uload4(S.voxel_pose, 1)) {
+        : prm(uload4<f4s>(S.voxel_params, 0)), p0(uload4<f4s>(S.voxel_pose, 0)), p1(uload4<f4s>(S.voxel_pose, 1)) {
         on = S.voxel_enable[0] != 0 && prm.w > 0.0f;
         inv_vs = uniform(1.0f / prm.w);
         nx = uniform(robust_floor(prm.x * inv_vs) + 1);

@@ -337,3 +337,22 @@ def test_unobserved_grid_has_no_gradient(name):
     # sums of unit point gradients times arms of metres, over the model's spheres
     np.testing.assert_allclose(out[0][1], out[1][1], rtol=0, atol=1e-5 * arr.n_spheres)
     assert np.abs(out[0][1]).max() > 0.1
+
+
+def test_grid_parameters_at_any_float():
+    """Layer parameters and pose need no more than a float's alignment."""
+    rob, n = S.Robot("panda"), 200
+    rng = np.random.default_rng(10)
+    prm, pose = W.esdf_grid(center=(0.5, 0.0, 0.5), n=48, voxel=0.03)
+    vals = up(rng.normal(0, 0.2, 48 ** 3).astype(np.float32))
+    one = torch.ones(1, dtype=torch.uint8, device=DEV)
+    q, plan, out = up(W.uniform_configs(rng, rob.arrays, n)), S.Plan.configs(rob, n), []
+    for shift in (0, 1, 3):
+        at = lambda a: up(np.concatenate([np.zeros(shift, np.float32), a.reshape(-1)]))[shift:].reshape(a.shape)
+        ds = S.DeviceScene(None, None, None, at(prm), at(pose), one, vals, esdf_interp=1)
+        assert ds.view().voxel_params is not None and at(prm).data_ptr() % 16 == 4 * shift
+        out.append((S.min_clearance_batched(plan, ds, q).cpu().numpy(),
+                    S.hinge_cost(plan, ds, q, S.cost_params(use_self=False), grad=True)[2].cpu().numpy()))
+    for x in out[1:]:
+        np.testing.assert_array_equal(x[0], out[0][0])
+        np.testing.assert_array_equal(x[1], out[0][1])
