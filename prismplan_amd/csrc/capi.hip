@@ -419,14 +419,20 @@ std::string hex64(unsigned long long v) {
     return b;
 }
 
+// Revision of the kernels that the choices were timed on, a part of the keys:
+// entries of another one are left alone and not taken. Raised when a tuned kernel
+// or the meaning of a choice changes (k2: k_collide with candidates by rows and
+// grid form 0 at kCollideWaves, k_state_cost, wrenches without atomics).
+constexpr const char* kTuneRev = "k2/";
+
 std::string collide_key(const ppl_robot_s* r, int max_obbs) {
-    return "collide/" + hex64(r->digest) + "/" + std::to_string(max_obbs) + "/" + gpu_arch();
+    return std::string("collide/") + kTuneRev + hex64(r->digest) + "/" + std::to_string(max_obbs) + "/" + gpu_arch();
 }
 
 std::string cost_key(const ppl_robot_s* r, bool grad, int max_obbs, long n_states) {
     int lg = 0;
     while ((1L << (lg + 1)) <= n_states) ++lg;
-    return std::string(grad ? "adjoint/" : "cost/") + hex64(r->digest) + "/" + std::to_string(max_obbs) + "/" +
+    return std::string(grad ? "adjoint/" : "cost/") + kTuneRev + hex64(r->digest) + "/" + std::to_string(max_obbs) + "/" +
            std::to_string(lg) + "/" + gpu_arch();
 }
 

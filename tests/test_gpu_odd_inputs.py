@@ -356,3 +356,26 @@ def test_grid_parameters_at_any_float():
     for x in out[1:]:
         np.testing.assert_array_equal(x[0], out[0][0])
         np.testing.assert_array_equal(x[1], out[0][1])
+
+
+def test_tuning_entries_of_other_kernels_are_not_taken(tmp_path):
+    """A cache file written for earlier kernels (keys without their revision)
+    leaves the built-in shapes."""
+    path = tmp_path / "tune.txt"
+    S.tune_cache_file(path)
+    try:
+        rob, n = S.Robot("panda"), 4000
+        rng = np.random.default_rng(2)
+        ds = S.DeviceScene.from_host(W.random_obbs(rng, 64))
+        q = up(W.uniform_configs(rng, rob.arrays, n))
+        S.Plan.configs(rob, n).autotune_collide(ds, q, reps=2)
+        assert S.Plan.configs(rob, n).collide_shape(64)[2] == 1
+        lines = path.read_text().splitlines()
+        old = ["/".join(w for w in l.split()[0].split("/") if not w.startswith("k")) + " 32 2 0.001" for l in lines
+               if l.startswith("collide/")]
+        assert old
+        path.write_text("\n".join(old) + "\n")
+        S.tune_cache_file(path)
+        assert S.Plan.configs(rob, n).collide_shape(64) == (64, 0, 0)
+    finally:
+        S.tune_cache_file("")
