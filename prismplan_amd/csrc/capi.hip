@@ -253,11 +253,11 @@ int grid_for(KernelKind k, const DRobot& R, int obb_cap, int G) {
     return (grad ? 1 : kCostWaves) * grid_cost(R, grad, lds_bytes_cost(obb_cap, R.n_dof, R.n_joints, G, grad));
 }
 
-// max_obbs: OBBs of the largest problem of the launch.
-DChunks implicit_chunks(long n_states, int grid_cap, int max_obbs, int* grid_out, int G = 1) {
+// max_obbs: OBBs of the largest problem of the launch; tile: records a staging holds.
+DChunks implicit_chunks(long n_states, int grid_cap, int max_obbs, int tile, int* grid_out, int G = 1) {
     DChunks C{};
-    C.obb_cap = obb_tile(max_obbs);
-    C.tiled = max_obbs > kMaxObbLds;
+    C.obb_cap = tile;
+    C.tiled = max_obbs > tile;
     C.tab = nullptr;
     C.chunk = kWave / G;
     C.n_chunks = (int)((n_states + C.chunk - 1) / C.chunk);
@@ -274,11 +274,30 @@ DChunks implicit_chunks(long n_states, int grid_cap, int max_obbs, int* grid_out
 // one workgroup per chunk there).
 constexpr int kCollideWaves = 8;
 
+// OBB records that an any-collision launch of n_states states stages at a time.
+// All of a problem's, up to kMaxObbLds, take so much LDS from about 190 on that
+// fewer than eight workgroups fit a CU, two waves a SIMD; a launch of more waves
+// than then fit the chip stages tiles of 128 instead and walks the joints once a
+// tile. 2,000 edges (100,000 configurations), us a call in one staging and in
+// tiles: Fetch 170 boxes 300 and 304 (313, 315), 200 436 and 338 (351, 348), 256
+// 592 and 424 (748, 423), 300 684 and 506 (864, 482); Baxter 170 323 and 332 (370,
+// 368), 200 465 and 377 (420, 413), 300 687 and 543 (1,034, 583); Panda 200 148 and 152
+// (144, 151), 256 197 and 179 (269, 182). 4,000 configurations fit at once: Panda 300
+// boxes 70 and 75, Baxter 172 and 174.
+constexpr int kCollideTile = 128;
+constexpr size_t kLdsPerCu = 160 * 1024;
+int collide_tile(const DRobot& R, long n_states, int max_obbs, int lanes) {
+    const int t = obb_tile(max_obbs);
+    if (!R.scene_gate_fused || t <= kCollideTile) return t;
+    const long fit = (long)(kLdsPerCu / lds_bytes_collide(t, R));
+    return fit < 8 && n_states * lanes > fit * device_cus() * kWave ? kCollideTile : t;
+}
+
 // Implicit chunks of an any-collision launch over a whole scene. n_states an
 // upper bound (counted on the device): the grid stays at what the chip holds.
 DChunks collide_chunks(long n_states, const DRobot& R, const DScene& S, int* grid_out, bool bound = false) {
-    return implicit_chunks(n_states, (bound ? 1 : kCollideWaves) * grid_collide(R, S, obb_tile(S.n_obbs)), S.n_obbs,
-                           grid_out, bound ? 1 : collide_lanes(R, n_states));
+    const int lanes = bound ? 1 : collide_lanes(R, n_states), tile = collide_tile(R, n_states, S.n_obbs, lanes);
+    return implicit_chunks(n_states, (bound ? 1 : kCollideWaves) * grid_collide(R, S, tile), S.n_obbs, tile, grid_out, lanes);
 }
 
 // The cost kernel over n_states implicit chunks: k_state_cost or k_cost_grad with one lane per
@@ -320,7 +339,8 @@ hipError_t launch_cost_flat(CostArgs& a, long n_states, hipStream_t s) {
     const bool tiled = a.S.n_obbs > kMaxObbLds;
     const KernelKind k = tiled ? (a.grad ? kKCostGrpGrad : kKCostGrp) : (a.grad ? kKCostGrad : kKCost);
     const int G = tiled ? kGrp : 1;
-    a.C = implicit_chunks(n_states, grid_for(k, a.R, obb_tile(a.S.n_obbs), G), a.S.n_obbs, &grid, G);
+    const int tile = obb_tile(a.S.n_obbs);
+    a.C = implicit_chunks(n_states, grid_for(k, a.R, tile, G), a.S.n_obbs, tile, &grid, G);
     a.group = tiled ? kGrp : 1;
     return tiled ? launch_cost_grp(a, grid, s) : launch_cost(a, grid, s);
 }
@@ -477,8 +497,7 @@ DChunks plan_chunks(const ppl_plan_s* P, KernelKind k, int max_obbs, int G, int*
 
 // The any-collision launch shape of plan P for problems of up to max_obbs
 // OBBs: this plan's tuned or set shape, else the tuning cache's entry for the
-// robot, OBB count and GPU, else the built-in one (every OBB of a problem in
-// one staging, grid form 0). tile: OBB records per LDS staging; gmode 0 up to
+// robot, OBB count and GPU, else the built-in one (collide_tile, grid form 0). tile: OBB records per LDS staging; gmode 0 up to
 // kCollideWaves times the workgroups the chip holds at once, 1 twice them, 2
 // one workgroup per chunk.
 void collide_shape(ppl_plan_s* P, int max_obbs, int* tile, int* gmode) {
@@ -494,7 +513,10 @@ void collide_shape(ppl_plan_s* P, int max_obbs, int* tile, int* gmode) {
             P->shape_src = 1;
         }
     }
-    *tile = P->ctile > 0 ? std::min(P->ctile, obb_tile(max_obbs)) : obb_tile(max_obbs);
+    const DRobot& R = P->robot->R;
+    *tile = P->ctile > 0        ? std::min(P->ctile, obb_tile(max_obbs))
+            : P->shape_src == 0 ? collide_tile(R, P->n_states, max_obbs, collide_lanes(R, P->n_states))
+                                : obb_tile(max_obbs);
     *gmode = P->cgrid;
 }
 
@@ -2978,7 +3000,7 @@ ppl_status ppl_plan_autotune_collide(ppl_plan P, const ppl_scene_view* view, con
         P->ctile = keep_tile; P->cgrid = keep_grid; P->shape_src = keep_src; P->shape_obbs = keep_obbs;
         return st;
     }
-    // the whole-problem tile is stored as 0 (the built-in choice for any OBB count)
+    // the whole-problem tile is stored as 0
     P->ctile = bt == tiles[0] ? 0 : bt;
     P->cgrid = bg;
     P->shape_src = 2;

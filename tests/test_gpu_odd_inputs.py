@@ -379,3 +379,26 @@ def test_tuning_entries_of_other_kernels_are_not_taken(tmp_path):
         assert S.Plan.configs(rob, n).collide_shape(64) == (64, 0, 0)
     finally:
         S.tune_cache_file("")
+
+
+@pytest.mark.parametrize("name,boxes,tile", [("panda", 212, 212), ("panda", 213, 128), ("baxter", 187, 128),
+                                             ("fetch", 256, 128), ("branched", 300, 128)])
+def test_many_boxes_pass_in_tiles(name, boxes, tile):
+    """Past some 190 boxes (212 of Panda's, 186 of Baxter's) a launch of more waves than then fit the chip stages
+    128 at a time, a small one all of them (up to 256): verdicts and first hits
+    are those of any tile."""
+    rob = S.Robot(_branched() if name == "branched" else name)
+    arr, rng = rob.arrays, np.random.default_rng(boxes)
+    ds = S.DeviceScene.from_host(W.random_obbs(rng, boxes, (0.5, -0.9, 0.3), (1.3, 0.9, 1.5), half_hi=0.04))
+    a = W.uniform_configs(rng, arr, 3000)
+    b = np.clip(a + rng.uniform(-0.6, 0.6, a.shape), arr.joint_lower, arr.joint_upper).astype(np.float32)
+    ns = rng.integers(20, 80, len(a)).astype(np.int32)
+    big, small = S.Plan.edges(rob, ns), S.Plan.edges(rob, ns[:300])
+    assert small.collide_shape(boxes) == (min(boxes, 256), 0, 0) and small.collide_shape(128)[0] == 128
+    assert big.collide_shape(boxes) == (tile, 0, 0) and big.collide_shape(170)[0] == 170
+    x = S.edge_check_batched(big, ds, up(a), up(b)).cpu().numpy()
+    y = S.edge_check_batched(small, ds, up(a[:300]), up(b[:300])).cpu().numpy()
+    np.testing.assert_array_equal(x[:300], y)
+    big.set_collide_shape(96, 0)
+    np.testing.assert_array_equal(x, S.edge_check_batched(big, ds, up(a), up(b)).cpu().numpy())
+    assert 0.02 < (x >= 0).mean() < 0.98
