@@ -168,6 +168,7 @@ struct ppl_plan_s {
     int* d_off = nullptr;            // [n_units+1]
     std::vector<long> pb, pe;        // state range of each problem
     int4* d_tab[kGroupKinds] = {};   // chunk tables for 64, 32, 16, 8, 4, 2 states
+    int tab_in_first = -1;           // the table, if any, that lies in the first one's allocation
     int n_chunks[kGroupKinds] = {};
     int* d_obb_off = nullptr;
     int wmajor = 0;                  // waypoint-major trajectory plan
@@ -458,13 +459,10 @@ std::string cost_key(const ppl_robot_s* r, bool grad, int max_obbs, long n_state
 
 int group_index(int G) { return G >= 32 ? 5 : G >= 16 ? 4 : G >= 8 ? 3 : G >= 4 ? 2 : G >= 2 ? 1 : 0; }
 
-// Chunk table of a plan for `G` lanes per state (64 / G states per chunk),
-// built on first use; chunks never cross a problem boundary.
-hipError_t ensure_table(ppl_plan_s* P, int G) {
-    const int gi = group_index(G);
-    if (P->d_tab[gi] || P->n_states == 0) return hipSuccess;
+// Appends the chunk table of a plan for `G` lanes per state (64 / G states per
+// chunk); chunks never cross a problem boundary.
+void chunk_table(const ppl_plan_s* P, int G, std::vector<int4>& tab) {
     const long chunk = kWave / G;
-    std::vector<int4> tab;
     // w = the unit (edge / trajectory) holding the chunk's first state
     for (size_t p = 0; p < P->pb.size(); ++p)
         for (long s = P->pb[p]; s < P->pe[p]; s += chunk) {
@@ -474,10 +472,39 @@ hipError_t ensure_table(ppl_plan_s* P, int G) {
                 u = (int)(std::upper_bound(P->h_off.begin(), P->h_off.end(), (int)s) - P->h_off.begin()) - 1;
             tab.push_back(make_int4((int)p, (int)s, (int)std::min(s + chunk, P->pe[p]), u));
         }
+}
+
+// A plan's chunk table for `G` lanes per state, built on first use.
+hipError_t ensure_table(ppl_plan_s* P, int G) {
+    const int gi = group_index(G);
+    if (P->d_tab[gi] || P->n_states == 0) return hipSuccess;
+    std::vector<int4> tab;
+    chunk_table(P, G, tab);
     if (tab.empty()) return hipSuccess;
     hipError_t e = hipMalloc((void**)&P->d_tab[gi], tab.size() * sizeof(int4));
     if (e == hipSuccess) e = hipMemcpy(P->d_tab[gi], tab.data(), tab.size() * sizeof(int4), hipMemcpyHostToDevice);
     if (e == hipSuccess) P->n_chunks[gi] = (int)tab.size();
+    return e;
+}
+
+// The tables made with a plan: for one lane per state and, where the
+// any-collision pass takes it, for collide_lanes; in one allocation and copy (two
+// of each took 13 us of the 54 of a small plan).
+hipError_t first_tables(ppl_plan_s* P) {
+    const int lanes = P->kind == PPL_PLAN_TRAJ ? 1 : collide_lanes(P->robot->R, P->n_states);
+    if (lanes == 1 || P->n_states == 0) return ensure_table(P, 1);
+    std::vector<int4> tab;
+    chunk_table(P, 1, tab);
+    const size_t n1 = tab.size();
+    chunk_table(P, lanes, tab);
+    hipError_t e = hipMalloc((void**)&P->d_tab[0], tab.size() * sizeof(int4));
+    if (e == hipSuccess) e = hipMemcpy(P->d_tab[0], tab.data(), tab.size() * sizeof(int4), hipMemcpyHostToDevice);
+    if (e != hipSuccess) return e;
+    const int gi = group_index(lanes);
+    P->d_tab[gi] = P->d_tab[0] + n1;
+    P->tab_in_first = gi;
+    P->n_chunks[0] = (int)n1;
+    P->n_chunks[gi] = (int)(tab.size() - n1);
     return e;
 }
 
@@ -1512,8 +1539,7 @@ ppl_status ppl_plan_create(ppl_robot r, const ppl_plan_desc* d, ppl_plan* out) t
     P->h_off.assign(uoff.size(), 0);
     for (size_t i = 0; i < uoff.size(); ++i) P->h_off[i] = (int)uoff[i];
     for (size_t i = 0; i + 1 < uoff.size(); ++i) P->t_max = std::max(P->t_max, (int)(uoff[i + 1] - uoff[i]));
-    hipError_t e = ensure_table(P, 1);
-    if (e == hipSuccess) e = ensure_table(P, collide_lanes(P->robot->R, P->n_states));   // the any-collision pass's
+    hipError_t e = first_tables(P);
     if (e == hipSuccess && !prob.empty()) {
         e = hipMalloc((void**)&P->d_prob, prob.size() * sizeof(int4));
         if (e == hipSuccess) e = hipMemcpy(P->d_prob, prob.data(), prob.size() * sizeof(int4), hipMemcpyHostToDevice);
@@ -1539,7 +1565,7 @@ ppl_status ppl_plan_destroy(ppl_plan P) try {
     if (!P) return PPL_OK;
     (void)hipDeviceSynchronize();
     for (int i = 0; i < kGroupKinds; ++i)
-        if (P->d_tab[i]) (void)hipFree(P->d_tab[i]);
+        if (P->d_tab[i] && i != P->tab_in_first) (void)hipFree(P->d_tab[i]);
     if (P->d_off) (void)hipFree(P->d_off);
     if (P->d_obb_off) (void)hipFree(P->d_obb_off);
     if (P->d_prob) (void)hipFree(P->d_prob);
