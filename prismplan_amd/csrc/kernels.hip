@@ -1288,12 +1288,10 @@ __device__ __forceinline__ float sphere_hinge_at(const CostArgs& a, const EsdfLa
             EsdfTap t;
             t.load(layer, px, py, pz, true);
             const float c = t.value(r), hh = m - c;
-            if (hh > 0.0f) {
-                world += hh;
-                if (GRAD && c < 1000.0f) {   // 1000: not from the grid, no gradient
-                    t.grad(layer, dx, dy, dz);
-                    gx += dx; gy += dy; gz += dz;
-                }
+            if (hh > 0.0f) world += hh;
+            if (GRAD && hh > 0.0f && c < 1000.0f) {   // 1000: not from the grid, no gradient
+                t.grad(layer, dx, dy, dz);
+                gx += dx; gy += dy; gz += dz;
             }
         } else {
             const float c = esdf_clearance(a.S, px, py, pz, r, sph_id, GRAD, dx, dy, dz);
