@@ -49,14 +49,14 @@ FLOPS_RULE = ("achieved = gated early-exit flops per state x states / kernel tim
 # The headline kernel's counters (rocprofv3 --pmc, median per dispatch over
 # the timed loop; profiles/edges_collide_counters.txt): VALU instructions and
 # SQ_INSTS_VALU_FLOPS_FP32 per dispatch, with the kernel time of that run.
-COUNTER_VALU_INSTS_EDGES = 16_513_783
+COUNTER_VALU_INSTS_EDGES = 16_263_095
 COUNTER_VALU_FLOPS_FP32_EDGES = 9_053_234
-COUNTER_KERNEL_US_EDGES = 38.84
+COUNTER_KERNEL_US_EDGES = 38.91
 CUS, SIMDS_PER_CU, CLOCK_HZ = 256, 4, 2.4e9
 # HBM bytes one headline launch moves (k_collide), from rocprofv3 FETCH_SIZE and
 # WRITE_SIZE scaled by a 256 MiB copy (same profile); the algorithmic bytes are
 # 16,384 edges x 69 B.
-TRAFFIC_BYTES_EDGES = 8_877_773
+TRAFFIC_BYTES_EDGES = 8_879_219
 ALGORITHMIC_BYTES_EDGES = 16384 * 69
 
 

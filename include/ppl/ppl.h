@@ -311,9 +311,10 @@ ppl_status ppl_tune_cache_file(const char* path);
  * problem's OBBs in one staging, then 128, 64 and 32 records below that; the
  * stagings of a problem then pass through LDS in turn) and each grid form
  * (0: up to eight times the workgroups the chip holds at once, 1: twice
- * them, 2: one workgroup per 64-state chunk), keeps the fastest for this plan's later any-collision calls and
- * records it in the tuning cache under the robot's tables, the largest
- * problem's OBB count and the GPU architecture; when the cache already holds
+ * them, 2: one workgroup per chunk of states), keeps the fastest for this
+ * plan's later any-collision calls and records it in the tuning cache under
+ * the kernels' revision, the robot's tables, the largest problem's OBB count
+ * and the GPU architecture; when the cache already holds
  * a choice for that key it is adopted without timing (*best_ms: the time
  * recorded with it). The fixed tile it replaces is the reference's
  * BATCH_SIZE (collision/scene_collision.cuh:9-11). Results do not depend on
@@ -329,7 +330,8 @@ ppl_status ppl_plan_collide_shape(ppl_plan plan, int max_obbs, int* tile, int* g
 
 /* Pin the any-collision launch shape (tile 0: every OBB of a problem in one
  * staging, up to 256; grid 0, 1, 2 as above); (0, 0) returns to the tuning
- * cache / built-in choice. */
+ * cache / built-in choice (grid 0; tiles of 128 where more than some 190 OBBs
+ * in one staging would leave a large launch too few workgroups a CU). */
 ppl_status ppl_plan_set_collide_shape(ppl_plan plan, int tile, int grid);
 
 /* Kernel timing (enable != 0: on): each later call of

@@ -1,21 +1,23 @@
 // kernels.hip -- gfx950 kernels of the collision-kinematics substrate.
 //
 // Execution model (wave64, CDNA4):
-//  * one lane = one robot state (configuration, edge state or waypoint);
-//    a 64-lane workgroup is one wavefront and runs persistently over a
-//    static, XCD-aware sweep of 64-state chunks (chunks never span two
-//    problems, so each wave sees one OBB set at a time);
-//  * the problem's enabled OBBs are re-packed into LDS once per problem
-//    switch; every lane then reads the same record (LDS broadcast);
-//  * FK walks the DFS-ordered joint table with wave-uniform (scalar) loads,
-//    keeping the live 3x4 transforms in VGPRs;
-//  * the any-collision predicate gates each (joint, OBB) pair on the joint's
-//    approximate bounding sphere with a wave ballot, tests the joint's exact
-//    spheres in box-local coordinates through one composed 3x4 matrix, and
-//    retires the wave as soon as every lane has a verdict;
-//  * the summed-hinge cost keeps per-joint adjoint accumulators in registers
-//    (joint loop unrolled to a compile-time bound) and differentiates through
-//    the argmin OBB of each active sphere in the same pass.
+//  * a workgroup is one wavefront; it walks chunks of robot states
+//    (configurations, edge states or waypoints) in a static, XCD-aware order
+//    (chunks never span two problems, so each wave sees one OBB set at a
+//    time), with 1 to 16 lanes per state by the kernel and the launch's size;
+//  * the problem's enabled OBBs are re-packed into LDS records once per
+//    problem switch, or tile by tile where one staging does not hold them;
+//  * FK walks the DFS-ordered joint table with wave-uniform (scalar) loads and
+//    the live 3x4 transforms in VGPRs, or, with 16 lanes per state, composes
+//    one joint per lane by pointer jumping through LDS;
+//  * the any-collision predicate narrows each joint's boxes by rows of 16
+//    states, then by each state's approximate sphere, and tests the exact
+//    spheres of the (state, box) pairs left in full waves;
+//  * the summed-hinge cost tests a sphere cluster's candidate boxes only; its
+//    adjoint differentiates through the argmin OBB of each active sphere in
+//    the same pass and sums the wrenches over the joint tree;
+//  * self collision goes by blocks of sphere-cluster pairs, large
+//    any-collision sets by rough distances first.
 #include "ppl_internal.hpp"
 
 #include <hip/hip_ext.h>
@@ -802,10 +804,10 @@ __device__ __forceinline__ float wave_sum(float v) {
 //  3. the pairs that hit are queued in LDS and taken 64 at a time, one pair
 //     per lane (fewer pairs: several lanes share one, each a part of the
 //     joint's spheres), with the frame out of the state's own lane.
-// Bound by VALU and SALU issue. The whole wave used to share one candidate
-// set, and tested the exact spheres of a pair in all lanes as soon as one lane
-// had it: on 16,384 edges among 64 boxes a wave went through 100 candidates
-// and 12 exact boxes, of which its states needed 2.7 x 64 pairs; on uncorrelated
+// Bound by VALU and SALU issue. With one candidate set for the whole wave, and
+// the exact spheres of a pair tested in all lanes as soon as one lane has it, a
+// wave goes through 100 candidates and 12 exact boxes on 16,384 edges among 64
+// boxes, of which its states need 2.7 x 64 pairs; on uncorrelated
 // configurations (20 boxes) 89 and 31, needing 1.4 x 64. Together with the
 // scalar table loads and the grid (kCollideWaves): the edges 321 -> 179 us a
 // call, 262,144 configurations of 64 requests 135 -> 48 us, 11 densified
@@ -1966,8 +1968,7 @@ __device__ __forceinline__ void cost_grp(const CostArgs& a) {
         // sphere walk its cluster's mask together, so each quarter-wave of an
         // LDS record read touches 4 records (broadcast) instead of 16 (bank
         // conflicts). Each state's spheres keep their lanes' relative order,
-        // so sums and atomics run in the same order as with lane = 16 *
-        // state + slot.
+        // so sums run in the same order as with lane = 16 * state + slot.
         const int rslot = lane & (kGrpStates - 1), rsub = lane >> 2;
         const bool ractive = (long)ch.y + rslot < ch.z;
         const float* Tr = s_T + rslot * fstride;
@@ -2534,7 +2535,8 @@ __global__ __launch_bounds__(64, 4) void k_self(SelfArgs a) {
 // pair with a's constants in SGPRs. val = |b - a|^2 - (ra + rb + slack)^2 above
 // its rounding err for all pairs proves the state free (slack bounds the frames'
 // and the transforms' errors), val below -(4 rs slack + err) for one proves it
-// hit. What is open is decided by the exact pass, so the verdicts are its own.
+// hit (of a slack up to the radii). What is open is decided by the exact pass, so
+// the verdicts are its own.
 // Bound by VALU issue: frames once per state instead of in every group's rounds,
 // and 210 pairs of near blocks a wave of states where the exact pass spends about
 // 1,000 instructions on four states. Where it runs: see self_far.
@@ -3746,9 +3748,11 @@ hipError_t launch_clear(const ClearArgs& a, hipStream_t s) {
 // keeps neighbours near (edges and trajectories; a wave's near blocks are then
 // few), of models of up to 64 blocks. Measured, edges of 10 boxes with the
 // self check, us a call with it and without: Panda (23 blocks) 51,132 states 67
-// and 66, 180,857 106 and 124, 736,240 290 and 416; Fetch (153 blocks) 174,587 219
-// and 222, 699,268 664 and 787, but 48,403 126 and 104; Baxter (150) 877 and 714.
-// Uncorrelated configurations: Panda 262,144 170 and 173, Fetch 605 and 371.
+// and 66, 180,857 106 and 124, 736,240 290 and 416; Fetch (153 blocks) 48,403 126
+// and 104, 174,587 219 and 222, 699,268 664 and 787; Baxter (150), some 700,000,
+// 877 and 714. Uncorrelated configurations: Panda 262,144 170 and 173, Fetch 605 and 371.
+// The limit of blocks takes what wins on every size from 65,536 on; the number of
+// blocks does not tell Fetch from Baxter, so large Fetch sets go without, too.
 static bool self_far(const DRobot& R, int mode, int source, long n_states) {
     return mode == 0 && R.far_blk && R.self_gate_implied && R.n_cpb <= 64 && n_states >= 65536 && source != kSrcConfig &&
            source != kSrcBfs && FarLds(R).bytes <= 65536;

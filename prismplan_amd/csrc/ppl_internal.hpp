@@ -212,7 +212,6 @@ struct SelfArgs {
                                 // indexed by plan order either way
 };
 
-// t0 / t1 (optional): events the runtime records at the kernel's start and end
 // Lanes per state of an any-collision launch of so many states (chunks hold 64
 // over that; models that need the gated form take one). A wave of 64 states is a
 // long chain when nothing else runs beside it, above all of box tests where the
@@ -225,6 +224,7 @@ struct SelfArgs {
 constexpr int kCollideParts = 4;
 constexpr long kCollideSplit = 32768;
 int collide_lanes(const DRobot& R, long n_states);
+// t0 / t1 (optional): events the runtime records at the kernel's start and end
 hipError_t launch_collide(const CollideArgs& a, int grid, hipStream_t s, hipEvent_t t0 = nullptr,
                           hipEvent_t t1 = nullptr);
 hipError_t launch_cost(const CostArgs& a, int grid, hipStream_t s, hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr);
