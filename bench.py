@@ -36,6 +36,9 @@ from pathlib import Path
 ROOT = Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT))
 sys.path.insert(0, str(ROOT / "oracle"))
+# autotuner choices stay in memory unless a cache file is named: those timed on
+# these worlds are not for the user's other programs
+os.environ.setdefault("PPL_TUNE_CACHE", "")
 
 METRIC = "collision-checked configs/s + CHOMP cost+grad traj/s, batched vs plain, 1 GPU"
 PEAK_FP32 = 157.3e12          # MI355X FP32 peak (packed issue)
